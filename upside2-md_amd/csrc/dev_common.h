@@ -8,60 +8,118 @@
 
 namespace upside {
 
-// Execution context of one workgroup.  A system is evaluated by a team of G
-// workgroups (G = 1: a single workgroup, no grid barriers).  Data-parallel
-// loops stride over the team's threads (gtid, gsize); team_sync separates
-// phases whose data cross workgroups.
 // Address-space-typed pointers.  Arena and table pointers reach the device
 // code through descriptors, so the compiler sees them as generic (flat)
 // pointers: every flat load is counted against both the vector-memory and
-// the LDS counters and waits serialise.  Hot loops re-type their pointers
-// with gmem()/lmem() so that loads become global_load / ds_read.
+// the LDS counters and waits serialise.  Device code therefore holds them as
+// global (gp, global_load) or LDS (lp, ds_read) pointers.  Descriptors and
+// programs are constant while a kernel runs: they are read through the
+// constant address space (cp), so that a record at a workgroup-uniform address
+// arrives in scalar registers through the scalar cache, which the team
+// barriers do not invalidate.
 #define UPS_GLOBAL __attribute__((address_space(1)))
 #define UPS_LDS __attribute__((address_space(3)))
+#define UPS_CONST __attribute__((address_space(4)))
 template <class T> using gp = UPS_GLOBAL T*;
 template <class T> using lp = UPS_LDS T*;
+template <class T> using cp = UPS_CONST const T*;
 template <class T> __device__ __forceinline__ gp<T> gmem(T* p) { return (gp<T>)p; }
-template <class T> __device__ __forceinline__ lp<T> lmem(T* p) { return (lp<T>)p; }
+template <class T> __device__ __forceinline__ cp<T> cmem(const T* p) { return (cp<T>)p; }
+using OpC = UPS_CONST const OpRec;
+using GraphC = UPS_CONST const PairGraph;
+using RotC = UPS_CONST const RotamerDev;
+using SysC = UPS_CONST const SysDesc;
 
-struct Ctx {
-    float* A;          // per-system float arena
-    int* I;            // per-system int arena
-    const float* CF;   // constant float arena
-    const int* CI;     // constant int arena
-    float* red;        // LDS reduction scratch [NWAVE]
-    int* ired;         // LDS reduction scratch [NWAVE] (ints)
-    float* lds;        // LDS staging area [LDS_FLOATS]
-    int tid;           // thread in the workgroup
-    unsigned long long* prof;  // wall-clock accumulators (null: profiling off)
-    int pbase;                 // first fixed profile slot
-    int cur_op;                // program op being run (team barriers are counted per op while profiling)
-    int err;                   // int arena offset of the error word this (sub-)team sets and reads
-    int early_done;            // this evaluation ran the early deriv ops beside the rotamer solve
-    int rot_graph_done;        // this evaluation refreshed the rotamer pair graph in a section lane
+// A value every lane holds alike, as a scalar.
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ float unif(float v) { return __int_as_float(uni(__float_as_int(v))); }
+__device__ __forceinline__ unsigned long long uni64(unsigned long long v) {
+    const unsigned lo = (unsigned)uni((int)(unsigned)v), hi = (unsigned)uni((int)(unsigned)(v >> 32));
+    return ((unsigned long long)hi << 32) | lo;
+}
+
+// The team that runs the current ops: G workgroups with a common arrival
+// counter (G = 1: one workgroup, no grid barriers).  Data-parallel loops
+// stride over the team's threads (gtid, gsize); team_sync separates phases
+// whose data cross workgroups.
+struct Team {
     int rank, G;       // workgroup rank in the team, team size
     int gtid, gsize;   // thread in the team, team threads
-    unsigned long long* bar;  // team barrier arrival counter
-    unsigned long long bar_next;  // count that opens this workgroup's next barrier on `bar` (thread 0)
-    unsigned* bar_flag;       // team barrier spin-timeout flag
-    int local;                // the whole team runs on one XCD (shares one L2)
-    unsigned long long* bar2; // arrival counter of the sub-team of ranks 1..G-1
-    float* tred2;             // the sub-team's reduction scratch
-    int tpar2;                // the sub-team's next reduction buffer parity
-    unsigned long long* bar_lo;  // sub-team of ranks 0..G/2-1: counter, scratch, parity
-    float* tred_lo;
-    int tpar_lo;
-    unsigned long long* bar_hi;  // sub-team of ranks G/2..G-1
-    float* tred_hi;
-    int tpar_hi;
-    unsigned long long* bar_q;   // the four quarter sub-teams: counters bar_q[j], scratch tred_q + 2*MAX_TEAM*j,
-    float* tred_q;               // and the parity of this workgroup's own quarter
-    int tpar_q;
-    float* tred;       // team reduction scratch, 2 buffers of G floats
-    int tpar;          // buffer parity of the next team reduction
-    int bp_layout;     // where rotamer solves run (see bp_on_one_wg)
-    const RunArgs* args;  // the launch's arguments (rotamer solve schedule, warm-start network)
+    gp<unsigned long long> bar;   // arrival counter
+    unsigned long long bar_next;  // count that opens this workgroup's next barrier on `bar`
+    gp<float> tred;    // reduction scratch, 2 buffers of G floats
+    int tpar;          // buffer parity of the next reduction
+    int err;           // int arena offset of the error word this team sets
+    unsigned long long* prof;  // wall-clock accumulators (null: profiling off)
 };
+
+// Execution context of one workgroup.  Everything here is uniform over the
+// workgroup except tid and gtid.  Functions that take a Ctx are inlined into
+// the few outlined phase functions of the kernel (PHASE), and within one a
+// context is a set of scalar registers: ctx_load reads it from LDS at the
+// phase's start.  (Passed by reference it lives in private memory, and every
+// phase begins by reloading it from L2, since a team barrier drops L1.
+// Measured with the program records in scalar registers, ms per step: 0.55 ->
+// 0.47 for 67 residues on 8 workgroups, 1.03 -> 0.95 for 500 on 32.)
+struct Ctx : Team {
+    gp<float> A;           // per-system float arena
+    gp<int> I;             // per-system int arena
+    gp<const float> CF;    // constant float arena
+    gp<const int> CI;      // constant int arena
+    cp<SysDesc> S;         // the system
+    cp<RunArgs> args;      // the launch's arguments
+    gp<unsigned> bar_flag; // team barrier spin-timeout flag
+    lp<float> red;         // LDS reduction scratch [NWAVE]
+    lp<int> ired;          // LDS reduction scratch [NWAVE] (ints)
+    lp<float> lds;         // LDS staging area [LDS_FLOATS]
+    int pbase;             // first fixed profile slot
+    int cur_op;            // program op being run (team barriers are counted per op while profiling)
+    int local;             // the whole team runs on one XCD (shares one L2)
+    int bp_layout;         // where rotamer solves run (see bp_on_one_wg)
+    int tid;               // thread in the workgroup
+};
+
+// A context in LDS, one copy per wave (no wave waits for another's).
+constexpr int CTX_WORDS = (sizeof(Ctx) + 15) / 16 * 4;
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ lp<i32x4> ctx_slot(lp<int> mem) {
+    return (lp<i32x4>)(mem + (int)(threadIdx.x >> 6) * CTX_WORDS);
+}
+__device__ __forceinline__ void ctx_store(lp<int> mem, const Ctx& c) {
+    int w[CTX_WORDS] = {};
+    __builtin_memcpy(w, &c, sizeof(Ctx));
+    lp<i32x4> m = ctx_slot(mem);
+#pragma unroll
+    for (int k = 0; k < CTX_WORDS / 4; ++k) m[k] = i32x4{w[4 * k], w[4 * k + 1], w[4 * k + 2], w[4 * k + 3]};
+}
+__device__ __forceinline__ Ctx ctx_load(lp<int> mem) {
+    int w[CTX_WORDS];
+    lp<i32x4> m = ctx_slot(mem);
+#pragma unroll
+    for (int k = 0; k < CTX_WORDS / 4; ++k) {
+        const i32x4 v = m[k];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) w[4 * k + q] = uni(v[q]);
+    }
+    Ctx c;
+    __builtin_memcpy(&c, w, sizeof(Ctx));
+    c.tid = (int)threadIdx.x;
+    c.gtid = c.rank * NT + c.tid;
+    return c;
+}
+
+// What a phase function gives back: the barrier state it advanced, and a
+// result.
+struct PhaseRet {
+    unsigned long long bar_next;
+    int tpar, value;
+};
+__device__ __forceinline__ PhaseRet phase_ret(const Ctx& c, int value) { return PhaseRet{c.bar_next, c.tpar, value}; }
+__device__ __forceinline__ int phase_done(Ctx& c, const PhaseRet& r) {
+    c.bar_next = uni64(r.bar_next);
+    c.tpar = uni(r.tpar);
+    return uni(r.value);
+}
 
 __device__ __forceinline__ unsigned long long ptick(const Ctx& c) { return c.prof ? wall_clock64() : 0ull; }
 __device__ __forceinline__ void pacc(const Ctx& c, int slot, unsigned long long t0) {
@@ -96,21 +154,22 @@ constexpr int WAIT_VMEM = 0x0F70;
 // Count that opens the first barrier of a team of G on counter `bar`, read
 // before this workgroup's first arrival: fewer than G arrivals of that
 // barrier can precede it (it cannot open without this workgroup), so the
-// count rounded down to a multiple of G is the base.  Thread 0.
-__device__ __forceinline__ unsigned long long bar_first(unsigned long long* bar, int G) {
-    const unsigned long long v = __hip_atomic_load(bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// count rounded down to a multiple of G is the base.
+__device__ __forceinline__ unsigned long long bar_first(gp<unsigned long long> bar, int G) {
+    const unsigned long long v = uni64(__hip_atomic_load(bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
     return (v / (unsigned long long)G + 1ull) * (unsigned long long)G;
 }
 
-__device__ void team_sync(Ctx& c) {
+__device__ __forceinline__ void team_sync(Ctx& c) {
     // every wave's stores acknowledged by L2 before the team can observe the arrival
     if (c.G > 1 && c.local) __builtin_amdgcn_s_waitcnt(WAIT_VMEM);
     __syncthreads();
     if (c.G > 1) {
+        const unsigned long long target = c.bar_next;
+        c.bar_next = target + (unsigned long long)c.G;
         if (c.tid == 0) {
             if (!c.local) __threadfence();
             (void)__hip_atomic_fetch_add(c.bar, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const unsigned long long target = c.bar_next;
             unsigned spins = 0;
             while (__hip_atomic_load(c.bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
                 __builtin_amdgcn_s_sleep(2);
@@ -122,7 +181,6 @@ __device__ void team_sync(Ctx& c) {
                     break;
                 }
             }
-            c.bar_next = target + (unsigned long long)c.G;
             if (c.local) asm volatile("buffer_inv sc1" ::: "memory");  // L1 (no L2 write-back)
             else __threadfence();
         }
@@ -134,33 +192,57 @@ __device__ void team_sync(Ctx& c) {
     }
 }
 
-// The sub-team of ranks [first, first + size) with its own barrier counter,
-// reduction scratch and buffer parity, for work that runs beside the rest of
-// the team.  Only rank 0 keeps the profile accumulators.
-__device__ __forceinline__ Ctx sub_team(const Ctx& c, int first, int size, unsigned long long* bar, float* tred,
-                                        int tpar) {
-    Ctx s = c;
-    s.G = size;
-    s.rank = c.rank - first;
-    s.gtid = s.rank * NT + c.tid;
-    s.gsize = size * NT;
-    s.bar = bar;
-    if (size > 1 && c.tid == 0) s.bar_next = bar_first(bar, size);
-    s.tred = tred;
-    s.tpar = tpar;
-    if (c.rank != 0) s.prof = nullptr;
-    return s;
+// Sub-teams: parts of a team that run beside each other, each with an arrival
+// counter and reduction scratch of its own.  A workgroup belongs to the same
+// part of each kind for a whole launch, so it keeps the kind's barrier count
+// (SubNext) from one use to the next.
+enum SubTeam : int {
+    SUB_REST = 0,   // ranks 1..G-1, beside rank 0's rotamer solve
+    SUB_HALF = 1,   // ranks [0, G/2) and [G/2, G)
+    SUB_QUARTER = 2 // ranks [j*G/4, (j+1)*G/4)
+};
+struct SubNext {  // named, not indexed: an indexed array would live in private memory
+    unsigned long long rest, half, quarter;
+};
+struct SubPart { int first, size, word, buf; };  // ranks, counter word, reduction buffer
+__device__ __forceinline__ SubPart sub_part(int kind, int rank, int G) {
+    if (kind == SUB_REST) return SubPart{1, G - 1, BAR_SUB1, 1};
+    if (kind == SUB_HALF) return rank < G / 2 ? SubPart{0, G / 2, BAR_LO, 2} : SubPart{G / 2, G - G / 2, BAR_HI, 3};
+    int j = 0;
+    while (j + 1 < 4 && rank >= (j + 1) * G / 4) ++j;
+    return SubPart{j * G / 4, (j + 1) * G / 4 - j * G / 4, BAR_Q + 2 * j, 4 + j};
 }
 
-// The sub-team of ranks 1..G-1 (G >= 2), for work that runs beside rank 0.
-__device__ __forceinline__ Ctx sub_team(const Ctx& c) { return sub_team(c, 1, c.G - 1, c.bar2, c.tred2, c.tpar2); }
+// Narrow the context from the whole team `root` to this workgroup's part of
+// kind `kind`.  Only rank 0 of the whole team keeps the profile accumulators
+// (with `part_prof` the part's first workgroup does, so that each part's ops
+// are timed).
+__device__ __forceinline__ void enter_sub(Ctx& c, const SubNext& next, const Team& root, int kind,
+                                          gp<int> words, unsigned long long* part_prof) {
+    const SubPart p = sub_part(kind, root.rank, root.G);
+    c.G = p.size;
+    c.rank = root.rank - p.first;
+    c.gtid = c.rank * NT + c.tid;
+    c.gsize = p.size * NT;
+    c.bar = (gp<unsigned long long>)(words + p.word);
+    c.bar_next = kind == SUB_REST ? next.rest : kind == SUB_HALF ? next.half : next.quarter;
+    c.tred = root.tred + p.buf * 2 * MAX_TEAM;
+    c.tpar = 0;
+    c.prof = c.rank == 0 ? part_prof : nullptr;
+}
+__device__ __forceinline__ void leave_sub(Ctx& c, SubNext& next, const Team& root, int kind) {
+    next.rest = kind == SUB_REST ? c.bar_next : next.rest;
+    next.half = kind == SUB_HALF ? c.bar_next : next.half;
+    next.quarter = kind == SUB_QUARTER ? c.bar_next : next.quarter;
+    (Team&)c = root;
+}
 
 // XCD of the calling workgroup (hardware register XCC_ID).
 __device__ __forceinline__ unsigned xcd_id() { return __builtin_amdgcn_s_getreg((15 << 11) | (0 << 6) | 20); }
 
 // At launch start of a team: every workgroup records its XCD; the team uses
 // L2-local barriers only if all agree.  All threads of the team.
-__device__ void team_place(Ctx& c, int* xtab) {
+__device__ __forceinline__ void team_place(Ctx& c, gp<int> xtab) {
     c.local = 0;
     if (c.G == 1) return;
     if (c.tid == 0) __hip_atomic_store(&xtab[c.rank], (int)xcd_id(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -169,7 +251,7 @@ __device__ void team_place(Ctx& c, int* xtab) {
     int x0 = __hip_atomic_load(&xtab[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     for (int r = 1; r < c.G; ++r) same &= __hip_atomic_load(&xtab[r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == x0;
     team_sync(c);  // every workgroup has read the table before it is rewritten
-    c.local = same;
+    c.local = uni(same);
     if (c.rank == 0 && c.tid == 0) xtab[-1] = same;  // reported to the host (barrier word 3)
 }
 
@@ -184,66 +266,68 @@ __device__ __forceinline__ float wave_max(float v) {
 
 // Block sum in a fixed order (lane tree, then waves in index order): the
 // result is the same on every run.  All threads must call it.
-__device__ float block_sum(Ctx& c, float v) {
+__device__ __forceinline__ float block_sum(Ctx& c, float v) {
     v = wave_sum(v);
-    __syncthreads();
+    __syncthreads();  // the previous reduction has been read
     if ((c.tid & 63) == 0) c.red[c.tid >> 6] = v;
     __syncthreads();
     float t = 0.f;
     for (int w = 0; w < NWAVE; ++w) t += c.red[w];
-    __syncthreads();
-    return t;
+    return unif(t);
 }
-__device__ float block_max(Ctx& c, float v) {
+__device__ __forceinline__ float block_max(Ctx& c, float v) {
     v = wave_max(v);
     __syncthreads();
     if ((c.tid & 63) == 0) c.red[c.tid >> 6] = v;
     __syncthreads();
     float t = c.red[0];
     for (int w = 1; w < NWAVE; ++w) t = fmaxf(t, c.red[w]);
-    __syncthreads();
-    return t;
-}
-__device__ int block_or(Ctx& c, int v) {
-    int any = __syncthreads_or(v);
-    return any;
+    return unif(t);
 }
 
 // Team reductions: workgroup partials combined in rank order (fixed order, so
-// the result is the same on every run).  All threads of the team.
-__device__ float team_sum(Ctx& c, float v) {
+// the result is the same on every run).  All threads of the team.  The
+// partials of all ranks (at most MAX_TEAM, one per lane) are read in one
+// memory trip and combined from registers; a loop over them in memory pays a
+// trip per unrolled group of ranks.
+static_assert(MAX_TEAM <= 64, "one lane per rank");
+__device__ __forceinline__ gp<float> team_partials(Ctx& c, float t) {
+    gp<float> buf = c.tred + c.tpar * c.G;
+    c.tpar ^= 1;
+    if (c.tid == 0) buf[c.rank] = t;
+    team_sync(c);
+    return buf;
+}
+__device__ __forceinline__ float lane_value(float v, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+__device__ __forceinline__ float team_sum(Ctx& c, float v) {
     float t = block_sum(c, v);
     if (c.G == 1) return t;
-    float* buf = c.tred + c.tpar * c.G;
-    c.tpar ^= 1;
-    if (c.tid == 0) buf[c.rank] = t;
-    team_sync(c);
+    gp<float> buf = team_partials(c, t);
+    const float x = buf[min(c.tid & 63, c.G - 1)];
     float s = 0.f;
-    for (int r = 0; r < c.G; ++r) s += buf[r];
-    return s;
+    for (int r = 0; r < c.G; ++r) s += lane_value(x, r);
+    return unif(s);
 }
-__device__ float team_max(Ctx& c, float v) {
+__device__ __forceinline__ float team_max(Ctx& c, float v) {
     float t = block_max(c, v);
     if (c.G == 1) return t;
-    float* buf = c.tred + c.tpar * c.G;
-    c.tpar ^= 1;
-    if (c.tid == 0) buf[c.rank] = t;
-    team_sync(c);
-    float s = buf[0];
-    for (int r = 1; r < c.G; ++r) s = fmaxf(s, buf[r]);
-    return s;
+    gp<float> buf = team_partials(c, t);
+    return unif(wave_max(buf[min(c.tid & 63, c.G - 1)]));
 }
-__device__ int team_or(Ctx& c, int v) {
-    int t = __syncthreads_or(v);
+__device__ __forceinline__ int team_or(Ctx& c, int v) {
+    int t = uni(__syncthreads_or(v));
     if (c.G == 1) return t;
-    return team_max(c, t ? 1.f : 0.f) > 0.f ? 1 : 0;
+    gp<float> buf = team_partials(c, t ? 1.f : 0.f);
+    return __any(buf[min(c.tid & 63, c.G - 1)] > 0.f) ? 1 : 0;
 }
 
 // In-place exclusive scan of the ints a[0..n) (any memory); returns the
 // total.  Each thread scans a contiguous chunk, chunk totals are scanned
 // across the block.  All threads must call it.
 template <class P>
-__device__ int block_exscan(Ctx& c, P a, int n) {
+__device__ __forceinline__ int block_exscan(Ctx& c, P a, int n) {
     int per = (n + NT - 1) / NT;
     int b = c.tid * per, e = min(b + per, n);
     int s = 0;
@@ -277,21 +361,21 @@ __device__ int block_exscan(Ctx& c, P a, int n) {
 // returns the total.  Each workgroup scans a contiguous chunk, chunk totals
 // are added in rank order.  All threads of the team.
 template <class P>
-__device__ int team_exscan(Ctx& c, P a, int n) {
-    if (c.G == 1) return block_exscan(c, a, n);
+__device__ __forceinline__ int team_exscan(Ctx& c, P a, int n) {
     int per = (n + c.G - 1) / c.G;
     int b = min(c.rank * per, n), e = min(b + per, n);
-    int tot = block_exscan(c, a + b, e - b);
-    float* buf = c.tred + c.tpar * c.G;
-    c.tpar ^= 1;
-    if (c.tid == 0) buf[c.rank] = __int_as_float(tot);
-    team_sync(c);
-    int before = 0, all = 0;
-    for (int r = 0; r < c.G; ++r) {
-        int x = __float_as_int(buf[r]);
-        if (r < c.rank) before += x;
-        all += x;
+    int tot = uni(block_exscan(c, a + b, e - b));
+    if (c.G == 1) return tot;
+    gp<float> buf = team_partials(c, __int_as_float(tot));
+    const int lane = c.tid & 63;
+    const int x = lane < c.G ? __float_as_int(buf[lane]) : 0;
+    int v = x;  // inclusive scan over the ranks
+    for (int o = 1; o < 64; o <<= 1) {
+        const int t = __shfl_up(v, o, 64);
+        if (lane >= o) v += t;
     }
+    const int all = __builtin_amdgcn_readlane(v, 63);
+    const int before = __builtin_amdgcn_readlane(v - x, c.rank);
     for (int i = b + c.tid; i < e; i += NT) a[i] += before;
     team_sync(c);
     return all;
@@ -387,7 +471,8 @@ __device__ __forceinline__ void quat_to_rot(P q, float* U) {
 // Fixed-order gather (see engine_dev.h): each target row adds the sum of its
 // contributions, in plan order.  A thread loads each contribution's index
 // once and all its components with it (per component the terms are summed in
-// plan order, as one component at a time would).  Called by all threads.
+// plan order, as one component at a time would).  Called by all threads of
+// the team; no barrier at the end.
 template <int CW>
 __device__ __forceinline__ void plan_gather_w(Ctx& c, gp<const int> off, gp<const int> idx, gp<float> sens,
                                               gp<const float> con, int nt, int ss, int col, int cs) {
@@ -408,14 +493,13 @@ __device__ __forceinline__ void plan_gather_w(Ctx& c, gp<const int> off, gp<cons
     }
 }
 
-__device__ void plan_gather(Ctx& c, int plan) {
-    if (plan < 0) return;
-    gp<const int> h = gmem(c.CI + plan);
+__device__ __forceinline__ void plan_gather(Ctx& c, int plan) {
+    cp<int> h = (cp<int>)(c.CI + plan);  // the header is uniform: scalar loads
     int nt = h[0], cw = h[1], so = h[2], ss = h[3], col = h[4], cb = h[5], cs = h[6];
-    gp<const int> off = h + PLAN_HDR;
+    gp<const int> off = c.CI + plan + PLAN_HDR;
     gp<const int> idx = off + nt + 1;
-    gp<float> sens = gmem(c.A + so);
-    gp<const float> con = gmem((const float*)c.A + cb);
+    gp<float> sens = c.A + so;
+    gp<const float> con = c.A + cb;
     switch (cw) {
     case 1: plan_gather_w<1>(c, off, idx, sens, con, nt, ss, col, cs); break;
     case 2: plan_gather_w<2>(c, off, idx, sens, con, nt, ss, col, cs); break;
@@ -432,7 +516,6 @@ __device__ void plan_gather(Ctx& c, int plan) {
             }
         }
     }
-    team_sync(c);
 }
 
 }  // namespace upside

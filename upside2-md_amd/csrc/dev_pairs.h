@@ -26,25 +26,25 @@ __device__ __forceinline__ float refine_dist2(float dx, float dy, float dz) {
     return __fmaf_rn(dx, dx, __fmaf_rn(dz, dz, __fmul_rn(dy, dy)));
 }
 
-__device__ __forceinline__ bool pg_accept(const PairGraph& G, int a, int b) {
+__device__ __forceinline__ bool pg_accept(GraphC& G, int a, int b) {
     if (G.excl < 0) return (a >> 4) != (b >> 4);
     int d = a - b;
     return d > G.excl || -d > G.excl;
 }
 
-__device__ __forceinline__ const float* pg_side2(const Ctx& c, const PairGraph& G) {
+__device__ __forceinline__ gp<const float> pg_side2(const Ctx& c, GraphC& G) {
     return c.A + G.pos_pack + (G.sym ? 0 : G.n1 * 3);
 }
 
 // Copy the current coordinates of both sides into pos_pack and report whether
 // the cache must be rebuilt (first use, or drift beyond half the buffer).
-__device__ bool pg_pack_and_check(Ctx& c, const PairGraph& G) {
-    gp<const int> loc1 = gmem(c.CI + G.loc1);
-    gp<const int> loc2 = gmem(c.CI + G.loc2);
-    gp<const float> P1 = gmem((const float*)c.A + G.out1);
-    gp<const float> P2 = gmem((const float*)c.A + G.out2);
-    gp<float> pack = gmem(c.A + G.pos_pack);
-    gp<const float> cache = gmem((const float*)c.A + G.cache_pos);
+__device__ __forceinline__ bool pg_pack_and_check(Ctx& c, GraphC& G) {
+    gp<const int> loc1 = c.CI + G.loc1;
+    gp<const int> loc2 = c.CI + G.loc2;
+    gp<const float> P1 = c.A + G.out1;
+    gp<const float> P2 = c.A + G.out2;
+    gp<float> pack = c.A + G.pos_pack;
+    gp<const float> cache = c.A + G.cache_pos;
     int n = G.sym ? G.n1 : G.n1 + G.n2;
     int valid = c.I[G.state];
     int moved = 0;
@@ -60,7 +60,7 @@ __device__ bool pg_pack_and_check(Ctx& c, const PairGraph& G) {
 }
 
 template <class P>
-__device__ int lower_bound_i(P a, int n, int v) {
+__device__ __forceinline__ int lower_bound_i(P a, int n, int v) {
     int lo = 0, hi = n;
     while (lo < hi) {
         int m = (lo + hi) >> 1;
@@ -116,8 +116,8 @@ __device__ __forceinline__ void el_put(lp<float> el, int k, float x, float y, fl
 }
 
 // Stage elements [t0, t0+n) of side pts (ids in id) as (x, y, z, id).
-__device__ void stage_tile(Ctx& c, gp<const float> pts, gp<const int> id, int t0, int n) {
-    lp<float> tile = lmem(c.lds);
+__device__ __forceinline__ void stage_tile(Ctx& c, gp<const float> pts, gp<const int> id, int t0, int n) {
+    lp<float> tile = c.lds;
     for (int k = c.tid; k < n; k += NT) {  // every workgroup stages its own copy
         int j = t0 + k;
         el_put(tile, k, pts[j * 3], pts[j * 3 + 1], pts[j * 3 + 2], id[j]);
@@ -130,10 +130,10 @@ __device__ void stage_tile(Ctx& c, gp<const float> pts, gp<const int> id, int t0
 // acceptable (SYM: also j > q).  !FILL adds row q's hits to off[q].  FILL
 // writes them at the cursor cur[q] (advanced).
 template <bool SYM, bool FILL>
-__device__ void tile_rows(Ctx& c, const PairGraph& G, gp<const float> qp, gp<const int> qid, int nq,
+__device__ __forceinline__ void tile_rows(Ctx& c, GraphC& G, gp<const float> qp, gp<const int> qid, int nq,
                           gp<const float> ep, gp<const int> eid, int ne, gp<int> off, gp<int> cur_arr, gp<int> nbr,
                           gp<int> row) {
-    lp<const float> tile = (lp<const float>)lmem(c.lds);
+    lp<const float> tile = (lp<const float>)c.lds;
     const float cc2 = G.cache_cut2;
     const GroupLanes L = group_lanes(c);
     const int grp = c.gtid / SG, ngrp = c.gsize / SG;
@@ -199,7 +199,7 @@ __device__ __forceinline__ bool lgrid_fits(int m) {
 
 // Build the grid of the m points pts (stride 3) in this workgroup's LDS
 // (every workgroup of a team builds its own copy).  All threads of the workgroup.
-__device__ LGrid lgrid_build(Ctx& c, const PairGraph& G, gp<const float> pts, gp<const int> ids, int m) {
+__device__ __forceinline__ LGrid lgrid_build(Ctx& c, GraphC& G, gp<const float> pts, gp<const int> ids, int m) {
     float mn0 = 3.0e38f, mn1 = 3.0e38f, mn2 = 3.0e38f;
     for (int i = c.tid; i < m; i += NT) {
         mn0 = fminf(mn0, pts[i * 3]);
@@ -215,7 +215,7 @@ __device__ LGrid lgrid_build(Ctx& c, const PairGraph& G, gp<const float> pts, gp
     g.inv = 1.f / (G.cache_cut * 1.0001f);
     int nb = lgrid_buckets(m);
     g.mask = nb - 1;
-    lp<float> L = lmem(c.lds);
+    lp<float> L = c.lds;
     g.ofs = (lp<int>)L;
     g.el = L + ((nb + 4) & ~3);
     g.eid = (lp<int>)(g.el + 4 * m);
@@ -227,7 +227,7 @@ __device__ LGrid lgrid_build(Ctx& c, const PairGraph& G, gp<const float> pts, gp
         atomicAdd((int*)(g.ofs + b + 1), 1);
     }
     __syncthreads();
-    block_exscan(c, (int*)(g.ofs + 1), nb);  // ofs[b+1] = start of bucket b
+    block_exscan(c, g.ofs + 1, nb);  // ofs[b+1] = start of bucket b
     for (int i = c.tid; i < m; i += NT) {
         float x = pts[i * 3], y = pts[i * 3 + 1], z = pts[i * 3 + 2];
         int b = cell_bucket(g.mask, cell_coord(x, g.ox, g.inv), cell_coord(y, g.oy, g.inv), cell_coord(z, g.oz, g.inv));
@@ -261,7 +261,7 @@ __device__ LGrid lgrid_build(Ctx& c, const PairGraph& G, gp<const float> pts, gp
 // Rows against the grid; same hit rule as tile_rows.  !FILL: off[q] = hits of
 // row q.  FILL: row q's hits are written from off[q] on.
 template <bool SYM, bool FILL>
-__device__ void grid_rows(Ctx& c, const PairGraph& G, const LGrid& g, gp<const float> qp, gp<const int> qid, int nq,
+__device__ __forceinline__ void grid_rows(Ctx& c, GraphC& G, const LGrid& g, gp<const float> qp, gp<const int> qid, int nq,
                           gp<int> off, gp<int> nbr, gp<int> row) {
     const float cc2 = G.cache_cut2;
     const GroupLanes L = group_lanes(c);
@@ -302,27 +302,27 @@ __device__ void grid_rows(Ctx& c, const PairGraph& G, const LGrid& g, gp<const f
 // r = number of entries of the column with a smaller slot.  Columns are split
 // among the team's workgroups; each workgroup stages runs of whole columns in
 // LDS.  All threads of the team.
-__device__ void pg_order_columns(Ctx& c, const PairGraph& G, int n2) {
-    gp<const int> toff = gmem((const int*)c.I + G.toff);
-    gp<const int> tmp = gmem((const int*)c.I + G.tmp);
-    gp<const int> nbr = gmem((const int*)c.I + G.nbr);
-    gp<int> tslot = gmem(c.I + G.tslot);
-    lp<int> sl = (lp<int>)lmem(c.lds);
+__device__ __forceinline__ void pg_order_columns(Ctx& c, GraphC& G, int n2) {
+    gp<const int> toff = c.I + G.toff;
+    gp<const int> tmp = c.I + G.tmp;
+    gp<const int> nbr = c.I + G.nbr;
+    gp<int> tslot = c.I + G.tslot;
+    lp<int> sl = (lp<int>)c.lds;
     const int CAP = LDS_FLOATS;
     int per = (n2 + c.G - 1) / c.G;
     int jb = min(c.rank * per, n2);
     const int jend = min(jb + per, n2);
     while (jb < jend) {
-        const int base = toff[jb];
+        const int base = uni(toff[jb]);
         // the longest run of whole columns [jb, je) that fits: largest je in
         // [jb+1, jend] with toff[je] - base <= CAP (je = jb+1 if none)
         int lo = jb + 1, hi = jend;
         while (lo < hi) {
             int mid = (lo + hi + 1) >> 1;
-            if (toff[mid] - base <= CAP) lo = mid; else hi = mid - 1;
+            if (uni(toff[mid]) - base <= CAP) lo = mid; else hi = mid - 1;
         }
         const int je = lo;
-        const int n = toff[je] - base;
+        const int n = uni(toff[je]) - base;
         if (n <= CAP) {
             for (int k = c.tid; k < n; k += NT) sl[k] = tmp[base + k];
             __syncthreads();
@@ -348,27 +348,27 @@ __device__ void pg_order_columns(Ctx& c, const PairGraph& G, int n2) {
     team_sync(c);
 }
 
-// Rebuild rows and transposed rows from pos_pack.  Sets state[1] on overflow
-// (the host grows the capacity and repeats the run).
+// Rebuild rows and transposed rows from pos_pack.  False, with state[1] set,
+// on overflow (the host grows the capacity and repeats the run).
 //   forward rows:    side-1 element i, partners j (symmetric: j > i) in the
 //                    canonical scan order;
 //   transposed rows: side-2 element j, the forward slots with partner j in
 //                    increasing slot order.
-__device__ void pg_rebuild(Ctx& c, const PairGraph& G) {
-    gp<const int> id1 = gmem(c.CI + G.id1);
+__device__ __forceinline__ bool pg_rebuild(Ctx& c, GraphC& G) {
+    gp<const int> id1 = c.CI + G.id1;
     const bool sym = G.sym != 0;
-    gp<const int> id2 = sym ? id1 : gmem(c.CI + G.id2);
-    gp<const float> pack = gmem((const float*)c.A + G.pos_pack);
-    gp<float> cache = gmem(c.A + G.cache_pos);
+    gp<const int> id2 = sym ? id1 : c.CI + G.id2;
+    gp<const float> pack = c.A + G.pos_pack;
+    gp<float> cache = c.A + G.cache_pos;
     gp<const float> p1 = pack;
-    gp<const float> p2 = gmem(pg_side2(c, G));
+    gp<const float> p2 = pg_side2(c, G);
     const int n1 = G.n1, n2 = sym ? G.n1 : G.n2;
-    gp<int> off = gmem(c.I + G.off);
-    gp<int> nbr = gmem(c.I + G.nbr);
-    gp<int> row = gmem(c.I + G.row);
-    gp<int> toff = gmem(c.I + G.toff);
-    gp<int> tmp = gmem(c.I + G.tmp);
-    gp<int> tcur = gmem(c.I + G.tcur);
+    gp<int> off = c.I + G.off;
+    gp<int> nbr = c.I + G.nbr;
+    gp<int> row = c.I + G.row;
+    gp<int> toff = c.I + G.toff;
+    gp<int> tmp = c.I + G.tmp;
+    gp<int> tcur = c.I + G.tcur;
     int npack = sym ? n1 : n1 + n2;
     for (int i = c.gtid; i < npack * 3; i += c.gsize) cache[i] = pack[i];
     for (int i = c.gtid; i <= n1; i += c.gsize) off[i] = 0;
@@ -396,11 +396,11 @@ __device__ void pg_rebuild(Ctx& c, const PairGraph& G) {
         else tile_rows<false, false>(c, G, p1, id1, n1, p2, id2, n2, off, off, off, off);
     }
     pacc(c, PROF_RB_SCAN, t1);
-    const int E = team_exscan(c, (int*)off, n1 + 1);
+    const int E = team_exscan(c, off, n1 + 1);
     if (E > G.ecap) {
         if (c.gtid == 0) { c.I[G.state + 1] = 1; c.I[G.state + 0] = 0; }
         team_sync(c);
-        return;
+        return false;
     }
     pacc(c, PROF_RB_COUNT, t0);
     t0 = ptick(c);
@@ -420,7 +420,7 @@ __device__ void pg_rebuild(Ctx& c, const PairGraph& G) {
     // transposed rows: column counts, arrival-order placement, slot order
     for (int s = c.gtid; s < E; s += c.gsize) atomicAdd((int*)(toff + nbr[s]), 1);
     team_sync(c);
-    team_exscan(c, (int*)toff, n2 + 1);
+    team_exscan(c, toff, n2 + 1);
     for (int j = c.gtid; j < n2; j += c.gsize) tcur[j] = toff[j];
     team_sync(c);
     for (int s = c.gtid; s < E; s += c.gsize) tmp[atomicAdd((int*)(tcur + nbr[s]), 1)] = s;
@@ -433,6 +433,7 @@ __device__ void pg_rebuild(Ctx& c, const PairGraph& G) {
         c.I[G.state + 3] = E;
     }
     team_sync(c);
+    return true;
 }
 
 // ---- edge functions -----------------------------------------------------
@@ -543,15 +544,22 @@ __device__ __forceinline__ float env_edge(P p, X x1, X x2, float* d1, float* d2)
     return score;
 }
 
+// a x b with the second product of each component rounded first.
+__device__ __forceinline__ void cross3_rn(const float* a, const float* b, float* o) {
+    o[0] = __fmaf_rn(a[1], b[2], -__fmul_rn(a[2], b[1]));
+    o[1] = __fmaf_rn(a[2], b[0], -__fmul_rn(a[0], b[2]));
+    o[2] = __fmaf_rn(a[0], b[1], -__fmul_rn(a[1], b[0]));
+}
+
 // BackbonePairs residue pair (src/backbone_steric.cpp:94-140): compact-sigmoid
 // repulsion between the placed backbone atoms (at most 4) of two residues;
 // derivatives are (force, torque) on each residue frame.
-__device__ float backbone_edge(const Ctx& c, const OpRec& op, int r1, int r2, float* d1, float* d2) {
-    gp<const float> aff = gmem((const float*)c.A + op.in_out[0]);
+__device__ __forceinline__ float backbone_edge(const Ctx& c, OpC& op, int r1, int r2, float* d1, float* d2) {
+    gp<const float> aff = c.A + op.in_out[0];
     int w = op.in_w[0];
-    gp<const float> ref = gmem(c.CF + op.ia[1]);
-    gp<const int> nat = gmem(c.CI + op.ia[2]);
-    gp<const int> res = gmem(c.CI + op.ia[0]);
+    gp<const float> ref = c.CF + op.ia[1];
+    gp<const int> nat = c.CI + op.ia[2];
+    gp<const int> res = c.CI + op.ia[0];
     int R1 = res[r1], R2 = res[r2];
     float a1[7], a2[7];
 #pragma unroll
@@ -588,13 +596,25 @@ __device__ float backbone_edge(const Ctx& c, const OpRec& op, int r1, int r2, fl
             compact_sigmoid(rm2 - 9.f, sharp, v, dv);
             pot += 4.f * v;
             float g = 2.f * 4.f * dv;
-            float gx = g * rx, gy = g * ry, gz = g * rz;
-            float p1x = X1[i][0] - a1[0], p1y = X1[i][1] - a1[1], p1z = X1[i][2] - a1[2];
-            float p2x = X2[j][0] - a2[0], p2y = X2[j][1] - a2[1], p2z = X2[j][2] - a2[2];
-            d1[0] += gx; d1[1] += gy; d1[2] += gz;
-            d1[3] += p1y * gz - p1z * gy; d1[4] += p1z * gx - p1x * gz; d1[5] += p1x * gy - p1y * gx;
-            d2[0] -= gx; d2[1] -= gy; d2[2] -= gz;
-            d2[3] -= p2y * gz - p2z * gy; d2[4] -= p2z * gx - p2x * gz; d2[5] -= p2x * gy - p2y * gx;
+            // the roundings are fixed here: left to the compiler, which product
+            // of a torque rounds first depends on the code around it, and a
+            // trajectory amplifies that
+            const float gv[3] = {g * rx, g * ry, g * rz};
+            const float p1[3] = {X1[i][0] - a1[0], X1[i][1] - a1[1], X1[i][2] - a1[2]};
+            const float p2[3] = {X2[j][0] - a2[0], X2[j][1] - a2[1], X2[j][2] - a2[2]};
+            float t1[3], t2[3];
+            cross3_rn(p1, gv, t1);
+            const bool flip = i == 0 && j < 2;  // the first pairs add g x p2, the others subtract p2 x g
+            if (flip) cross3_rn(gv, p2, t2);
+            else cross3_rn(p2, gv, t2);
+            const float r[3] = {rx, ry, rz};
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                d1[k] = __fmaf_rn(r[k], g, d1[k]);
+                d2[k] = __fmaf_rn(-r[k], g, d2[k]);
+                d1[3 + k] += t1[k];
+                d2[3 + k] += flip ? t2[k] : -t2[k];
+            }
         }
     }
     return pot;
@@ -603,22 +623,22 @@ __device__ float backbone_edge(const Ctx& c, const OpRec& op, int r1, int r2, fl
 // Refine every cached slot against the cutoff and evaluate the active edges;
 // param is the coefficient table (LDS or memory).
 template <int KIND, int DD1, int DD2, class P>
-__device__ void pg_edges_impl(Ctx& c, const PairGraph& G, const OpRec& op, P param) {
-    gp<const int> nbr = gmem((const int*)c.I + G.nbr);
-    gp<const int> row = gmem((const int*)c.I + G.row);
-    gp<int> act = gmem(c.I + G.act);
-    gp<float> val = gmem(c.A + G.val);
-    gp<float> D1 = gmem(c.A + G.d1);
-    gp<float> D2 = gmem(c.A + G.d2);
-    gp<const float> pack = gmem((const float*)c.A + G.pos_pack);
-    gp<const float> pk2 = gmem(pg_side2(c, G));
-    gp<const int> loc1 = gmem(c.CI + G.loc1);
-    gp<const int> loc2 = gmem(c.CI + G.loc2);
-    gp<const int> t1 = gmem(c.CI + G.type1);
-    gp<const int> t2 = gmem(c.CI + G.type2);
-    gp<const float> P1 = gmem((const float*)c.A + G.out1);
-    gp<const float> P2 = gmem((const float*)c.A + G.out2);
-    const int E = c.I[G.state + 3];
+__device__ __forceinline__ void pg_edges_impl(Ctx& c, GraphC& G, OpC& op, P param) {
+    gp<const int> nbr = c.I + G.nbr;
+    gp<const int> row = c.I + G.row;
+    gp<int> act = c.I + G.act;
+    gp<float> val = c.A + G.val;
+    gp<float> D1 = c.A + G.d1;
+    gp<float> D2 = c.A + G.d2;
+    gp<const float> pack = c.A + G.pos_pack;
+    gp<const float> pk2 = pg_side2(c, G);
+    gp<const int> loc1 = c.CI + G.loc1;
+    gp<const int> loc2 = c.CI + G.loc2;
+    gp<const int> t1 = c.CI + G.type1;
+    gp<const int> t2 = c.CI + G.type2;
+    gp<const float> P1 = c.A + G.out1;
+    gp<const float> P2 = c.A + G.out2;
+    const int E = uni(c.I[G.state + 3]);
     const int cap = G.ecap;
     for (int s = c.gtid; s < E; s += c.gsize) {
         int i1 = row[s], j = nbr[s];
@@ -664,10 +684,10 @@ __device__ void pg_edges_impl(Ctx& c, const PairGraph& G, const OpRec& op, P par
 // Stage the graph's coefficient table in this workgroup's LDS when it has one
 // that fits, then evaluate.
 template <int KIND, int DD1, int DD2>
-__device__ void pg_edges_t(Ctx& c, const PairGraph& G, const OpRec& op) {
-    gp<const float> src = gmem(c.CF + G.param);
+__device__ __forceinline__ void pg_edges_t(Ctx& c, GraphC& G, OpC& op) {
+    gp<const float> src = c.CF + G.param;
     if (G.param_len > 0) {
-        lp<float> L = lmem(c.lds);
+        lp<float> L = c.lds;
         for (int k = c.tid; k < G.param_len; k += NT) L[k] = src[k];
         __syncthreads();
         pg_edges_impl<KIND, DD1, DD2>(c, G, op, (lp<const float>)L);
@@ -676,7 +696,7 @@ __device__ void pg_edges_t(Ctx& c, const PairGraph& G, const OpRec& op) {
     }
 }
 
-__device__ void pg_edges(Ctx& c, const PairGraph& G, const OpRec& op) {
+__device__ __forceinline__ void pg_edges(Ctx& c, GraphC& G, OpC& op) {
     switch (G.kind) {
     case EDGE_ROTAMER: pg_edges_t<EDGE_ROTAMER, 6, 6>(c, G, op); break;
     case EDGE_HBOND_COVERAGE: pg_edges_t<EDGE_HBOND_COVERAGE, 7, 6>(c, G, op); break;
@@ -694,18 +714,18 @@ constexpr int GW = 16;
 static_assert(GW <= 32 && (GW & (GW - 1)) == 0, "a lane group is a power of two within half a wave");
 
 template <int D1N, int D2N>
-__device__ void pg_gather_t(Ctx& c, const PairGraph& G) {
-    gp<const int> off = gmem((const int*)c.I + G.off);
-    gp<const int> toff = gmem((const int*)c.I + G.toff);
-    gp<const int> tslot = gmem((const int*)c.I + G.tslot);
-    gp<const int> act = gmem((const int*)c.I + G.act);
-    gp<const float> es = gmem((const float*)c.A + G.esens);
-    gp<const float> D1 = gmem((const float*)c.A + G.d1);
-    gp<const float> D2 = gmem((const float*)c.A + G.d2);
-    gp<const int> loc1 = gmem(c.CI + G.loc1);
-    gp<const int> loc2 = gmem(c.CI + G.loc2);
-    gp<float> S1 = gmem(c.A + G.sens1);
-    gp<float> S2 = gmem(c.A + G.sens2);
+__device__ __forceinline__ void pg_gather_t(Ctx& c, GraphC& G) {
+    gp<const int> off = c.I + G.off;
+    gp<const int> toff = c.I + G.toff;
+    gp<const int> tslot = c.I + G.tslot;
+    gp<const int> act = c.I + G.act;
+    gp<const float> es = c.A + G.esens;
+    gp<const float> D1 = c.A + G.d1;
+    gp<const float> D2 = c.A + G.d2;
+    gp<const int> loc1 = c.CI + G.loc1;
+    gp<const int> loc2 = c.CI + G.loc2;
+    gp<float> S1 = c.A + G.sens1;
+    gp<float> S2 = c.A + G.sens2;
     const int cap = G.ecap;
     int grp = c.gtid / GW, gl = c.gtid % GW;
     const int NG = c.gsize / GW;
@@ -782,7 +802,7 @@ __device__ void pg_gather_t(Ctx& c, const PairGraph& G) {
     team_sync(c);
 }
 
-__device__ void pg_gather(Ctx& c, const PairGraph& G) {
+__device__ __forceinline__ void pg_gather(Ctx& c, GraphC& G) {
     unsigned long long t0 = ptick(c);
     switch (G.kind) {
     case EDGE_HBOND_COVERAGE: pg_gather_t<7, 6>(c, G); break;
@@ -795,10 +815,10 @@ __device__ void pg_gather(Ctx& c, const PairGraph& G) {
 // Sum of the active edge values of each row (side 1) or transposed row
 // (side 2), in slot order: out[k*stride] = sum.  Groups of 16 lanes.
 template <class O>
-__device__ void pg_row_sums(Ctx& c, const PairGraph& G, bool side2, O out, int stride) {
-    gp<const int> off = gmem((const int*)c.I + (side2 ? G.toff : G.off));
-    gp<const int> tslot = gmem((const int*)c.I + G.tslot);
-    gp<const float> val = gmem((const float*)c.A + G.val);
+__device__ __forceinline__ void pg_row_sums(Ctx& c, GraphC& G, bool side2, O out, int stride) {
+    gp<const int> off = c.I + (side2 ? G.toff : G.off);
+    gp<const int> tslot = c.I + G.tslot;
+    gp<const float> val = c.A + G.val;
     int n = side2 ? G.n2 : G.n1;
     int grp = c.gtid / GW, gl = c.gtid % GW;
     for (int base = 0; base < n; base += c.gsize / GW) {
@@ -814,19 +834,6 @@ __device__ void pg_row_sums(Ctx& c, const PairGraph& G, bool side2, O out, int s
         acc = group_sum<GW>(acc);
         if (ok && gl == 0) out[r * stride] = acc;
     }
-}
-
-// Prepare a graph for an evaluation: pack, maybe rebuild, refine and evaluate.
-// Returns false when the slot capacity overflowed (the evaluation is void).
-__device__ bool pg_refresh(Ctx& c, const PairGraph& G, const OpRec& op) {
-    unsigned long long t0 = ptick(c);
-    if (pg_pack_and_check(c, G)) pg_rebuild(c, G);
-    pacc(c, PROF_PG_REBUILD, t0);
-    if (!c.I[G.state + 0]) return false;
-    t0 = ptick(c);
-    pg_edges(c, G, op);
-    pacc(c, PROF_PG_EDGES, t0);
-    return true;
 }
 
 }  // namespace upside

@@ -32,19 +32,19 @@ struct RotView {
     int cap;
 };
 
-__device__ RotView rot_view(Ctx& c, const RotamerDev& R) {
+__device__ __forceinline__ RotView rot_view(Ctx& c, RotC& R) {
     RotView v;
-    v.nrot = gmem(c.CI + R.node_nrot); v.bead0 = gmem(c.CI + R.node_bead0); v.brot = gmem(c.CI + R.bead_rot);
-    v.bnode = gmem(c.CI + R.bead_node);
-    v.coff = gmem(c.I + R.coff); v.ca = gmem(c.I + R.ca); v.cb = gmem(c.I + R.cb); v.scand = gmem(c.I + R.slot_cand);
-    v.ioff = gmem(c.I + R.ioff); v.iinc = gmem(c.I + R.iinc); v.eidx = gmem(c.I + R.eidx);
-    v.bpc = gmem(c.I + R.bpc); v.bpf = gmem(c.I + R.bpf); v.bps = gmem(c.I + R.bps); v.ninc = gmem(c.I + R.ninc);
-    v.binc = gmem(c.I + R.binc); v.stats = gmem(c.I + R.stats);
-    v.P = gmem(c.A + R.P); v.msg = gmem(c.A + R.msg); v.marg = gmem(c.A + R.marg); v.e1x = gmem(c.A + R.e1x);
-    v.nprob = gmem(c.A + R.nprob); v.ncur = gmem(c.A + R.ncur); v.nold = gmem(c.A + R.nold);
-    v.noff = gmem(c.A + R.noff);
-    v.feat = gmem(c.A + R.feat);
-    v.nprev = gmem(c.A + R.nprev);
+    v.nrot = c.CI + R.node_nrot; v.bead0 = c.CI + R.node_bead0; v.brot = c.CI + R.bead_rot;
+    v.bnode = c.CI + R.bead_node;
+    v.coff = c.I + R.coff; v.ca = c.I + R.ca; v.cb = c.I + R.cb; v.scand = c.I + R.slot_cand;
+    v.ioff = c.I + R.ioff; v.iinc = c.I + R.iinc; v.eidx = c.I + R.eidx;
+    v.bpc = c.I + R.bpc; v.bpf = c.I + R.bpf; v.bps = c.I + R.bps; v.ninc = c.I + R.ninc;
+    v.binc = c.I + R.binc; v.stats = c.I + R.stats;
+    v.P = c.A + R.P; v.msg = c.A + R.msg; v.marg = c.A + R.marg; v.e1x = c.A + R.e1x;
+    v.nprob = c.A + R.nprob; v.ncur = c.A + R.ncur; v.nold = c.A + R.nold;
+    v.noff = c.A + R.noff;
+    v.feat = c.A + R.feat;
+    v.nprev = c.A + R.nprev;
     v.cap = R.ccap;
     return v;
 }
@@ -54,7 +54,7 @@ __device__ RotView rot_view(Ctx& c, const RotamerDev& R) {
 // handled by a 16-lane group testing 16 partners at a time (ballot
 // compaction keeps partner order).  Returns false on capacity overflow.
 template <class P>
-__device__ bool rot_candidate_lists(Ctx& c, const PairGraph& G, const RotamerDev& R, const RotView& v, P cen) {
+__device__ __forceinline__ bool rot_candidate_lists(Ctx& c, GraphC& G, RotC& R, const RotView& v, P cen) {
     const int n = R.n_node;
     const float rc = G.cache_cut;
     auto near = [&](int a, int b) {
@@ -139,12 +139,12 @@ __device__ bool rot_candidate_lists(Ctx& c, const PairGraph& G, const RotamerDev
 // incidence list of node x names (candidate, 1) for partners a < x first, in
 // increasing a, then (candidate, 0) for its own candidates.  Returns false on
 // capacity overflow.
-__device__ bool rot_rebuild(Ctx& c, const PairGraph& G, const RotamerDev& R) {
+__device__ __forceinline__ bool rot_rebuild(Ctx& c, GraphC& G, RotC& R) {
     RotView v = rot_view(c, R);
-    gp<const float> pack = gmem((const float*)c.A + G.pos_pack);
-    gp<float> cen = gmem(c.A + R.ncen);
-    gp<const int> row = gmem((const int*)c.I + G.row);
-    gp<const int> nbr = gmem((const int*)c.I + G.nbr);
+    gp<const float> pack = c.A + G.pos_pack;
+    gp<float> cen = c.A + R.ncen;
+    gp<const int> row = c.I + G.row;
+    gp<const int> nbr = c.I + G.nbr;
     const int n = R.n_node;
     for (int a = c.gtid; a < n; a += c.gsize) {
         int b0 = v.bead0[a], b1 = v.bead0[a + 1];
@@ -163,7 +163,7 @@ __device__ bool rot_rebuild(Ctx& c, const PairGraph& G, const RotamerDev& R) {
     // every workgroup reads the spheres from its own LDS copy when they fit
     bool ok;
     if (4 * n <= LDS_FLOATS) {
-        lp<float> L = lmem(c.lds);
+        lp<float> L = c.lds;
         for (int k = c.tid; k < 4 * n; k += NT) L[k] = cen[k];
         __syncthreads();
         ok = rot_candidate_lists(c, G, R, v, (lp<const float>)L);
@@ -172,7 +172,7 @@ __device__ bool rot_rebuild(Ctx& c, const PairGraph& G, const RotamerDev& R) {
     }
     if (!ok) return false;
     // candidate of every bead slot
-    const int E = c.I[G.state + 3];
+    const int E = uni(c.I[G.state + 3]);
     int bad = 0;
     for (int s = c.gtid; s < E; s += c.gsize) {
         int a = v.bnode[row[s]], b = v.bnode[nbr[s]];
@@ -193,18 +193,18 @@ __device__ bool rot_rebuild(Ctx& c, const PairGraph& G, const RotamerDev& R) {
 }
 
 // Node probabilities, BP-edge compaction and edge matrices for this evaluation.
-__device__ void rot_fill(Ctx& c, const PairGraph& G, const RotamerDev& R) {
+__device__ __forceinline__ void rot_fill(Ctx& c, GraphC& G, RotC& R) {
     RotView v = rot_view(c, R);
-    const int* off = c.I + G.off;
-    const int* nbr = c.I + G.nbr;
-    const int* row = c.I + G.row;
-    const int* toff = c.I + G.toff;
-    const int* tslot = c.I + G.tslot;
-    const int* act = c.I + G.act;
-    const float* val = c.A + G.val;
-    const int* loc1 = c.CI + G.loc1;
-    const int E = c.I[G.state + 3];
-    const int C = v.coff[R.n_node];
+    gp<const int> off = c.I + G.off;
+    gp<const int> nbr = c.I + G.nbr;
+    gp<const int> row = c.I + G.row;
+    gp<const int> toff = c.I + G.toff;
+    gp<const int> tslot = c.I + G.tslot;
+    gp<const int> act = c.I + G.act;
+    gp<const float> val = c.A + G.val;
+    gp<const int> loc1 = c.CI + G.loc1;
+    const int E = uni(c.I[G.state + 3]);
+    const int C = uni(v.coff[R.n_node]);
     // energies of each bead's edges to 1-rotamer residues (folded into the node)
     {
         int grp = c.gtid / GW, gl = c.gtid % GW;
@@ -419,7 +419,7 @@ __device__ __forceinline__ void rot_edge_cls(const BpMem<F, I, J>& m, int cls, c
 // e+nt together when they are of one class (edges sorted by class keep most
 // waves on one code path).
 template <bool TEAM, class F, class I, class J>
-__device__ void rot_edge_pass(Ctx& c, const BpMem<F, I, J>& m, int nbp, F nold_) {
+__device__ __forceinline__ void rot_edge_pass(Ctx& c, const BpMem<F, I, J>& m, int nbp, F nold_) {
     auto cls = [&](int k) { return k < m.c1 ? 0 : (k < m.c2 ? 1 : 2); };
     const int nt = bp_nt<TEAM>(c);
     int e = bp_t<TEAM>(c);
@@ -488,7 +488,7 @@ __device__ __forceinline__ void bp_node_store(int x, const float* pr, const floa
 }
 
 template <bool TEAM, class F, class I, class J>
-__device__ void rot_node_pass(Ctx& c, const BpMem<F, I, J>& m, int n_node, F ncur_, F nold_, float damping,
+__device__ __forceinline__ void rot_node_pass(Ctx& c, const BpMem<F, I, J>& m, int n_node, F ncur_, F nold_, float damping,
                               bool swap_first) {
     if (TEAM) {
         const int t = bp_t<TEAM>(c), gl = t % NODE_LANES;
@@ -567,7 +567,7 @@ __device__ void rot_node_pass(Ctx& c, const BpMem<F, I, J>& m, int n_node, F ncu
 // need one team barrier instead of two.  Results equal rot_edge_pass +
 // rot_node_pass.
 template <class F, class I, class J>
-__device__ void rot_fused_pass(Ctx& c, const BpMem<F, I, J>& m, gp<const float> min_, gp<float> mout, int n_node,
+__device__ __forceinline__ void rot_fused_pass(Ctx& c, const BpMem<F, I, J>& m, gp<const float> min_, gp<float> mout, int n_node,
                                F ncur_, F nold_, float damping, bool swap_first) {
     const int t = c.gtid, gl = t % NODE_LANES;
     for (int x = t / NODE_LANES; x < n_node; x += c.gsize / NODE_LANES) {  // uniform in a group
@@ -635,7 +635,7 @@ __device__ void rot_fused_pass(Ctx& c, const BpMem<F, I, J>& m, gp<const float> 
 //   rest 0.
 // Nodes with one state get a row of zeros.
 template <bool TEAM, class F, class I, class J>
-__device__ void bp_features(Ctx& c, const BpMem<F, I, J>& m, int n_node, F b0, gp<const float> prev,
+__device__ __forceinline__ void bp_features(Ctx& c, const BpMem<F, I, J>& m, int n_node, F b0, gp<const float> prev,
                             gp<float> feat) {
     for (int x = bp_t<TEAM>(c); x < n_node; x += bp_nt<TEAM>(c)) {
         float f[MLP_IN];
@@ -688,7 +688,7 @@ __device__ void bp_features(Ctx& c, const BpMem<F, I, J>& m, int n_node, F b0, g
 // beliefs of node x are exp(z_r - max z), z_r = feat[6 + r] + out_r over its
 // states (max-normalised, as the damped update leaves beliefs), into cur.
 template <bool TEAM, class F, class I, class J>
-__device__ void bp_warm_beliefs(Ctx& c, const BpMem<F, I, J>& m, const MlpDev& w, int n_node,
+__device__ __forceinline__ void bp_warm_beliefs(Ctx& c, const BpMem<F, I, J>& m, const MlpDev& w, int n_node,
                                 gp<const float> feat, F cur) {
     const int t = bp_t<TEAM>(c), nw = bp_nt<TEAM>(c) / 64;
     const int l = t & 63, g = l >> 4, cl = l & 15;
@@ -724,7 +724,7 @@ __device__ void bp_warm_beliefs(Ctx& c, const BpMem<F, I, J>& m, const MlpDev& w
 // from the other side's cavity belief b / message, scaled to unit L1 norm,
 // as in rot_edge_w).  Every edge on the 6x6 path (padding is zero).
 template <bool TEAM, class F, class I, class J>
-__device__ void bp_local_messages(Ctx& c, const BpMem<F, I, J>& m, int nbp, F b, int K) {
+__device__ __forceinline__ void bp_local_messages(Ctx& c, const BpMem<F, I, J>& m, int nbp, F b, int K) {
     for (int e = bp_t<TEAM>(c); e < nbp; e += bp_nt<TEAM>(c)) {
         const int ends = m.ends[e];
         const int f = ends & 0xFFFF, s = ends >> 16;
@@ -772,7 +772,7 @@ __device__ void bp_local_messages(Ctx& c, const BpMem<F, I, J>& m, int nbp, F b,
 
 // The plain start: messages 1, old beliefs = probabilities (:1110-1133).
 template <bool TEAM, class F, class I, class J>
-__device__ void bp_plain_start(Ctx& c, const BpMem<F, I, J>& m, int nbp, int n_node, F old) {
+__device__ __forceinline__ void bp_plain_start(Ctx& c, const BpMem<F, I, J>& m, int nbp, int n_node, F old) {
     for (int e = bp_t<TEAM>(c); e < nbp; e += bp_nt<TEAM>(c))
 #pragma unroll
         for (int r = 0; r < 12; ++r) m.msg[m.mi(r, e)] = 1.f;
@@ -794,7 +794,7 @@ __device__ void bp_plain_start(Ctx& c, const BpMem<F, I, J>& m, int nbp, int n_n
 // restart.  Schedules 1-3 also leave the features of the
 // first pass in R.feat (training rows for the network).
 template <bool TEAM, class F, class I, class J>
-__device__ int bp_iterate(Ctx& c, const RotamerDev& R, const RotView& v, const BpMem<F, I, J>& m, int nbp, F cur,
+__device__ __forceinline__ int bp_iterate(Ctx& c, RotC& R, const RotView& v, const BpMem<F, I, J>& m, int nbp, F cur,
                           F old) {
     const int n = R.n_node;
     const int cap = v.cap;
@@ -808,7 +808,7 @@ __device__ int bp_iterate(Ctx& c, const RotamerDev& R, const RotView& v, const B
     // buffer holding the current messages.
     BpMem<F, I, J> mm = m;
     F other{};
-    if constexpr (TEAM) other = gmem(c.A + R.msg2);
+    if constexpr (TEAM) other = c.A + R.msg2;
     // The first (undamped) pass writes the product into `old`, which the
     // fused pass's message updates are still reading: it keeps two phases.
     auto iterate = [&](F cur_, F old_, float damping, bool swap_first) {
@@ -832,7 +832,9 @@ __device__ int bp_iterate(Ctx& c, const RotamerDev& R, const RotView& v, const B
         if (mode > 0 && total == 0)  // old: the first pass's product
             bp_features<TEAM>(c, mm, n, old, (gp<const float>)v.nprev, v.feat);
         if (warm) {
-            bp_warm_beliefs<TEAM>(c, mm, c.args->mlp, n, (gp<const float>)v.feat, cur);
+            const auto& w = c.args->mlp;
+            const MlpDev net = {w.w1, w.w2p, w.w3p, w.w3tp, w.w2tp, w.b1, w.b2, w.b3};
+            bp_warm_beliefs<TEAM>(c, mm, net, n, (gp<const float>)v.feat, cur);
             bp_local_messages<TEAM>(c, mm, nbp, cur, c.args->bp_klocal);
         }
         const float tol = resid || (mode == 3 && c.args->bp_residual > 0.f) ? c.args->bp_residual : R.tol;
@@ -872,7 +874,7 @@ __device__ int bp_iterate(Ctx& c, const RotamerDev& R, const RotView& v, const B
     unsigned long long t0 = ptick(c);
     // node marginals (:283-290) into memory and into `old` (free now; cur and
     // old are always distinct buffers)
-    gp<float> ncur = gmem(v.ncur);
+    gp<float> ncur = v.ncur;
     for (int x = t; x < n; x += nt) {
         int nr = m.nrot[x];
         float b[6];
@@ -887,7 +889,7 @@ __device__ int bp_iterate(Ctx& c, const RotamerDev& R, const RotView& v, const B
     }
     bp_sync<TEAM>(c);
     // edge marginals (:425-449), written in the order of the BP edges
-    gp<float> marg = gmem(v.marg);
+    gp<float> marg = v.marg;
     for (int e = t; e < nbp; e += nt) {
         const int k = m.pos ? m.pos[e] : e;
         const int ends = m.ends[k];
@@ -936,15 +938,15 @@ __device__ __forceinline__ bool bp_fits_lds(int nbp, int n, int cap) {
 // (3x3, 3x6, 6x6; stable) and their matrices copied in that order into the
 // memory message area, which the LDS solve does not use.  Returns the
 // iteration count.
-__device__ int rot_solve_wg(Ctx& c, const RotamerDev& R) {
+__device__ __forceinline__ int rot_solve_wg(Ctx& c, RotC& R) {
     RotView v = rot_view(c, R);
-    const int nbp = v.stats[4];
+    const int nbp = uni(v.stats[4]);
     const int n = R.n_node;
     const int cap = v.cap;
     unsigned long long t0 = ptick(c);
     if (bp_fits_lds(nbp, n, cap)) {
         if (c.tid == 0) v.stats[6] += 1;  // solves held in LDS
-        lp<float> L = lmem(c.lds);
+        lp<float> L = c.lds;
         BpMem<lp<float>, lp<int>, lp<unsigned short>> m;
         m.nrot = v.nrot; m.prob = (gp<const float>)v.nprob;
         m.msg = L; m.ms = nbp; L += 12 * nbp;
@@ -1030,9 +1032,9 @@ __device__ int rot_solve_wg(Ctx& c, const RotamerDev& R) {
 // beliefs, incidences): every pass is spread over all the team's threads and
 // separated by team barriers.  Every thread of the team returns the
 // iteration count.
-__device__ int rot_solve_team(Ctx& c, const RotamerDev& R) {
+__device__ __forceinline__ int rot_solve_team(Ctx& c, RotC& R) {
     RotView v = rot_view(c, R);
-    const int nbp = v.stats[4];
+    const int nbp = uni(v.stats[4]);
     const int n = R.n_node;
     unsigned long long t0 = ptick(c);
     BpMem<gp<float>, gp<int>, gp<int>> m;
@@ -1056,7 +1058,7 @@ __device__ int rot_solve_team(Ctx& c, const RotamerDev& R) {
 // the team has one workgroup, else several; 1: always the whole team; 2:
 // always one workgroup; 3: always several.  Uniform over the team (nbp is
 // read after a team barrier).
-__device__ __forceinline__ bool bp_on_one_wg(const Ctx& c, const RotamerDev& R, int nbp, int bp_layout) {
+__device__ __forceinline__ bool bp_on_one_wg(const Ctx& c, RotC& R, int nbp, int bp_layout) {
     if (c.G == 1 || bp_layout == 2) return true;
     if (bp_layout == 1 || bp_layout == 3) return false;
     return bp_fits_lds(nbp, R.n_node, R.ccap);
@@ -1064,8 +1066,8 @@ __device__ __forceinline__ bool bp_on_one_wg(const Ctx& c, const RotamerDev& R, 
 
 // Solve by rank 0 of the team while the others wait at the barrier, or by
 // the whole team (see bp_on_one_wg).
-__device__ int rot_solve(Ctx& c, const RotamerDev& R, int bp_layout) {
-    const int nbp = c.I[R.stats + 4];
+__device__ __forceinline__ int rot_solve(Ctx& c, RotC& R, int bp_layout) {
+    const int nbp = uni(c.I[R.stats + 4]);
     if (!bp_on_one_wg(c, R, nbp, bp_layout)) return rot_solve_team(c, R);
     int it = 0;
     if (c.rank == 0) it = rot_solve_wg(c, R);
@@ -1074,7 +1076,7 @@ __device__ int rot_solve(Ctx& c, const RotamerDev& R, int bp_layout) {
 }
 
 // Bethe free energy (calculate_energy_from_marginals, :915-927).
-__device__ float rot_free_energy(Ctx& c, const PairGraph& G, const RotamerDev& R) {
+__device__ __forceinline__ float rot_free_energy(Ctx& c, GraphC& G, RotC& R) {
     RotView v = rot_view(c, R);
     const int cap = v.cap;
     float en = 0.f;
@@ -1088,14 +1090,14 @@ __device__ float rot_free_energy(Ctx& c, const PairGraph& G, const RotamerDev& R
         en += e;
     }
     // 1-rotamer pairs: -log P with P the probability of their single bead pair
-    const int* row = c.I + G.row;
-    const int* nbr = c.I + G.nbr;
-    const int* act = c.I + G.act;
-    const float* val = c.A + G.val;
-    const int E = c.I[G.state + 3];
+    gp<const int> row = c.I + G.row;
+    gp<const int> nbr = c.I + G.nbr;
+    gp<const int> act = c.I + G.act;
+    gp<const float> val = c.A + G.val;
+    const int E = uni(c.I[G.state + 3]);
     for (int s = c.gtid; s < E; s += c.gsize)
         if (act[s] && v.nrot[v.bnode[row[s]]] == 1 && v.nrot[v.bnode[nbr[s]]] == 1) en += -logf(expf(-val[s]));
-    const int nbp = v.stats[4];
+    const int nbp = uni(v.stats[4]);
     for (int e = c.gtid; e < nbp; e += c.gsize) {
         int f = v.bpf[e], s = v.bps[e];
 #pragma unroll
@@ -1112,14 +1114,14 @@ __device__ float rot_free_energy(Ctx& c, const PairGraph& G, const RotamerDev& R
 
 // Edge sensitivities of bead pairs (src/rotamer.cpp:1057-1066) and the 1-body
 // sensitivities (:1074-1085).
-__device__ void rot_sens(Ctx& c, const PairGraph& G, const RotamerDev& R) {
+__device__ __forceinline__ void rot_sens(Ctx& c, GraphC& G, RotC& R) {
     RotView v = rot_view(c, R);
-    const int* row = c.I + G.row;
-    const int* nbr = c.I + G.nbr;
-    const int* act = c.I + G.act;
-    float* es = c.A + G.esens;
-    const int* loc1 = c.CI + G.loc1;
-    const int E = c.I[G.state + 3];
+    gp<const int> row = c.I + G.row;
+    gp<const int> nbr = c.I + G.nbr;
+    gp<const int> act = c.I + G.act;
+    gp<float> es = c.A + G.esens;
+    gp<const int> loc1 = c.CI + G.loc1;
+    const int E = uni(c.I[G.state + 3]);
     const int cap = v.cap;
     for (int s = c.gtid; s < E; s += c.gsize) {
         if (!act[s]) { es[s] = 0.f; continue; }

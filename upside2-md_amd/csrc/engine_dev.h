@@ -1,6 +1,6 @@
 // Device-side data model of the MI355X Upside engine.
 //
-// One system (a chain replica) is evaluated by one workgroup.  The node graph
+// One system (a chain replica) is evaluated by a team of workgroups.  The node graph
 // of a `.up` file (src/deriv_engine.cpp:353-426) is lowered on the host into a
 // program of OpRec records; the persistent kernel interprets the program in
 // germ order (values) and deriv order (sensitivity pushes), mirroring
@@ -13,11 +13,11 @@
 
 namespace upside {
 
-// Dynamic LDS per workgroup (159 KB of the 160 KB a gfx950 workgroup may
-// hold, the rest being the static reduction scratch): staging for pair-graph
+// Dynamic LDS per workgroup (158 KB of the 160 KB a gfx950 workgroup may
+// hold, the rest being the static reduction scratch and the waves' contexts): staging for pair-graph
 // coefficient tables (the largest, the rotamer pair table, is 20*20*54 floats
 // = 86.4 KB, plus read-past padding), cell grids, and the rotamer solve state.
-constexpr int LDS_FLOATS = 40704;
+constexpr int LDS_FLOATS = 40448;
 // Rotamer statistics words: [0] iterations of the last solve, [1] solves at
 // the iteration limit, [2] total iterations, [3] solves, [4] BP edges, [5]
 // residue-pair candidates, [6] solves held in LDS, [7] warm-started solves,
@@ -201,6 +201,8 @@ struct OpRec {
     int early;             // deriv op that may run beside the rotamer solve, after its overlap ops
     int rot_graph_op;      // first op of a section: the rotamer op whose pair-list refresh and edge
     int rot_graph_lane;    // evaluation lane rot_graph_lane runs first (-1: none)
+    int lane_graphs;       // first op of a section, rotamer with an overlap range: it runs pair-graph ops
+                           // beside each other (their lists may overflow, so the error words are read)
 };
 
 struct SysDesc {

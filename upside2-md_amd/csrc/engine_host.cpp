@@ -1670,6 +1670,12 @@ struct Program {
             for (size_t d = 0; d < T.deriv.size(); ++d) any = any || prog[ng + d].early;
             if (!any) prog[k].overlap_end = 0;
         }
+        for (int k = 0; k < ng; ++k) {
+            prog[k].lane_graphs = prog[k].lane_end > k && prog[k].rot_graph_op >= 0;
+            const int e = std::max(prog[k].lane_end, prog[k].kind == OP_ROTAMER ? prog[k].overlap_end : 0);
+            for (int q = prog[k].kind == OP_ROTAMER ? k + 1 : k; q < e; ++q)
+                if (prog[q].graph >= 0) prog[k].lane_graphs = 1;
+        }
         if (!upload) return;  // lowering only (check_program)
         auto up = [](void** dst, const void* src, size_t bytes, const char* what) {
             hip_check(hipMalloc(dst, std::max(bytes, (size_t)16)), what);

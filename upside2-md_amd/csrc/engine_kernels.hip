@@ -1,7 +1,7 @@
 // Persistent force-and-integration kernel of the MI355X Upside engine.
 //
-// One workgroup evaluates one system: it interprets the lowered node program
-// (value pass in germ order, sensitivity pass in deriv order, as
+// A team of workgroups evaluates one system: it interprets the lowered node
+// program (value pass in germ order, sensitivity pass in deriv order, as
 // DerivEngine::compute, src/deriv_engine.cpp:239-260), then applies the
 // symplectic-Euler stages of integration_cycle (src/deriv_engine.cpp:317-331)
 // and the Ornstein-Uhlenbeck thermostat (src/thermostat.cpp:9-18), for many
@@ -11,13 +11,13 @@
 
 namespace upside {
 
-// operand pointers, typed as global memory (see gmem)
-#define OUT(op) gmem(c.A + (op).out)
-#define SENS(op) gmem(c.A + (op).sens)
-#define IN(op, k) gmem(c.A + (op).in_out[k])
-#define INS(op, k) gmem(c.A + (op).in_sens[k])
-#define CIA(op, k) gmem(c.CI + (op).ia[k])
-#define CFA(op, k) gmem(c.CF + (op).ia[k])
+// operand pointers
+#define OUT(op) (c.A + (op).out)
+#define SENS(op) (c.A + (op).sens)
+#define IN(op, k) (c.A + (op).in_out[k])
+#define INS(op, k) (c.A + (op).in_sens[k])
+#define CIA(op, k) (c.CI + (op).ia[k])
+#define CFA(op, k) (c.CF + (op).ia[k])
 
 // Profile accumulation (op slots by index, fixed slots through pacc).
 __device__ __forceinline__ void prof_op(const Ctx& c, int slot, unsigned long long t0) {
@@ -25,14 +25,14 @@ __device__ __forceinline__ void prof_op(const Ctx& c, int slot, unsigned long lo
         __hip_atomic_fetch_add(c.prof + slot, wall_clock64() - t0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__device__ __forceinline__ void put_pot(Ctx& c, const SysDesc& S, const OpRec& op, float e) {
+__device__ __forceinline__ void put_pot(Ctx& c, SysC& S, OpC& op, float e) {
     if (c.gtid == 0) c.A[S.pot + op.pot_slot] = e;
 }
 
 // ---- Distance3D (src/coord_basic.cpp:13-66) --------------------------------
-__device__ void dist3d_fwd(Ctx& c, const OpRec& op) {
+__device__ __forceinline__ void dist3d_fwd(Ctx& c, OpC& op) {
     auto id = CIA(op, 0);
-    auto der = gmem(c.A + op.scratch);
+    auto der = c.A + op.scratch;
     for (int e = c.gtid; e < op.n_elem; e += c.gsize) {
         auto a = IN(op, 0) + id[2 * e] * op.in_w[0];
         auto b = IN(op, 1) + id[2 * e + 1] * op.in_w[1];
@@ -44,9 +44,9 @@ __device__ void dist3d_fwd(Ctx& c, const OpRec& op) {
         der[e * 3 + 0] = dx * inv; der[e * 3 + 1] = dy * inv; der[e * 3 + 2] = dz * inv;
     }
 }
-__device__ void dist3d_bwd(Ctx& c, const OpRec& op) {
-    auto der = gmem(c.A + op.scratch);
-    auto con = gmem(c.A + op.ia[1]);
+__device__ __forceinline__ void dist3d_bwd(Ctx& c, OpC& op) {
+    auto der = c.A + op.scratch;
+    auto con = c.A + op.ia[1];
     for (int e = c.gtid; e < op.n_elem; e += c.gsize) {
         float s = SENS(op)[e];
         for (int k = 0; k < 3; ++k) {
@@ -54,15 +54,12 @@ __device__ void dist3d_bwd(Ctx& c, const OpRec& op) {
             con[(e * 2 + 1) * 3 + k] = -s * der[e * 3 + k];
         }
     }
-    team_sync(c);
-    plan_gather(c, op.plans[0]);
-    plan_gather(c, op.plans[1]);
 }
 
 // ---- Angle: cosine at the third atom (src/coord_basic.cpp:183-243) ---------
-__device__ void angle_fwd(Ctx& c, const OpRec& op) {
+__device__ __forceinline__ void angle_fwd(Ctx& c, OpC& op) {
     auto id = CIA(op, 0);
-    auto der = gmem(c.A + op.scratch);
+    auto der = c.A + op.scratch;
     auto P = IN(op, 0);
     int w = op.in_w[0];
     for (int e = c.gtid; e < op.n_elem; e += c.gsize) {
@@ -83,9 +80,9 @@ __device__ void angle_fwd(Ctx& c, const OpRec& op) {
         }
     }
 }
-__device__ void angle_bwd(Ctx& c, const OpRec& op) {
-    auto der = gmem(c.A + op.scratch);
-    auto con = gmem(c.A + op.ia[1]);
+__device__ __forceinline__ void angle_bwd(Ctx& c, OpC& op) {
+    auto der = c.A + op.scratch;
+    auto con = c.A + op.ia[1];
     for (int e = c.gtid; e < op.n_elem; e += c.gsize) {
         float s = SENS(op)[e];
         for (int k = 0; k < 3; ++k) {
@@ -95,8 +92,6 @@ __device__ void angle_bwd(Ctx& c, const OpRec& op) {
             con[(e * 3 + 2) * 3 + k] = -d1 - d2;
         }
     }
-    team_sync(c);
-    plan_gather(c, op.plans[0]);
 }
 
 // ---- Dihedral (src/coord_basic.cpp:311-374, src/vector_math.h:764-797) -----
@@ -109,9 +104,9 @@ __device__ __forceinline__ void cross3(P a, Q b, O o) {
 template <class P, class Q>
 __device__ __forceinline__ float dot3(P a, Q b) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2]; }
 
-__device__ void dihedral_fwd(Ctx& c, const OpRec& op) {
+__device__ __forceinline__ void dihedral_fwd(Ctx& c, OpC& op) {
     auto id = CIA(op, 0);
-    auto jac = gmem(c.A + op.scratch);
+    auto jac = c.A + op.scratch;
     auto P = IN(op, 0);
     int w = op.in_w[0];
     for (int e = c.gtid; e < op.n_elem; e += c.gsize) {
@@ -144,25 +139,23 @@ __device__ void dihedral_fwd(Ctx& c, const OpRec& op) {
         OUT(op)[e] = atan2f(dot3(C, G), dot3(A, B) * Gm);
     }
 }
-__device__ void dihedral_bwd(Ctx& c, const OpRec& op) {
-    auto jac = gmem(c.A + op.scratch);
-    auto con = gmem(c.A + op.ia[1]);
+__device__ __forceinline__ void dihedral_bwd(Ctx& c, OpC& op) {
+    auto jac = c.A + op.scratch;
+    auto con = c.A + op.ia[1];
     for (int e = c.gtid; e < op.n_elem; e += c.gsize) {
         float s = SENS(op)[e];
         for (int k = 0; k < 12; ++k) con[e * 12 + k] = s * jac[e * 12 + k];
     }
-    team_sync(c);
-    plan_gather(c, op.plans[0]);
 }
 
 // ---- Spring (src/spring.cpp:9-81) -------------------------------------------
-__device__ void spring_fwd(Ctx& c, const SysDesc& S, const OpRec& op) {
+__device__ __forceinline__ void spring_fwd(Ctx& c, SysC& S, OpC& op) {
     auto id = CIA(op, 0);
     auto eq = CFA(op, 1);
     auto kk = CFA(op, 2);
     int dim1 = op.ia[3], pbc = op.ia[4], n = op.ia[5];
     float box = op.fa[0];
-    auto con = gmem(c.A + op.scratch);
+    auto con = c.A + op.scratch;
     float pot = 0.f;
     for (int e = c.gtid; e < n; e += c.gsize) {
         float x = IN(op, 0)[id[e] * op.in_w[0] + dim1];
@@ -178,11 +171,10 @@ __device__ void spring_fwd(Ctx& c, const SysDesc& S, const OpRec& op) {
     }
     pot = team_sum(c, pot);
     put_pot(c, S, op, pot);
-    plan_gather(c, op.plans[0]);
 }
 
 // ---- rama_coord / cat_pos (src/coord_map.cpp:69-161) -----------------------
-__device__ void rama_coord_fwd(Ctx& c, const OpRec& op) {
+__device__ __forceinline__ void rama_coord_fwd(Ctx& c, OpC& op) {
     auto i1 = CIA(op, 0);
     auto i2 = CIA(op, 1);
     for (int e = c.gtid; e < op.n_elem; e += c.gsize) {
@@ -190,7 +182,7 @@ __device__ void rama_coord_fwd(Ctx& c, const OpRec& op) {
         OUT(op)[2 * e + 1] = IN(op, 1)[i2[e] * op.in_w[1]];
     }
 }
-__device__ void cat_pos_fwd(Ctx& c, const OpRec& op) {
+__device__ __forceinline__ void cat_pos_fwd(Ctx& c, OpC& op) {
     auto idx = CIA(op, 0);
     int n1 = op.ia[1], w = op.width;
     for (int e = c.gtid; e < op.n_elem; e += c.gsize) {
@@ -199,19 +191,14 @@ __device__ void cat_pos_fwd(Ctx& c, const OpRec& op) {
         for (int d = 0; d < w; ++d) OUT(op)[e * w + d] = src[d];
     }
 }
-__device__ void passthrough_bwd(Ctx& c, const OpRec& op) {
-    plan_gather(c, op.plans[0]);
-    plan_gather(c, op.plans[1]);
-}
-
 // ---- rama_map_pot (src/rama_map_pot.cpp:15-94) -------------------------------
-__device__ void rama_map_fwd(Ctx& c, const SysDesc& S, const OpRec& op) {
+__device__ __forceinline__ void rama_map_fwd(Ctx& c, SysC& S, OpC& op) {
     auto res = CIA(op, 0);
     auto mid = CIA(op, 1);
     auto coef = CFA(op, 2);
     int nx = op.ia[3], n = op.ia[4];
     float scale = op.fa[0], shift = op.fa[1];
-    auto con = gmem(c.A + op.scratch);
+    auto con = c.A + op.scratch;
     float pot = 0.f;
     for (int e = c.gtid; e < n; e += c.gsize) {
         auto r = IN(op, 0) + res[e] * op.in_w[0];
@@ -227,7 +214,6 @@ __device__ void rama_map_fwd(Ctx& c, const SysDesc& S, const OpRec& op) {
     }
     pot = team_sum(c, pot);
     put_pot(c, S, op, pot);
-    plan_gather(c, op.plans[0]);
 }
 
 // ---- affine_alignment (src/eig.cpp:277-471) ----------------------------------
@@ -244,7 +230,7 @@ __device__ __forceinline__ bool quad_any(bool p) {
     return ((m >> (lane & ~3)) & 0xFull) != 0;
 }
 
-__device__ void eig4_grouped(float* A, float* d, float* rot) {
+__device__ __forceinline__ void eig4_grouped(float* A, float* d, float* rot) {
     float beta[2];
     for (int k = 0; k < 2; ++k) {
         int m = 3 - k;
@@ -332,11 +318,11 @@ __device__ void eig4_grouped(float* A, float* d, float* rot) {
     }
 }
 
-__device__ void affine_fwd(Ctx& c, const OpRec& op) {
+__device__ __forceinline__ void affine_fwd(Ctx& c, OpC& op) {
     auto atoms = CIA(op, 0);
     auto ref = CFA(op, 1);
-    auto ev = gmem(c.A + op.scratch);            // n*4 eigenvalues
-    auto ec = gmem(c.A + op.scratch + 4 * op.n_elem);  // n*16 eigenvector rows
+    auto ev = c.A + op.scratch;            // n*4 eigenvalues
+    auto ec = c.A + op.scratch + 4 * op.n_elem;  // n*16 eigenvector rows
     auto P = IN(op, 0);
     int w = op.in_w[0];
     int n = op.n_elem;
@@ -367,11 +353,11 @@ __device__ void affine_fwd(Ctx& c, const OpRec& op) {
         o[3] = rot[0]; o[4] = rot[1]; o[5] = rot[2]; o[6] = rot[3];
     }
 }
-__device__ void affine_bwd(Ctx& c, const OpRec& op) {
+__device__ __forceinline__ void affine_bwd(Ctx& c, OpC& op) {
     auto ref = CFA(op, 1);
-    auto ev = gmem(c.A + op.scratch);
-    auto ec = gmem(c.A + op.scratch + 4 * op.n_elem);
-    auto con = gmem(c.A + op.ia[2]);
+    auto ev = c.A + op.scratch;
+    auto ec = c.A + op.scratch + 4 * op.n_elem;
+    auto con = c.A + op.ia[2];
     for (int r = c.gtid; r < op.n_elem; r += c.gsize) {
         auto s = SENS(op) + r * 7;
         auto E = ec + r * 16;
@@ -409,12 +395,10 @@ __device__ void affine_bwd(Ctx& c, const OpRec& op) {
             }
         }
     }
-    team_sync(c);
-    plan_gather(c, op.plans[0]);
 }
 
 // ---- placement (src/placement.cpp:20-314) -------------------------------------
-__device__ void placement_fwd(Ctx& c, const OpRec& op) {
+__device__ __forceinline__ void placement_fwd(Ctx& c, OpC& op) {
     auto ares = CIA(op, 0);
     auto layer = CIA(op, 1);
     auto data = CFA(op, 2);
@@ -447,17 +431,15 @@ __device__ void placement_fwd(Ctx& c, const OpRec& op) {
         if (dim == 7) o[6] = v[6];
     }
 }
-__device__ void placement_bwd(Ctx& c, const OpRec& op) {
+__device__ __forceinline__ void placement_bwd(Ctx& c, OpC& op) {
     int is_rama = op.ia[3];
-    auto con = gmem(c.A + op.ia[8]);
+    auto con = c.A + op.ia[8];
     if (is_rama) {
         for (int e = c.gtid; e < op.n_elem; e += c.gsize) {
             float s = SENS(op)[e];
             con[2 * e] = s * c.A[op.scratch + 2 * e];
             con[2 * e + 1] = s * c.A[op.scratch + 2 * e + 1];
         }
-        team_sync(c);
-        plan_gather(c, op.plans[1]);
         return;
     }
     auto ares = CIA(op, 0);
@@ -476,15 +458,13 @@ __device__ void placement_bwd(Ctx& c, const OpRec& op) {
             con[e * 6 + 3 + k] = tq1[k] + tq2[k];
         }
     }
-    team_sync(c);
-    plan_gather(c, op.plans[0]);
 }
 
 // ---- infer_H_O (src/hbond.cpp:20-127) ------------------------------------------
-__device__ void infer_fwd(Ctx& c, const OpRec& op) {
+__device__ __forceinline__ void infer_fwd(Ctx& c, OpC& op) {
     auto id = CIA(op, 0);
     auto bl = CFA(op, 1);
-    auto cache = gmem(c.A + op.scratch);
+    auto cache = c.A + op.scratch;
     auto P = IN(op, 0);
     int w = op.in_w[0];
     for (int e = c.gtid; e < op.n_elem; e += c.gsize) {
@@ -502,10 +482,10 @@ __device__ void infer_fwd(Ctx& c, const OpRec& op) {
         for (int k = 0; k < 3; ++k) { o[k] = cc[k] - bl[e] * ds[k]; o[3 + k] = -ds[k]; }
     }
 }
-__device__ void infer_bwd(Ctx& c, const OpRec& op) {
+__device__ __forceinline__ void infer_bwd(Ctx& c, OpC& op) {
     auto bl = CFA(op, 1);
-    auto cache = gmem(c.A + op.scratch);
-    auto con = gmem(c.A + op.ia[2]);
+    auto cache = c.A + op.scratch;
+    auto con = c.A + op.ia[2];
     for (int e = c.gtid; e < op.n_elem; e += c.gsize) {
         auto s = SENS(op) + e * 6;
         auto cs = cache + e * 12;
@@ -524,25 +504,14 @@ __device__ void infer_bwd(Ctx& c, const OpRec& op) {
             con[(e * 3 + 2) * 3 + k] = sx[k];
         }
     }
-    team_sync(c);
-    plan_gather(c, op.plans[0]);
-}
-
-// A pair-graph capacity overflow voids the evaluation: the system's error
-// word is set, the remaining ops are skipped and the host grows the
-// capacities and repeats the run.
-__device__ void graph_overflow(Ctx& c, const SysDesc& S) {
-    if (c.gtid == 0) c.I[c.err] = 1;
-    team_sync(c);
 }
 
 // ---- protein_hbond (src/hbond.cpp:357-435) ---------------------------------------
-__device__ void protein_hbond_fwd(Ctx& c, const SysDesc& S, const OpRec& op, const PairGraph& G) {
-    if (!pg_refresh(c, G, op)) { graph_overflow(c, S); return; }
+__device__ __forceinline__ void protein_hbond_fwd(Ctx& c, OpC& op, GraphC& G) {
     int nd = G.n1;
-    auto loc1 = gmem(c.CI + G.loc1);
-    auto loc2 = gmem(c.CI + G.loc2);
-    auto ss = gmem(c.A + op.scratch);  // per-site sum of hb_log
+    auto loc1 = c.CI + G.loc1;
+    auto loc2 = c.CI + G.loc2;
+    auto ss = c.A + op.scratch;  // per-site sum of hb_log
     pg_row_sums(c, G, false, ss, 1);
     pg_row_sums(c, G, true, ss + nd, 1);
     team_sync(c);
@@ -556,21 +525,23 @@ __device__ void protein_hbond_fwd(Ctx& c, const SysDesc& S, const OpRec& op, con
         o[6] = 1.f - expf(-ss[v]);
     }
 }
-__device__ void protein_hbond_bwd(Ctx& c, const OpRec& op, const PairGraph& G) {
+__device__ __forceinline__ void protein_hbond_bwd(Ctx& c, OpC& op, GraphC& G) {
     int nd = G.n1;
-    auto ss = gmem(c.A + op.scratch);
+    auto ss = c.A + op.scratch;
     for (int v = c.gtid; v < op.n_elem; v += c.gsize) ss[v] = SENS(op)[v * 7 + 6] * (1.f - OUT(op)[v * 7 + 6]);
     team_sync(c);
-    auto row = gmem(c.I + G.row);
-    auto nbr = gmem(c.I + G.nbr);
-    auto es = gmem(c.A + G.esens);
-    const int E = c.I[G.state + 3];
+    auto row = c.I + G.row;
+    auto nbr = c.I + G.nbr;
+    auto es = c.A + G.esens;
+    const int E = uni(c.I[G.state + 3]);
     for (int s = c.gtid; s < E; s += c.gsize) es[s] = ss[row[s]] + ss[nd + nbr[s]];
-    team_sync(c);
-    pg_gather(c, G);
+}
+// After the gather of the hydrogen-bond edges.
+__device__ __forceinline__ void protein_hbond_pass(Ctx& c, OpC& op, GraphC& G) {
+    const int nd = G.n1;
     // pass the coordinate sensitivities through to infer_H_O (:419-433)
-    auto loc1 = gmem(c.CI + G.loc1);
-    auto loc2 = gmem(c.CI + G.loc2);
+    auto loc1 = c.CI + G.loc1;
+    auto loc2 = c.CI + G.loc2;
     for (int i = c.gtid; i < G.n1; i += c.gsize)
 #pragma unroll
         for (int k = 0; k < 6; ++k) INS(op, 0)[loc1[i] * op.in_w[0] + k] += SENS(op)[i * 7 + k];
@@ -582,23 +553,17 @@ __device__ void protein_hbond_bwd(Ctx& c, const OpRec& op, const PairGraph& G) {
 }
 
 // ---- hbond_coverage (src/hbond.cpp:438-484) ----------------------------------------
-__device__ void hbond_coverage_fwd(Ctx& c, const SysDesc& S, const OpRec& op, const PairGraph& G) {
-    if (!pg_refresh(c, G, op)) { graph_overflow(c, S); return; }
-    pg_row_sums(c, G, true, OUT(op), 1);
-}
-__device__ void hbond_coverage_bwd(Ctx& c, const OpRec& op, const PairGraph& G) {
-    auto nbr = gmem(c.I + G.nbr);
-    auto es = gmem(c.A + G.esens);
-    const int E = c.I[G.state + 3];
+__device__ __forceinline__ void hbond_coverage_bwd(Ctx& c, OpC& op, GraphC& G) {
+    auto nbr = c.I + G.nbr;
+    auto es = c.A + G.esens;
+    const int E = uni(c.I[G.state + 3]);
     for (int s = c.gtid; s < E; s += c.gsize) es[s] = SENS(op)[nbr[s]];
-    team_sync(c);
-    pg_gather(c, G);
 }
 
 // ---- hbond_energy (src/hbond.cpp:487-739) -------------------------------------------
 // ia: 0 n_res, 1 hb1 off (n_res+1), 2 hb1 idx, 3 hb2 off (n_res), 4 hb2 idx,
 //     5 first donor of residue, 6 first acceptor of residue (virtual index or -1)
-__device__ void hbond_energy_fwd(Ctx& c, const SysDesc& S, const OpRec& op) {
+__device__ __forceinline__ void hbond_energy_fwd(Ctx& c, SysC& S, OpC& op) {
     int n_res = op.ia[0];
     auto h1o = CIA(op, 1);
     auto h1i = CIA(op, 2);
@@ -655,7 +620,7 @@ __device__ void hbond_energy_fwd(Ctx& c, const SysDesc& S, const OpRec& op) {
 }
 
 // ---- weighted_pos (src/environment.cpp:489-533) -------------------------------------
-__device__ void weighted_pos_fwd(Ctx& c, const OpRec& op) {
+__device__ __forceinline__ void weighted_pos_fwd(Ctx& c, OpC& op) {
     auto ip = CIA(op, 0);
     auto iw = CIA(op, 1);
     for (int e = c.gtid; e < op.n_elem; e += c.gsize) {
@@ -665,32 +630,28 @@ __device__ void weighted_pos_fwd(Ctx& c, const OpRec& op) {
         o[3] = expf(-IN(op, 1)[iw[e] * op.in_w[1]]);
     }
 }
-__device__ void weighted_pos_bwd(Ctx& c, const OpRec& op) {
-    auto con = gmem(c.A + op.scratch);
+__device__ __forceinline__ void weighted_pos_bwd(Ctx& c, OpC& op) {
+    auto con = c.A + op.scratch;
     for (int e = c.gtid; e < op.n_elem; e += c.gsize) con[e] = -OUT(op)[e * 4 + 3] * SENS(op)[e * 4 + 3];
-    team_sync(c);
-    plan_gather(c, op.plans[0]);
-    plan_gather(c, op.plans[1]);
 }
 
 // ---- environment_coverage (src/environment.cpp:288-348) -----------------------------
 // Output row i holds the coverage of element i by each residue type: the
 // active edge values of its slots binned by the partner's amino-acid type.
-__device__ void env_coverage_fwd(Ctx& c, const SysDesc& S, const OpRec& op, const PairGraph& G) {
-    if (!pg_refresh(c, G, op)) { graph_overflow(c, S); return; }
+__device__ __forceinline__ void env_coverage_fwd(Ctx& c, OpC& op, GraphC& G) {
     int naa = op.ia[0];
     auto aa = CIA(op, 1);
-    auto id2 = gmem(c.CI + G.id2);
-    auto off = gmem(c.I + G.off);
-    auto nbr = gmem(c.I + G.nbr);
-    auto val = gmem(c.A + G.val);
-    auto act = gmem(c.I + G.act);
+    auto id2 = c.CI + G.id2;
+    auto off = c.I + G.off;
+    auto nbr = c.I + G.nbr;
+    auto val = c.A + G.val;
+    auto act = c.I + G.act;
     auto out = OUT(op);
     // one 16-lane group per element: each lane strides the element's slots
     // into its own type bins (LDS), then lane t of the group sums bin t over
     // the group's lanes in lane order
-    lp<float> mine = lmem(c.lds) + c.tid * naa;
-    lp<float> grp_bins = lmem(c.lds) + (c.tid & ~(GW - 1)) * naa;
+    lp<float> mine = c.lds + c.tid * naa;
+    lp<float> grp_bins = c.lds + (c.tid & ~(GW - 1)) * naa;
     const int grp = c.gtid / GW, gl = c.gtid % GW, NG = c.gsize / GW;
     for (int base = 0; base < G.n1; base += NG) {
         const int i = base + grp;
@@ -712,36 +673,28 @@ __device__ void env_coverage_fwd(Ctx& c, const SysDesc& S, const OpRec& op, cons
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
 }
-__device__ void env_coverage_bwd(Ctx& c, const OpRec& op, const PairGraph& G) {
+__device__ __forceinline__ void env_coverage_bwd(Ctx& c, OpC& op, GraphC& G) {
     int naa = op.ia[0];
     auto aa = CIA(op, 1);
-    auto id2 = gmem(c.CI + G.id2);
-    auto row = gmem(c.I + G.row);
-    auto nbr = gmem(c.I + G.nbr);
-    auto es = gmem(c.A + G.esens);
-    const int E = c.I[G.state + 3];
+    auto id2 = c.CI + G.id2;
+    auto row = c.I + G.row;
+    auto nbr = c.I + G.nbr;
+    auto es = c.A + G.esens;
+    const int E = uni(c.I[G.state + 3]);
     for (int s = c.gtid; s < E; s += c.gsize) es[s] = SENS(op)[row[s] * naa + aa[id2[nbr[s]]]];
-    team_sync(c);
-    pg_gather(c, G);
 }
 
 // ---- hb_environment_coverage (src/environment.cpp:350-385) ------------------------
-__device__ void hb_env_fwd(Ctx& c, const SysDesc& S, const OpRec& op, const PairGraph& G) {
-    if (!pg_refresh(c, G, op)) { graph_overflow(c, S); return; }
-    pg_row_sums(c, G, false, OUT(op), 1);
-}
-__device__ void hb_env_bwd(Ctx& c, const OpRec& op, const PairGraph& G) {
-    auto row = gmem(c.I + G.row);
-    auto es = gmem(c.A + G.esens);
-    const int E = c.I[G.state + 3];
+__device__ __forceinline__ void hb_env_bwd(Ctx& c, OpC& op, GraphC& G) {
+    auto row = c.I + G.row;
+    auto es = c.A + G.esens;
+    const int E = uni(c.I[G.state + 3]);
     for (int s = c.gtid; s < E; s += c.gsize) es[s] = SENS(op)[row[s]];
-    team_sync(c);
-    pg_gather(c, G);
 }
 
 // ---- sigmoid_coupling (src/environment.cpp:851-1003) -------------------------------
 // ia: 0 n_res, 1 coupling types, 2 weights (nt*nt), 3 scale, 4 center, 5 sharpness, 6 nt
-__device__ void sigmoid_coupling_fwd(Ctx& c, const SysDesc& S, const OpRec& op) {
+__device__ __forceinline__ void sigmoid_coupling_fwd(Ctx& c, SysC& S, OpC& op) {
     int n = op.ia[0], nt = op.ia[6];
     auto ct = CIA(op, 1);
     auto W = CFA(op, 2);
@@ -765,7 +718,7 @@ __device__ void sigmoid_coupling_fwd(Ctx& c, const SysDesc& S, const OpRec& op) 
 }
 
 // ---- bb_sigmoid_coupling (src/environment.cpp:1054-1138) ---------------------------
-__device__ void bb_sigmoid_fwd(Ctx& c, const SysDesc& S, const OpRec& op) {
+__device__ __forceinline__ void bb_sigmoid_fwd(Ctx& c, SysC& S, OpC& op) {
     int nt = op.ia[0];
     auto W = CFA(op, 1);
     int n = op.ia[2];
@@ -791,12 +744,11 @@ __device__ void bb_sigmoid_fwd(Ctx& c, const SysDesc& S, const OpRec& op) {
 }
 
 // ---- backbone_pairs (src/backbone_steric.cpp:38-146) --------------------------------
-__device__ void backbone_fwd(Ctx& c, const SysDesc& S, const OpRec& op, const PairGraph& G) {
-    if (!pg_refresh(c, G, op)) { graph_overflow(c, S); return; }
-    auto val = gmem(c.A + G.val);
-    auto act = gmem(c.I + G.act);
-    auto es = gmem(c.A + G.esens);
-    const int E = c.I[G.state + 3];
+__device__ __forceinline__ void backbone_fwd(Ctx& c, SysC& S, OpC& op, GraphC& G) {
+    auto val = c.A + G.val;
+    auto act = c.I + G.act;
+    auto es = c.A + G.esens;
+    const int E = uni(c.I[G.state + 3]);
     float pot = 0.f;
     for (int s = c.gtid; s < E; s += c.gsize) {
         es[s] = 1.f;
@@ -804,71 +756,74 @@ __device__ void backbone_fwd(Ctx& c, const SysDesc& S, const OpRec& op, const Pa
     }
     pot = team_sum(c, pot);
     put_pot(c, S, op, pot);
-    pg_gather(c, G);
 }
 
-// ---- rotamer (src/rotamer.cpp:840-850) ----------------------------------------------
-// Rotamer node, before the solve: cache check and rebuild, edge energies,
-// BP fill.  Returns false on capacity overflow (error word set, team synced).
-// The rotamer's pair list (refreshed when the beads moved past half the
-// buffer, with the residue-pair candidates) and its edge energies.  Reads only
-// the bead placements; false on a capacity overflow.
-__device__ bool rotamer_graph(Ctx& c, const SysDesc& S, const OpRec& op, const PairGraph& G, const RotamerDev& R) {
+// ---- phases -----------------------------------------------------------------------
+// The outlined functions of the kernel.  Each reads the context from LDS, runs
+// one phase on the current team and gives back the barrier state.
+#define PHASE static __device__ __attribute__((noinline)) PhaseRet
+
+// Bring the cache lines of a record into the scalar cache together: read field
+// by field as the code comes to them, each line costs a trip of its own.
+template <class T>
+__device__ __forceinline__ void touch(const T& r) {
+    cp<int> w = (cp<int>)&r;
+    constexpr int n = (int)sizeof(T) / 4;
+    int x = 0;
+#pragma unroll
+    for (int k = 0; k < n; k += 16) x |= w[k];
+    x |= w[n - 1];
+    asm volatile("" ::"s"(x));
+}
+
+// Pair list of a graph op for this evaluation: pack, and rebuild when an
+// element moved past half the buffer (with the residue-pair candidates of a
+// rotamer graph).  0, with the team's error word set, when a list outgrew its
+// capacity: the evaluation is void, the remaining ops are skipped and the host
+// grows the capacities and repeats the run.  Only a rebuild can fail, so
+// nothing else reads the error word.
+PHASE ph_lists(lp<int> mem, int at) {
+    Ctx c = ctx_load(mem);
+    OpC& op = cmem(c.S->ops)[uni(at)];
+    GraphC& G = cmem(c.S->graphs)[op.graph];
+    touch(G);
+    const bool rot = op.kind == OP_ROTAMER;
     unsigned long long t0 = ptick(c);
-    bool rebuild = pg_pack_and_check(c, G);
-    if (rebuild) {
-        pg_rebuild(c, G);
-        unsigned long long t1 = ptick(c);
-        if (c.I[G.state + 0]) rot_rebuild(c, G, R);
-        pacc(c, PROF_ROT_REBUILD, t1);
+    bool ok = true;
+    if (pg_pack_and_check(c, G)) {
+        ok = pg_rebuild(c, G);
+        if (ok && rot) {
+            unsigned long long t1 = ptick(c);
+            ok = rot_rebuild(c, G, cmem(c.S->rots)[op.rot]);
+            pacc(c, PROF_ROT_REBUILD, t1);
+        }
     }
-    pacc(c, PROF_REBUILD, t0);
-    if (!c.I[G.state + 0]) { graph_overflow(c, S); return false; }
-    t0 = ptick(c);
-    pg_edges(c, G, op);
+    pacc(c, rot ? PROF_REBUILD : PROF_PG_REBUILD, t0);
+    if (!ok) {
+        if (c.gtid == 0) c.I[c.err] = 1;
+        team_sync(c);
+    }
+    return phase_ret(c, ok);
+}
+
+// Refine the cached slots and evaluate the edges of a graph op.
+PHASE ph_edges(lp<int> mem, int at) {
+    Ctx c = ctx_load(mem);
+    OpC& op = cmem(c.S->ops)[uni(at)];
+    unsigned long long t0 = ptick(c);
+    pg_edges(c, cmem(c.S->graphs)[op.graph], op);
     pacc(c, PROF_PG_EDGES, t0);
-    return true;
+    return phase_ret(c, 1);
 }
 
-__device__ bool rotamer_pre(Ctx& c, const SysDesc& S, const OpRec& op, const PairGraph& G, const RotamerDev& R) {
-    if (!c.rot_graph_done && !rotamer_graph(c, S, op, G, R)) return false;
-    unsigned long long t0 = ptick(c);
-    rot_fill(c, G, R);
-    pacc(c, PROF_ROT_FILL, t0);
-    return true;
-}
-
-// Rotamer node, after the solve (it: iteration count, on gtid 0): statistics,
-// edge and 1-body sensitivities, their gather, free energy.  Ends with a team
-// barrier.
-__device__ void rotamer_post(Ctx& c, const SysDesc& S, const OpRec& op, const PairGraph& G, const RotamerDev& R,
-                             int mode, int it) {
-    if (c.gtid == 0) {
-        auto st = gmem(c.I + R.stats);
-        st[0] = it;
-        if (it >= R.max_iter - R.chunk - 1) st[1] += 1;
-        st[2] += it;
-        st[3] += 1;
-        st[BP_HIST + min(it, BP_HIST_BINS - 1)] += 1;
-    }
-    rot_sens(c, G, R);
-    pg_gather(c, G);
-    float fe = mode ? rot_free_energy(c, G, R) : 0.f;
-    put_pot(c, S, op, fe);
-}
-
-__device__ void rotamer_fwd(Ctx& c, const SysDesc& S, const OpRec& op, const PairGraph& G,
-                            const RotamerDev& R, int mode) {
-    if (!rotamer_pre(c, S, op, G, R)) return;
-    unsigned long long t0 = ptick(c);
-    int it = rot_solve(c, R, c.bp_layout);
-    pacc(c, PROF_BP, t0);
-    rotamer_post(c, S, op, G, R, mode, it);
-}
-
-// ---- program interpreter ----------------------------------------------------------
-__device__ void run_value(Ctx& c, const SysDesc& S, const OpRec& op, int mode) {
-    const PairGraph* G = op.graph >= 0 ? S.graphs + op.graph : nullptr;
+// The body of a value op other than the rotamer (whose graph, if it has one,
+// is refreshed).
+PHASE ph_value(lp<int> mem, int at) {
+    Ctx c = ctx_load(mem);
+    SysC& S = *c.S;
+    OpC& op = cmem(S.ops)[uni(at)];
+    touch(op);
+    GraphC& G = cmem(S.graphs)[op.graph >= 0 ? op.graph : 0];
     switch (op.kind) {
     case OP_DIST3D: dist3d_fwd(c, op); break;
     case OP_ANGLE: angle_fwd(c, op); break;
@@ -880,311 +835,345 @@ __device__ void run_value(Ctx& c, const SysDesc& S, const OpRec& op, int mode) {
     case OP_AFFINE: affine_fwd(c, op); break;
     case OP_PLACEMENT: placement_fwd(c, op); break;
     case OP_INFER_HO: infer_fwd(c, op); break;
-    case OP_PROTEIN_HBOND: protein_hbond_fwd(c, S, op, *G); break;
-    case OP_HBOND_COVERAGE: hbond_coverage_fwd(c, S, op, *G); break;
+    case OP_PROTEIN_HBOND: protein_hbond_fwd(c, op, G); break;
+    case OP_HBOND_COVERAGE:
+    case OP_HB_ENV_COVERAGE: pg_row_sums(c, G, op.kind == OP_HBOND_COVERAGE, OUT(op), 1); break;
     case OP_HBOND_ENERGY: hbond_energy_fwd(c, S, op); break;
-    case OP_ROTAMER: rotamer_fwd(c, S, op, *G, S.rots[op.rot], mode); return;  // ends with a team barrier
     case OP_WEIGHTED_POS: weighted_pos_fwd(c, op); break;
-    case OP_ENV_COVERAGE: env_coverage_fwd(c, S, op, *G); break;
-    case OP_HB_ENV_COVERAGE: hb_env_fwd(c, S, op, *G); break;
+    case OP_ENV_COVERAGE: env_coverage_fwd(c, op, G); break;
     case OP_SIGMOID_COUPLING: sigmoid_coupling_fwd(c, S, op); break;
     case OP_BB_SIGMOID_COUPLING: bb_sigmoid_fwd(c, S, op); break;
-    case OP_BACKBONE_PAIRS: backbone_fwd(c, S, op, *G); break;
+    case OP_BACKBONE_PAIRS: backbone_fwd(c, S, op, G); break;
     default: break;
     }
-    team_sync(c);
+    if (op.kind == OP_SPRING || op.kind == OP_RAMA_MAP_POT) plan_gather(c, op.plans[0]);
+    if (op.kind != OP_BACKBONE_PAIRS) team_sync(c);
+    return phase_ret(c, 0);
 }
 
-__device__ void run_deriv(Ctx& c, const SysDesc& S, const OpRec& op) {
-    const PairGraph* G = op.graph >= 0 ? S.graphs + op.graph : nullptr;
+// A deriv op: the contributions of each element and their sums in plan order;
+// for a graph op, the sensitivity of each edge.  Ends with a team barrier.
+PHASE ph_deriv(lp<int> mem, int at) {
+    Ctx c = ctx_load(mem);
+    SysC& S = *c.S;
+    OpC& op = cmem(S.ops)[uni(at)];
+    touch(op);
+    GraphC& G = cmem(S.graphs)[op.graph >= 0 ? op.graph : 0];
     switch (op.kind) {
     case OP_DIST3D: dist3d_bwd(c, op); break;
     case OP_ANGLE: angle_bwd(c, op); break;
     case OP_DIHEDRAL: dihedral_bwd(c, op); break;
-    case OP_RAMA_COORD: passthrough_bwd(c, op); break;
-    case OP_CAT_POS: passthrough_bwd(c, op); break;
     case OP_AFFINE: affine_bwd(c, op); break;
     case OP_PLACEMENT: placement_bwd(c, op); break;
     case OP_INFER_HO: infer_bwd(c, op); break;
-    // these end with their own team barrier (the sensitivity gather)
-    case OP_PROTEIN_HBOND: protein_hbond_bwd(c, op, *G); return;
-    case OP_HBOND_COVERAGE: hbond_coverage_bwd(c, op, *G); return;
     case OP_WEIGHTED_POS: weighted_pos_bwd(c, op); break;
-    case OP_ENV_COVERAGE: env_coverage_bwd(c, op, *G); return;
-    case OP_HB_ENV_COVERAGE: hb_env_bwd(c, op, *G); return;
-    default: break;  // potential nodes push in their value pass
+    case OP_PROTEIN_HBOND: protein_hbond_bwd(c, op, G); break;
+    case OP_HBOND_COVERAGE: hbond_coverage_bwd(c, op, G); break;
+    case OP_ENV_COVERAGE: env_coverage_bwd(c, op, G); break;
+    case OP_HB_ENV_COVERAGE: hb_env_bwd(c, op, G); break;
+    default: break;  // rama_coord, cat_pos: the gather reads their sensitivities as they are
     }
     team_sync(c);
-}
-
-// A team context narrowed to rank 0's workgroup alone (team barriers become
-// workgroup barriers, team reductions block reductions).
-__device__ __forceinline__ Ctx solo_ctx(const Ctx& c) {
-    Ctx l = c;
-    l.G = 1;
-    l.rank = 0;
-    l.gtid = c.tid;
-    l.gsize = NT;
-    return l;
-}
-
-// End of the run of solo ops starting at k (ops [k, end) are all solo).
-__device__ __forceinline__ int solo_run_end(const SysDesc& S, int k, int end) {
-    while (k < end && S.ops[k].solo) ++k;
-    return k;
-}
-
-// The deriv ops marked early, in deriv order, on the (sub-)team s that ran the
-// rotamer's overlap ops: their sensitivities are complete once those ops are
-// done, and nothing the solve or the rotamer's sensitivity push touches is
-// read or written by them.  Runs of solo ops go to s's rank 0.
-__device__ void run_early_derivs(Ctx& s, const SysDesc& S) {
-    const int nd = S.n_germ + S.n_deriv;
-    for (int k = S.n_germ; k < nd;) {
-        const OpRec& op = S.ops[k];
-        if (!op.early) { ++k; continue; }
-        s.cur_op = k;
-        if (s.G > 1 && op.solo) {
-            int k2 = k;
-            while (k2 < nd && (!S.ops[k2].early || S.ops[k2].solo)) ++k2;
-            if (s.rank == 0) {
-                Ctx l = solo_ctx(s);
-                for (int q = k; q < k2; ++q) {
-                    if (!S.ops[q].early) continue;
-                    unsigned long long t0 = ptick(l);
-                    run_deriv(l, S, S.ops[q]);
-                    prof_op(l, q, t0);
-                }
-            }
-            team_sync(s);
-            k = k2;
-            continue;
+    if (op.graph < 0) {
+        int p0 = op.plans[0], p1 = op.plans[1];
+        if (op.kind == OP_PLACEMENT) {
+            if (op.ia[3]) p0 = -1;
+            else p1 = -1;
         }
-        unsigned long long t0 = ptick(s);
-        run_deriv(s, S, op);
-        prof_op(s, k, t0);
-        ++k;
-    }
-}
-
-// The ops of one lane of a two-lane section [k0, k1) on half-team s: ops of
-// the other lane are skipped (they run on the other half, and the host made
-// the two lanes independent: neither reads what the other writes).  A lane's
-// solo ops up to its next team op run on the half's rank 0.  Returns false
-// when an op set the half's error word.
-__device__ bool run_lane(Ctx& s, const SysDesc& S, int k0, int k1, unsigned lanes, int mode) {
-    const OpRec& first = S.ops[k0];
-    auto mine = [&](const OpRec& o) { return ((lanes >> o.lane) & 1u) != 0u; };
-    if (first.rot_graph_op >= 0 && ((lanes >> first.rot_graph_lane) & 1u)) {
-        const OpRec& ro = S.ops[first.rot_graph_op];
-        s.cur_op = first.rot_graph_op;
-        if (!rotamer_graph(s, S, ro, S.graphs[ro.graph], S.rots[ro.rot])) return false;
-    }
-    for (int k = k0; k < k1;) {
-        const OpRec& op = S.ops[k];
-        if (!mine(op)) { ++k; continue; }
-        s.cur_op = k;
-        if (s.G > 1 && op.solo) {
-            int k2 = k;
-            while (k2 < k1 && (!mine(S.ops[k2]) || S.ops[k2].solo)) ++k2;
-            if (s.rank == 0) {
-                Ctx l = solo_ctx(s);
-                for (int q = k; q < k2; ++q) {
-                    if (!mine(S.ops[q])) continue;
-                    unsigned long long t0 = ptick(l);
-                    run_value(l, S, S.ops[q], mode);
-                    prof_op(l, q, t0);
-                    if (l.I[l.err]) break;
-                }
-            }
-            team_sync(s);
-            if (s.I[s.err]) return false;
-            k = k2;
-            continue;
-        }
-        unsigned long long t0 = ptick(s);
-        run_value(s, S, op, mode);
-        prof_op(s, k, t0);
-        if (s.I[s.err]) return false;
-        ++k;
-    }
-    return true;
-}
-
-// Value ops [k0, k1) in germ order on the team c.  Ops marked solo
-// (elementwise work over at most a few thousand elements) run on rank 0 of
-// the team alone: a run of them goes back to back with workgroup barriers and
-// ends with one team barrier, since a team barrier costs more than such an
-// op.  With SPLIT, a rotamer op with an overlap range runs its solve on rank 0
-// while the other ranks evaluate the following independent ops.  Returns
-// false when an op set the error word.
-template <bool SPLIT>
-__device__ bool run_germ_range(Ctx& c, const SysDesc& S, int k0, int k1, int mode) {
-    for (int k = k0; k < k1;) {
-        const OpRec& op = S.ops[k];
-        c.cur_op = k;
-        if (SPLIT && op.lane_end > k && op.lane_end <= k1 && c.G >= 4) {
-            // section: the team splits into nq sub-teams (four quarters when
-            // the program has four lanes, the team eight or more workgroups
-            // and the launch asks for them, else two halves), each with its own barrier
-            // counter, reduction scratch and error word; sub-team j runs
-            // lane j, or lanes j and j+2 (four lanes on two halves) in program
-            // order.  The join barrier makes every error word readable.
-            const int nl = S.n_lanes;
-            const int nq = (nl == 4 && c.G >= 8 && c.args->lane_split == 4) ? 4 : 2;
-            int j = 0;
-            while (j + 1 < nq && c.rank >= (j + 1) * c.G / nq) ++j;
-            const int r0 = j * c.G / nq, r1 = (j + 1) * c.G / nq;
-            const unsigned mask = (nq == nl) ? (1u << j) : ((1u << j) | (1u << (j + 2)));
-            if (nq == 2) {
-                Ctx s = sub_team(c, r0, r1 - r0, j ? c.bar_hi : c.bar_lo, j ? c.tred_hi : c.tred_lo,
-                                 j ? c.tpar_hi : c.tpar_lo);
-                if (s.rank == 0) s.prof = S.prof;  // profiling: each sub-team's ops are timed by its rank 0
-                s.err = S.error + 1 + j;
-                run_lane(s, S, k, op.lane_end, mask, mode);
-                (j ? c.tpar_hi : c.tpar_lo) = s.tpar;
-            } else {
-                Ctx s = sub_team(c, r0, r1 - r0, c.bar_q + j, c.tred_q + 2 * MAX_TEAM * j, c.tpar_q);
-                if (s.rank == 0) s.prof = S.prof;
-                s.err = S.error + 1 + j;
-                run_lane(s, S, k, op.lane_end, mask, mode);
-                c.tpar_q = s.tpar;
-            }
+        for (int q = 0; q < 2; ++q) {  // both plans may add into the same sensitivities
+            const int plan = q ? p1 : p0;
+            if (plan < 0) continue;
+            plan_gather(c, plan);
             team_sync(c);
-            int lane_err = 0;
-            for (int q = 1; q <= nq; ++q) lane_err |= c.I[S.error + q];
-            if (lane_err) {
-                if (c.gtid == 0) c.I[c.err] = 1;
-                team_sync(c);
-                return false;
-            }
-            if (op.rot_graph_op >= 0) c.rot_graph_done = 1;
-            k = op.lane_end;
-            continue;
         }
-        if (c.G > 1 && op.solo) {
-            const int k2 = solo_run_end(S, k, k1);
-            if (c.rank == 0) {
-                Ctx l = solo_ctx(c);
-                for (int q = k; q < k2; ++q) {
-                    unsigned long long t0 = ptick(l);
-                    run_value(l, S, S.ops[q], mode);
-                    prof_op(l, q, t0);
-                    if (l.I[l.err]) break;
-                }
-            }
-            team_sync(c);
-            if (c.I[c.err]) return false;
-            k = k2;
-            continue;
-        }
-        if (SPLIT && op.kind == OP_ROTAMER && op.overlap_end > k && op.overlap_end <= k1) {
-            // A rotamer op with an overlap range: the ops of the range and the
-            // early deriv ops run beside the solve where the team can split,
-            // else between the solve and the rotamer's sensitivity push.
-            // Either way they come after the solve's start and before the push,
-            // so every sum sees its terms in the same order: same bits on
-            // every team size and layout.
-            unsigned long long t0 = ptick(c);
-            const PairGraph& G = S.graphs[op.graph];
-            const RotamerDev& R = S.rots[op.rot];
-            if (!rotamer_pre(c, S, op, G, R)) return false;
-            int it = 0;
-            const bool one_wg = bp_on_one_wg(c, R, c.I[R.stats + 4], c.bp_layout);
-            unsigned long long t1 = ptick(c);
-            if (c.G > 1 && !one_wg && c.bp_layout != 1 && c.G >= 4) {
-                // the state does not fit one workgroup's LDS: the first half
-                // solves while the second half runs the range
-                const int gb = c.G / 2;
-                if (c.rank < gb) {
-                    Ctx b = sub_team(c, 0, gb, c.bar_lo, c.tred_lo, c.tpar_lo);
-                    it = rot_solve_team(b, R);
-                    c.tpar_lo = b.tpar;
-                } else {
-                    Ctx o = sub_team(c, gb, c.G - gb, c.bar_hi, c.tred_hi, c.tpar_hi);
-                    if (o.rank == 0) o.prof = S.prof;  // profiling: the ops of this half are timed by its rank 0
-                    const unsigned long long t2 = S.prof ? wall_clock64() : 0ull;
-                    if (run_germ_range<false>(o, S, k + 1, op.overlap_end, mode)) run_early_derivs(o, S);
-                    c.tpar_hi = o.tpar;
-                    // profiling: the half's own time, by its first thread (rank 0 keeps the others)
-                    if (S.prof && o.gtid == 0)
-                        __hip_atomic_fetch_add(S.prof + c.pbase + PROF_BESIDE, wall_clock64() - t2, __ATOMIC_RELAXED,
-                                               __HIP_MEMORY_SCOPE_AGENT);
-                }
-                team_sync(c);  // join; an error in the range is read after the rotamer
-            } else if (c.G > 1 && one_wg) {
-                // rank 0 solves in its LDS while ranks 1..G-1 run the range
-                if (c.rank == 0) {
-                    it = rot_solve_wg(c, R);
-                } else {
-                    Ctx s = sub_team(c);
-                    if (s.rank == 0) s.prof = S.prof;
-                    const unsigned long long t2 = S.prof ? wall_clock64() : 0ull;
-                    if (run_germ_range<false>(s, S, k + 1, op.overlap_end, mode)) run_early_derivs(s, S);
-                    c.tpar2 = s.tpar;
-                    if (S.prof && s.gtid == 0)
-                        __hip_atomic_fetch_add(S.prof + c.pbase + PROF_BESIDE, wall_clock64() - t2, __ATOMIC_RELAXED,
-                                               __HIP_MEMORY_SCOPE_AGENT);
-                }
-                team_sync(c);  // join; an error in the range is read after the rotamer
-            } else {
-                // one workgroup, or the whole team solves: the range follows
-                it = rot_solve(c, R, c.bp_layout);
-                if (!run_germ_range<false>(c, S, k + 1, op.overlap_end, mode)) return false;
-                run_early_derivs(c, S);
-            }
-            pacc(c, PROF_BP, t1);
-            c.early_done = 1;
-            rotamer_post(c, S, op, G, R, mode, it);
-            prof_op(c, k, t0);
-            if (c.I[c.err]) return false;
-            k = op.overlap_end;
-            continue;
-        }
-        unsigned long long t0 = ptick(c);
-        run_value(c, S, op, mode);
-        prof_op(c, k, t0);
-        if (c.I[c.err]) return false;  // uniform: read after the op's final barrier
-        ++k;
     }
-    return true;
+    return phase_ret(c, 0);
 }
 
-// One evaluation: value ops in germ order, then sensitivity pushes.
-__device__ void compute(Ctx& c, const SysDesc& S, int mode) {
-    c.cur_op = S.n_germ + S.n_deriv;  // outside the ops
-    c.early_done = 0;
-    c.rot_graph_done = 0;
-    const int* zr = c.I + S.sens_zero;
+// The sums of a graph op's edges.  Ends with a team barrier.
+PHASE ph_gather(lp<int> mem, int at, int value) {
+    Ctx c = ctx_load(mem);
+    OpC& op = cmem(c.S->ops)[uni(at)];
+    GraphC& G = cmem(c.S->graphs)[op.graph];
+    touch(op);
+    touch(G);
+    pg_gather(c, G);
+    if (!uni(value) && op.kind == OP_PROTEIN_HBOND) protein_hbond_pass(c, op, G);
+    return phase_ret(c, 0);
+}
+
+// ---- rotamer (src/rotamer.cpp:840-850) ----------------------------------------------
+// Before the solve: node probabilities, BP edges and their matrices.
+PHASE ph_fill(lp<int> mem, int at) {
+    Ctx c = ctx_load(mem);
+    OpC& op = cmem(c.S->ops)[uni(at)];
+    unsigned long long t0 = ptick(c);
+    rot_fill(c, cmem(c.S->graphs)[op.graph], cmem(c.S->rots)[op.rot]);
+    pacc(c, PROF_ROT_FILL, t0);
+    return phase_ret(c, 0);
+}
+
+// The solve, on this workgroup or on the team; gives the iterations.
+PHASE ph_solve_wg(lp<int> mem, int rot) {
+    Ctx c = ctx_load(mem);
+    const int it = rot_solve_wg(c, cmem(c.S->rots)[uni(rot)]);
+    return phase_ret(c, it);
+}
+PHASE ph_solve_team(lp<int> mem, int rot) {
+    Ctx c = ctx_load(mem);
+    const int it = rot_solve_team(c, cmem(c.S->rots)[uni(rot)]);
+    return phase_ret(c, it);
+}
+
+// After the solve (it: iteration count, on gtid 0): statistics, edge and
+// 1-body sensitivities; ends with a team barrier.
+PHASE ph_sens(lp<int> mem, int at, int it) {
+    Ctx c = ctx_load(mem);
+    OpC& op = cmem(c.S->ops)[uni(at)];
+    RotC& R = cmem(c.S->rots)[op.rot];
+    if (c.gtid == 0) {
+        auto st = c.I + R.stats;
+        st[0] = it;
+        if (it >= R.max_iter - R.chunk - 1) st[1] += 1;
+        st[2] += it;
+        st[3] += 1;
+        st[BP_HIST + min(it, BP_HIST_BINS - 1)] += 1;
+    }
+    rot_sens(c, cmem(c.S->graphs)[op.graph], R);
+    return phase_ret(c, 0);
+}
+PHASE ph_free_energy(lp<int> mem, int at) {
+    Ctx c = ctx_load(mem);
+    OpC& op = cmem(c.S->ops)[uni(at)];
+    const float fe = rot_free_energy(c, cmem(c.S->graphs)[op.graph], cmem(c.S->rots)[op.rot]);
+    put_pot(c, *c.S, op, fe);
+    return phase_ret(c, 0);
+}
+
+
+// ---- program interpreter ----------------------------------------------------------
+// Run a phase function on the team c.
+#define RUN(call) phase_done(c, (ctx_store(mem, c), call))
+
+// One evaluation: value ops in germ order, then sensitivity pushes in deriv
+// order.  False on a capacity overflow (uniform over the team).
+//
+// One loop runs every op, whatever part of the team it runs on:
+//  * MAIN: the value ops on the whole team.  Ops marked solo (elementwise work
+//    over at most a few thousand elements) run on rank 0 of the team alone: a
+//    run of them goes back to back with workgroup barriers and ends with one
+//    team barrier, since a team barrier costs more than such an op.
+//  * SECTION: value ops of a section, dealt to lanes the host made independent
+//    of each other.  The team splits into four quarters (when the program has
+//    four lanes, the team eight or more workgroups and the launch asks for
+//    them), else into two halves; sub-team j runs lane j, or lanes j and j+2
+//    (four lanes on two halves) in program order, each with its own barrier
+//    counter, reduction scratch and error word.  The lane that starts with the
+//    rotamer's pair-list refresh and edge evaluation (which reads only the bead
+//    placements) runs that first.
+//  * BESIDE, BESIDE_DERIV: a rotamer op's overlap range, then the early deriv
+//    ops, beside the rotamer solve where the team can split (the half that does
+//    not solve, or ranks 1..G-1 beside a solve in rank 0's LDS), else between
+//    the solve and the rotamer's sensitivity push.  Either way they come after
+//    the solve's start and before the push, so every sum sees its terms in the
+//    same order: same bits on every team size and layout.
+//  * DERIV: the deriv ops (those not already run early) on the whole team.
+enum Where : int { MAIN = 0, SECTION, BESIDE, BESIDE_DERIV, DERIV };
+
+__device__ __forceinline__ bool compute(Ctx& c, SubNext& next, lp<int> mem, gp<int> words, int mode) {
+    SysC& S = *c.S;
+    cp<OpRec> ops = cmem(S.ops);
+    const int ng = S.n_germ, nd = S.n_germ + S.n_deriv;
+    c.cur_op = nd;  // outside the ops
     for (int r = 0; r < S.sens_zero_cnt; ++r) {
-        float* p = c.A + zr[2 * r];
-        int n = zr[2 * r + 1];
+        cp<int> zr = (cp<int>)(c.I + S.sens_zero + 2 * r);  // written once, by the host
+        gp<float> p = c.A + zr[0];
+        const int n = zr[1];
         for (int i = c.gtid; i < n; i += c.gsize) p[i] = 0.f;
     }
     team_sync(c);
-    if (!run_germ_range<true>(c, S, 0, S.n_germ, mode)) return;
-    const int nd = S.n_germ + S.n_deriv;
-    for (int k = S.n_germ; k < nd;) {
-        c.cur_op = k;
-        if (c.early_done && S.ops[k].early) { ++k; continue; }  // ran beside the rotamer solve
-        if (c.G > 1 && S.ops[k].solo) {
-            const int k2 = solo_run_end(S, k, nd);
-            if (c.rank == 0) {
-                Ctx l = solo_ctx(c);
-                for (int q = k; q < k2; ++q) {
-                    if (c.early_done && S.ops[q].early) continue;
-                    unsigned long long t0 = ptick(l);
-                    run_deriv(l, S, S.ops[q]);
-                    prof_op(l, q, t0);
-                }
-            }
+
+    Team root = c;              // the whole team, while c is narrowed to a part of it
+    int sub = -1;               // kind of the part (SubTeam), -1: the whole team
+    int where = MAIN, k = 0, end = ng;
+    unsigned lanes = 0;         // SECTION: lanes this part runs
+    int section = 0;            // SECTION: its first op
+    int rot_graph = -1;         // SECTION: rotamer op whose graph to refresh first
+    int rot_ready = -1;         // rotamer op whose graph a section has refreshed
+    bool early_done = false;
+    int rot_k = -1;             // rotamer op being solved
+    bool post = false;          // its sensitivities are next
+    int it = 0;                 // its iterations
+    int solo_of = 0;            // team size outside the current run of solo ops (0: not in one)
+    unsigned long long t_rot = 0, t_bp = 0, t_beside = 0;
+    for (;;) {
+        // the interpreter's state is uniform; said once per op, it stays in scalar registers
+        where = uni(where); k = uni(k); end = uni(end); sub = uni(sub); lanes = (unsigned)uni((int)lanes);
+        rot_graph = uni(rot_graph); rot_k = uni(rot_k); solo_of = uni(solo_of); section = uni(section);
+        rot_ready = uni(rot_ready); post = uni(post) != 0; early_done = uni(early_done) != 0;
+        // the next op of the range that is this team's
+        if (rot_graph < 0 && !post) {
+            if (where == SECTION)
+                while (k < end && !((lanes >> ops[k].lane) & 1u)) ++k;
+            else if (where == BESIDE_DERIV)
+                while (k < end && !ops[k].early) ++k;
+            else if (where == DERIV && early_done)
+                while (k < end && ops[k].early) ++k;
+        }
+        const int at = uni(rot_graph >= 0 ? rot_graph : post ? rot_k : k);
+        const bool done = rot_graph < 0 && !post && k >= end;
+        OpC& op = ops[done ? 0 : at];
+        const bool starts_section = !done && where == MAIN && !post && op.lane_end > k && (solo_of ? solo_of : c.G) >= 4;
+        const bool solo = !done && !post && rot_graph < 0 && !starts_section && op.solo && (solo_of || c.G > 1);
+        if (solo_of && !solo) {  // a run of solo ops ends
+            c.G = solo_of;
+            c.gsize = c.G * NT;
+            solo_of = 0;
             team_sync(c);
-            k = k2;
+        }
+        if (done) {
+            if (where == MAIN) {
+                where = DERIV;
+                k = ng;
+                end = nd;
+            } else if (where == SECTION) {
+                leave_sub(c, next, root, sub);
+                sub = -1;
+                team_sync(c);
+                OpC& first = ops[section];
+                if (first.lane_graphs) {  // the join made every part's error word readable
+                    int e = 0;
+                    for (int q = 1; q <= MAX_LANES; ++q) e |= c.I[S.error + q];
+                    if (uni(e)) {
+                        if (c.gtid == 0) c.I[c.err] = 1;
+                        team_sync(c);
+                        return false;
+                    }
+                }
+                if (first.rot_graph_op >= 0) rot_ready = first.rot_graph_op;
+                where = MAIN;
+                k = first.lane_end;
+                end = ng;
+            } else if (where == BESIDE) {
+                where = BESIDE_DERIV;
+                k = ng;
+                end = nd;
+            } else if (where == BESIDE_DERIV) {
+                if (sub >= 0) {
+                    // profiling: this part's own time, by its first thread (rank 0 keeps the others)
+                    if (S.prof && c.gtid == 0)
+                        __hip_atomic_fetch_add(S.prof + c.pbase + PROF_BESIDE, wall_clock64() - t_beside,
+                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    leave_sub(c, next, root, sub);
+                    sub = -1;
+                    team_sync(c);
+                }
+                pacc(c, PROF_BP, t_bp);
+                post = true;
+                where = MAIN;
+                end = ng;
+            } else {
+                return true;
+            }
             continue;
         }
+        if (starts_section) {
+            root = c;
+            sub = (S.n_lanes == 4 && c.G >= 8 && c.args->lane_split == 4) ? SUB_QUARTER : SUB_HALF;
+            const SubPart p = sub_part(sub, c.rank, c.G);
+            const int j = sub == SUB_QUARTER ? (p.word - BAR_Q) / 2 : (p.first ? 1 : 0);
+            lanes = (sub == SUB_QUARTER || S.n_lanes == 2) ? (1u << j) : ((1u << j) | (1u << (j + 2)));
+            enter_sub(c, next, root, sub, words, S.prof);
+            c.err = S.error + 1 + j;
+            section = k;
+            where = SECTION;
+            end = op.lane_end;
+            if (op.rot_graph_op >= 0 && ((lanes >> op.rot_graph_lane) & 1u)) rot_graph = op.rot_graph_op;
+            continue;
+        }
+        if (solo) {
+            if (!solo_of) {
+                solo_of = c.G;
+                if (c.rank == 0) { c.G = 1; c.gsize = NT; }
+            }
+            if (c.rank != 0) { ++k; continue; }
+        }
+        c.cur_op = at;
+        const bool value = where <= BESIDE;
+        const bool rot = op.kind == OP_ROTAMER;
         unsigned long long t0 = ptick(c);
-        run_deriv(c, S, S.ops[k]);
-        prof_op(c, k, t0);
+        if (value && op.graph >= 0 && !post && at != rot_ready) {
+            if (!RUN(ph_lists(mem, at))) {
+                if (where == MAIN) return false;
+                rot_graph = -1;  // to the join
+                if (where == BESIDE) where = BESIDE_DERIV;
+                k = end = 0;
+                continue;
+            }
+            RUN(ph_edges(mem, at));
+            if (rot_graph >= 0) { rot_graph = -1; continue; }
+        }
+        if (rot && !post) {
+            RotC& R = cmem(S.rots)[op.rot];
+            t_rot = t0;
+            RUN(ph_fill(mem, at));
+            t_bp = ptick(c);
+            rot_k = k;
+            const bool ranged = where == MAIN && op.overlap_end > k;
+            const bool wg = bp_on_one_wg(c, R, uni(c.I[R.stats + 4]), c.bp_layout);
+            // the part that solves: the first half when the state does not fit
+            // one workgroup's LDS, or rank 0 alone, beside the range; else the
+            // whole team (or its rank 0), and the range follows
+            bool solve = !wg || c.rank == 0;
+            if (ranged && c.G > 1 && (wg || (c.bp_layout != 1 && c.G >= 4))) {
+                root = c;
+                sub = wg ? SUB_REST : SUB_HALF;
+                solve = wg ? c.rank == 0 : c.rank < c.G / 2;
+                if (!wg || c.rank != 0) enter_sub(c, next, root, sub, words, S.prof);
+                t_beside = S.prof ? wall_clock64() : 0ull;
+            }
+            if (solve) it = wg ? RUN(ph_solve_wg(mem, op.rot)) : RUN(ph_solve_team(mem, op.rot));
+            if (sub >= 0 && solve) {  // join; an error in the range is read after the rotamer
+                if (!wg) leave_sub(c, next, root, sub);
+                sub = -1;
+                team_sync(c);
+                pacc(c, PROF_BP, t_bp);
+                post = true;
+                early_done = true;
+                continue;
+            }
+            if (sub < 0 && wg && c.G > 1) team_sync(c);
+            if (ranged) {
+                early_done = true;
+                where = BESIDE;
+                ++k;
+                end = op.overlap_end;
+            } else {
+                pacc(c, PROF_BP, t_bp);
+                post = true;
+            }
+            continue;
+        }
+        // the op's body, then the sums it leaves
+        if (post) {
+            RUN(ph_sens(mem, at, it));
+            RUN(ph_gather(mem, at, 1));
+            if (mode) RUN(ph_free_energy(mem, at));
+            else put_pot(c, S, op, 0.f);
+            prof_op(c, at, t_rot);
+            if (op.lane_graphs && uni(c.I[c.err])) return false;
+            post = false;
+            k = op.overlap_end > at ? op.overlap_end : at + 1;
+            continue;
+        }
+        if (value) {
+            RUN(ph_value(mem, at));
+            if (op.kind == OP_BACKBONE_PAIRS) RUN(ph_gather(mem, at, 1));
+        } else {
+            RUN(ph_deriv(mem, at));
+            if (op.graph >= 0) RUN(ph_gather(mem, at, 0));
+        }
+        prof_op(c, at, t0);
         ++k;
     }
 }
@@ -1192,7 +1181,7 @@ __device__ void compute(Ctx& c, const SysDesc& S, int mode) {
 // Threefry-4x32-20 (Salmon et al., SC'11), key (seed, stream, 0, 0) and counter
 // (step lo, step hi, atom, 0) as RandomGenerator (src/random.h:19-67).
 __device__ __forceinline__ uint32_t rotl32(uint32_t v, int r) { return (v << r) | (v >> (32 - r)); }
-__device__ void threefry4x32_20(const uint32_t ctr[4], const uint32_t key[4], uint32_t out[4]) {
+__device__ __forceinline__ void threefry4x32_20(const uint32_t ctr[4], const uint32_t key[4], uint32_t out[4]) {
     const int R0[8] = {10, 11, 13, 23, 6, 17, 25, 18};
     const int R1[8] = {26, 21, 27, 5, 20, 11, 10, 20};
     uint32_t ks[5] = {key[0], key[1], key[2], key[3], 0x1BD11BDAu ^ key[0] ^ key[1] ^ key[2] ^ key[3]};
@@ -1215,7 +1204,7 @@ __device__ void threefry4x32_20(const uint32_t ctr[4], const uint32_t key[4], ui
 }
 
 // normal3 of RandomGenerator: Box-Muller on u01/uneg11 (src/boxmuller.hpp, src/uniform.hpp).
-__device__ void normal3(uint32_t seed, uint32_t stream, uint32_t atom, uint64_t step, float* o) {
+__device__ __forceinline__ void normal3(uint32_t seed, uint32_t stream, uint32_t atom, uint64_t step, float* o) {
     uint32_t key[4] = {seed, stream, 0u, 0u};
     uint32_t ctr[4] = {(uint32_t)(step & 0xffffffffull), (uint32_t)(step >> 32), atom, 0u};
     uint32_t b[4];
@@ -1236,7 +1225,7 @@ __device__ void normal3(uint32_t seed, uint32_t stream, uint32_t atom, uint64_t 
 // Temperature of the annealing schedule at `time` (the anneal_temp lambda of
 // src/main.cpp:603-612, in double): T0 until the start, T0*factor after the
 // end, between them the square of a linear blend of the square roots.
-__device__ double anneal_temperature(const RunArgs& a, double T0, double time) {
+__device__ __forceinline__ double anneal_temperature(UPS_CONST const RunArgs& a, double T0, double time) {
     const double T1 = T0 * a.anneal_factor;
     if (time <= a.anneal_start) return T0;
     if (time > a.anneal_end) return T1;
@@ -1246,19 +1235,23 @@ __device__ double anneal_temperature(const RunArgs& a, double T0, double time) {
     return s * s;
 }
 
-__device__ void thermostat(Ctx& c, SysDesc& S, float noise_scale) {
-    auto mom = gmem(c.A + S.mom);
+// One thermostat application: invocation `inv` of this system's stream.  No
+// barrier: the momenta are next read after the barriers of an evaluation.
+// The roundings are pinned: the momentum's product rounds before the noise is added.
+PHASE ph_thermostat(lp<int> mem, float noise_scale, uint64_t inv) {
+    Ctx c = ctx_load(mem);
+    SysC& S = *c.S;
+    auto mom = c.A + S.mom;
     for (int a = c.gtid; a < S.n_atom; a += c.gsize) {
         float n[3];
-        normal3(S.seed, 0u, (uint32_t)a, S.n_invocations, n);
-        for (int k = 0; k < 3; ++k) mom[a * 3 + k] = S.mom_scale * mom[a * 3 + k] + noise_scale * n[k];
+        normal3(S.seed, 0u, (uint32_t)a, inv, n);
+        for (int k = 0; k < 3; ++k)
+            mom[a * 3 + k] = __fmaf_rn(noise_scale, n[k], __fmul_rn(S.mom_scale, mom[a * 3 + k]));
     }
-    team_sync(c);
-    if (c.gtid == 0) S.n_invocations += 1;
-    team_sync(c);
+    return phase_ret(c, 0);
 }
 
-__device__ float total_potential(Ctx& c, const SysDesc& S) {
+__device__ __forceinline__ float total_potential(Ctx& c, SysC& S) {
     float t = 0.f;
     for (int k = 0; k < S.n_pot; ++k) t += c.A[S.pot + k];
     return t;
@@ -1268,7 +1261,7 @@ __device__ float total_potential(Ctx& c, const SysDesc& S) {
 // exchange (teams on different XCDs: device-scope fences on both sides), on a
 // monotonic arrival counter as team_sync.  Bounded: a timeout sets the flag,
 // which the host turns into an error, and no later wait blocks.
-__device__ void grid_sync(Ctx& c, const RexDev& x) {
+__device__ __forceinline__ void grid_sync(Ctx& c, UPS_CONST const RexDev& x) {
     __syncthreads();
     if (c.tid == 0) {
         __threadfence();
@@ -1289,7 +1282,7 @@ __device__ void grid_sync(Ctx& c, const RexDev& x) {
 }
 
 // One replica-exchange attempt after `done` completed rounds (see RexDev):
-// all teams of the launch.  The decisions follow attempt_swaps
+// all teams of the launch, each having evaluated its potential.  The decisions follow attempt_swaps
 // (src/main.cpp:243-316): criterion 0 keeps a swap unless the change of the
 // summed log Boltzmann weights is negative and exp(change) falls below a
 // uniform draw; criterion 1 swaps when the change lb[s2] - lb[s1] is
@@ -1297,11 +1290,14 @@ __device__ void grid_sync(Ctx& c, const RexDev& x) {
 // stream 1, counter (done, 0, k), one per test that needs it.  With one
 // shared potential the weights after a swap are those of the partner's
 // positions, -beta_s E(x_partner), evaluated once per system.
-__device__ __noinline__ void rex_attempt(Ctx& c, SysDesc& S, const RexDev& x, int sys, int n_sys, long long done) {
-    compute(c, S, 1);
+PHASE ph_exchange(lp<int> mem, int sys_, long long done) {
+    Ctx c = ctx_load(mem);
+    SysC& S = *c.S;
+    UPS_CONST const RexDev& x = c.args->rex;
+    const int n_sys = c.args->n_sys, sys = uni(sys_);
     if (c.gtid == 0) x.energy[sys] = total_potential(c, S);
     {
-        auto pos = gmem(c.A + S.pos_out);
+        auto pos = c.A + S.pos_out;
         auto st = gmem(x.stage + (size_t)sys * x.stage_stride);
         for (int i = c.gtid; i < S.n_atom * 3; i += c.gsize) st[i] = pos[i];
     }
@@ -1349,11 +1345,12 @@ __device__ __noinline__ void rex_attempt(Ctx& c, SysDesc& S, const RexDev& x, in
     grid_sync(c, x);
     const int q = x.partner[sys];
     if (q >= 0) {
-        auto pos = gmem(c.A + S.pos_out);
+        auto pos = c.A + S.pos_out;
         auto st = gmem((const float*)x.stage + (size_t)q * x.stage_stride);
         for (int i = c.gtid; i < S.n_atom * 3; i += c.gsize) pos[i] = st[i];
     }
     team_sync(c);
+    return phase_ret(c, 0);
 }
 
 // One launch evaluates or integrates every system of a batch; system s is
@@ -1361,12 +1358,15 @@ __device__ __noinline__ void rex_attempt(Ctx& c, SysDesc& S, const RexDev& x, in
 // by two kernel symbols so that the integration launches (the hot path) and
 // the single evaluations / thermostat applications show up separately in a
 // kernel trace.
-__device__ __forceinline__ void engine_body(SysDesc* systems, const RunArgs& args, float* red, int* ired,
-                                            float* lds) {
+__device__ __forceinline__ void engine_body(SysDesc* systems, lp<float> red, lp<int> ired, lp<int> mem,
+                                            lp<float> lds) {
+    // the launch's arguments where they lie (after the first kernel argument): taking the
+    // address of a by-value parameter would copy it to private memory
+    UPS_CONST const RunArgs& args = *(cp<RunArgs>)((UPS_CONST const char*)__builtin_amdgcn_kernarg_segment_ptr() + 8);
     int G = args.team;
     int sys = blockIdx.x, rank = 0;
     if (args.blockmap) {  // per-system teams, placed by the host
-        const int e = args.blockmap[blockIdx.x];
+        const int e = cmem(args.blockmap)[blockIdx.x];
         if (e < 0) return;  // padding workgroup
         sys = e >> 14;
         G = (e >> 7) & 127;
@@ -1377,9 +1377,11 @@ __device__ __forceinline__ void engine_body(SysDesc* systems, const RunArgs& arg
         rank = slot % G;
         if (sys >= args.n_sys) return;  // padding workgroup
     }
-    SysDesc& S = systems[sys];
+    sys = uni(sys); rank = uni(rank); G = uni(G);
+    SysC& S = cmem(systems)[sys];
     Ctx c;
-    c.A = S.arena; c.I = S.iarena; c.CF = S.cf; c.CI = S.ci;
+    c.S = &S;
+    c.A = gmem(S.arena); c.I = gmem(S.iarena); c.CF = gmem(S.cf); c.CI = gmem(S.ci);
     c.red = red; c.ired = ired; c.lds = lds;
     c.tid = (int)threadIdx.x;
     c.prof = rank == 0 ? S.prof : nullptr;
@@ -1388,63 +1390,80 @@ __device__ __forceinline__ void engine_body(SysDesc* systems, const RunArgs& arg
     c.err = S.error;
     c.rank = rank; c.G = G;
     c.gtid = rank * NT + c.tid; c.gsize = G * NT;
-    c.bar = reinterpret_cast<unsigned long long*>(S.iarena + S.bar);  // 16-byte aligned words
-    c.bar_flag = reinterpret_cast<unsigned*>(S.iarena + S.bar + 2);
-    c.bar_next = (G > 1 && c.tid == 0) ? bar_first(c.bar, G) : 0ull;
-    c.tred = S.arena + S.tred;
+    const gp<int> words = c.I + S.bar;
+    c.bar = (gp<unsigned long long>)words;  // 16-byte aligned words
+    c.bar_flag = (gp<unsigned>)(words + 2);
+    c.bar_next = 0;
+    SubNext next = {0, 0, 0};
+    if (G > 1) {
+        // read before this workgroup's first arrival at any of them
+        auto first = [&](int kind) {
+            const SubPart p = sub_part(kind, rank, G);
+            return bar_first((gp<unsigned long long>)(words + p.word), p.size);
+        };
+        c.bar_next = bar_first(c.bar, G);
+        if (rank > 0) next.rest = first(SUB_REST);
+        if (G >= 4) next.half = first(SUB_HALF);
+        if (G >= 8) next.quarter = first(SUB_QUARTER);
+    }
+    c.tred = c.A + S.tred;
     c.tpar = 0;
-    c.bar2 = reinterpret_cast<unsigned long long*>(S.iarena + S.bar + BAR_SUB1);
-    c.tred2 = c.tred + 2 * MAX_TEAM;
-    c.tpar2 = 0;
-    c.bar_lo = reinterpret_cast<unsigned long long*>(S.iarena + S.bar + BAR_LO);
-    c.tred_lo = c.tred + 4 * MAX_TEAM;
-    c.tpar_lo = 0;
-    c.bar_hi = reinterpret_cast<unsigned long long*>(S.iarena + S.bar + BAR_HI);
-    c.tred_hi = c.tred + 6 * MAX_TEAM;
-    c.tpar_hi = 0;
-    c.bar_q = reinterpret_cast<unsigned long long*>(S.iarena + S.bar + BAR_Q);
-    c.tred_q = c.tred + 8 * MAX_TEAM;
-    c.tpar_q = 0;
     c.bp_layout = args.bp_layout;
     c.args = &args;
-    team_place(c, S.iarena + S.bar + 4);
-    if (args.n_round == 0) {
-        compute(c, S, args.mode);
-        return;
-    }
+    team_place(c, words + 4);
+    uint64_t inv = S.n_invocations;  // thermostat applications so far (kept here, stored after each one)
+    SysDesc& D = systems[sys];
     if (args.n_round < 0) {  // thermostat application only (fresh-start thermalisation)
-        thermostat(c, S, S.noise_scale);
+        RUN(ph_thermostat(mem, S.noise_scale, inv));
+        if (c.gtid == 0) D.n_invocations = inv + 1;
         return;
     }
-    auto pos = gmem(c.A + S.pos_out);
-    auto der = gmem(c.A + S.pos_sens);
-    auto mom = gmem(c.A + S.mom);
-    int nf = 0;
-    for (int rr = 0; rr < args.n_round; ++rr) {
-        int round = args.first_round + rr;
-        if (args.frame_interval > 0 && round % args.frame_interval == 0) {
-            compute(c, S, 1);
-            if (c.I[c.err]) return;
+    // one evaluation at a time: the frame a round may start with, its three
+    // integration stages, the replica exchange it may end with
+    enum { EV_SINGLE, EV_FRAME, EV_STAGE, EV_REX };
+    auto pos = c.A + S.pos_out;
+    auto der = c.A + S.pos_sens;
+    auto mom = c.A + S.mom;
+    int nf = 0, rr = 0, stage = 0;
+    bool start_round = args.n_round > 0, framed = false;
+    int ev = EV_SINGLE;
+    for (;;) {
+        const int round = args.first_round + rr;
+        if (start_round) {
+            if (!framed && args.frame_interval > 0 && round % args.frame_interval == 0) {
+                ev = EV_FRAME;
+            } else {
+                unsigned long long t0 = ptick(c);
+                if (args.thermostat_interval > 0 && round % args.thermostat_interval == 0) {
+                    float ns = S.noise_scale;
+                    if (args.anneal) {  // set_temperature then the update_parameters of src/thermostat.h:9-12
+                        const float time = 3.f * args.dt * (float)(round + 1);
+                        const float temp = (float)anneal_temperature(args, (double)S.temp0, (double)time);
+                        ns = sqrtf(temp * (1.f - S.mom_scale * S.mom_scale));
+                    }
+                    RUN(ph_thermostat(mem, ns, inv));
+                    ++inv;
+                    if (c.gtid == 0) D.n_invocations = inv;
+                }
+                pacc(c, PROF_THERMO, t0);
+                ev = EV_STAGE;
+                stage = 0;
+                start_round = false;
+            }
+        }
+        const bool ok = compute(c, next, mem, words, ev == EV_STAGE ? 0 : ev == EV_SINGLE ? args.mode : 1);
+        if (!ok && ev != EV_REX) return;  // capacity overflow: the host repeats the run
+        if (ev == EV_SINGLE) return;
+        if (ev == EV_FRAME) {
             if (args.frame_pot && c.gtid == 0 && nf < args.n_frames)
                 args.frame_pot[sys * args.n_frames + nf] = total_potential(c, S);
             ++nf;
+            framed = true;
             team_sync(c);
+            continue;
         }
-        unsigned long long t0 = ptick(c);
-        if (args.thermostat_interval > 0 && round % args.thermostat_interval == 0) {
-            float ns = S.noise_scale;
-            if (args.anneal) {  // set_temperature then the update_parameters of src/thermostat.h:9-12
-                const float time = 3.f * args.dt * (float)(round + 1);
-                const float temp = (float)anneal_temperature(args, (double)S.temp0, (double)time);
-                ns = sqrtf(temp * (1.f - S.mom_scale * S.mom_scale));
-            }
-            thermostat(c, S, ns);
-        }
-        pacc(c, PROF_THERMO, t0);
-        for (int stage = 0; stage < 3; ++stage) {
-            compute(c, S, 0);
-            if (c.I[c.err]) return;  // capacity overflow: the host repeats the run
-            t0 = ptick(c);
+        if (ev == EV_STAGE) {
+            unsigned long long t0 = ptick(c);
             c.cur_op = S.n_germ + S.n_deriv;
             for (int i = c.gtid; i < S.n_atom * 3; i += c.gsize) {
                 float p = mom[i] - args.dt * der[i];
@@ -1453,14 +1472,21 @@ __device__ __forceinline__ void engine_body(SysDesc* systems, const RunArgs& arg
             }
             team_sync(c);
             pacc(c, PROF_INTEGRATE, t0);
+            if (++stage < 3) continue;
+            // replica exchange where a segment of the reference's loop ends
+            // (src/main.cpp:991-997): after this round the count of completed
+            // rounds is round + 1
+            if (args.rex.interval > 0 && (long long)round + 1 == (long long)uni64((unsigned long long)args.rex.state[1])) {
+                ev = EV_REX;
+                continue;
+            }
+        } else {
+            RUN(ph_exchange(mem, sys, (long long)round + 1));
+            if (!ok) return;
         }
-        // replica exchange where a segment of the reference's loop ends
-        // (src/main.cpp:991-997): after this round the count of completed
-        // rounds is round + 1
-        if (args.rex.interval > 0 && (long long)round + 1 == args.rex.state[1]) {
-            rex_attempt(c, S, args.rex, sys, args.n_sys, (long long)round + 1);
-            if (c.I[c.err]) return;
-        }
+        if (++rr >= args.n_round) return;
+        start_round = true;
+        framed = false;
     }
 }
 
@@ -1468,16 +1494,18 @@ __device__ __forceinline__ void engine_body(SysDesc* systems, const RunArgs& arg
 __global__ void __launch_bounds__(NT) engine_step_kernel(SysDesc* systems, RunArgs args) {
     __shared__ float red[NWAVE];
     __shared__ int ired[NWAVE];
+    __shared__ __attribute__((aligned(16))) int ctx[NWAVE * CTX_WORDS];
     extern __shared__ float lds[];
-    engine_body(systems, args, red, ired, lds);
+    engine_body(systems, (lp<float>)red, (lp<int>)ired, (lp<int>)ctx, (lp<float>)lds);
 }
 
 // One evaluation (args.n_round == 0) or one thermostat application (< 0).
 __global__ void __launch_bounds__(NT) engine_eval_kernel(SysDesc* systems, RunArgs args) {
     __shared__ float red[NWAVE];
     __shared__ int ired[NWAVE];
+    __shared__ __attribute__((aligned(16))) int ctx[NWAVE * CTX_WORDS];
     extern __shared__ float lds[];
-    engine_body(systems, args, red, ired, lds);
+    engine_body(systems, (lp<float>)red, (lp<int>)ired, (lp<int>)ctx, (lp<float>)lds);
 }
 
 // ---- parameter derivatives of spline pair graphs ------------------------------
