@@ -43,13 +43,13 @@ __device__ __forceinline__ unsigned long long uni64(unsigned long long v) {
 // stride over the team's threads (gtid, gsize); team_sync separates phases
 // whose data cross workgroups.
 struct Team {
-    int rank, G;       // workgroup rank in the team, team size
-    int gtid, gsize;   // thread in the team, team threads
-    gp<unsigned long long> bar;   // arrival counter
     unsigned long long bar_next;  // count that opens this workgroup's next barrier on `bar`
-    gp<float> tred;    // reduction scratch, 2 buffers of G floats
     int tpar;          // buffer parity of the next reduction
+    int rank, G;       // workgroup rank in the team, team size (rank is the fourth word: sync_store)
+    int gtid, gsize;   // thread in the team, team threads
     int err;           // int arena offset of the error word this team sets
+    gp<unsigned long long> bar;   // arrival counter
+    gp<float> tred;    // reduction scratch, 2 buffers of G floats
     unsigned long long* prof;  // wall-clock accumulators (null: profiling off)
 };
 
@@ -79,22 +79,24 @@ struct Ctx : Team {
     int tid;               // thread in the workgroup
 };
 
-// A context in LDS, one copy per wave (no wave waits for another's).
+// The context in LDS, one copy per wave (no wave waits for another's): the
+// current one, the whole team's while the current one is narrowed to a part of
+// it, and the next barrier counts of the parts this workgroup belongs to.
 constexpr int CTX_WORDS = (sizeof(Ctx) + 15) / 16 * 4;
+constexpr int CTX_ROOT = CTX_WORDS, CTX_NEXT = 2 * CTX_WORDS;
+constexpr int CTX_WAVE = 2 * CTX_WORDS + 8;
 typedef int i32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ lp<i32x4> ctx_slot(lp<int> mem) {
-    return (lp<i32x4>)(mem + (int)(threadIdx.x >> 6) * CTX_WORDS);
-}
-__device__ __forceinline__ void ctx_store(lp<int> mem, const Ctx& c) {
+__device__ __forceinline__ lp<int> ctx_wave(lp<int> mem) { return mem + (int)(threadIdx.x >> 6) * CTX_WAVE; }
+__device__ __forceinline__ void ctx_store(lp<int> mem, const Ctx& c, int at = 0) {
     int w[CTX_WORDS] = {};
     __builtin_memcpy(w, &c, sizeof(Ctx));
-    lp<i32x4> m = ctx_slot(mem);
+    lp<i32x4> m = (lp<i32x4>)(ctx_wave(mem) + at);
 #pragma unroll
     for (int k = 0; k < CTX_WORDS / 4; ++k) m[k] = i32x4{w[4 * k], w[4 * k + 1], w[4 * k + 2], w[4 * k + 3]};
 }
-__device__ __forceinline__ Ctx ctx_load(lp<int> mem) {
+__device__ __forceinline__ Ctx ctx_load(lp<int> mem, int at = 0) {
     int w[CTX_WORDS];
-    lp<i32x4> m = ctx_slot(mem);
+    lp<i32x4> m = (lp<i32x4>)(ctx_wave(mem) + at);
 #pragma unroll
     for (int k = 0; k < CTX_WORDS / 4; ++k) {
         const i32x4 v = m[k];
@@ -107,18 +109,14 @@ __device__ __forceinline__ Ctx ctx_load(lp<int> mem) {
     c.gtid = c.rank * NT + c.tid;
     return c;
 }
-
-// What a phase function gives back: the barrier state it advanced, and a
-// result.
-struct PhaseRet {
-    unsigned long long bar_next;
-    int tpar, value;
-};
-__device__ __forceinline__ PhaseRet phase_ret(const Ctx& c, int value) { return PhaseRet{c.bar_next, c.tpar, value}; }
-__device__ __forceinline__ int phase_done(Ctx& c, const PhaseRet& r) {
-    c.bar_next = uni64(r.bar_next);
-    c.tpar = uni(r.tpar);
-    return uni(r.value);
+// After barriers and reductions: the words they advance.
+__device__ __forceinline__ void sync_store(lp<int> mem, const Ctx& c) {
+    *(lp<i32x4>)ctx_wave(mem) = i32x4{(int)(unsigned)c.bar_next, (int)(unsigned)(c.bar_next >> 32), c.tpar, c.rank};
+}
+// End of a phase function: leaves the barrier state in LDS, gives back a result.
+__device__ __forceinline__ int phase_ret(lp<int> mem, const Ctx& c, int value) {
+    sync_store(mem, c);
+    return value;
 }
 
 __device__ __forceinline__ unsigned long long ptick(const Ctx& c) { return c.prof ? wall_clock64() : 0ull; }
@@ -195,14 +193,11 @@ __device__ __forceinline__ void team_sync(Ctx& c) {
 // Sub-teams: parts of a team that run beside each other, each with an arrival
 // counter and reduction scratch of its own.  A workgroup belongs to the same
 // part of each kind for a whole launch, so it keeps the kind's barrier count
-// (SubNext) from one use to the next.
+// (two words at CTX_NEXT) from one use to the next.
 enum SubTeam : int {
     SUB_REST = 0,   // ranks 1..G-1, beside rank 0's rotamer solve
     SUB_HALF = 1,   // ranks [0, G/2) and [G/2, G)
     SUB_QUARTER = 2 // ranks [j*G/4, (j+1)*G/4)
-};
-struct SubNext {  // named, not indexed: an indexed array would live in private memory
-    unsigned long long rest, half, quarter;
 };
 struct SubPart { int first, size, word, buf; };  // ranks, counter word, reduction buffer
 __device__ __forceinline__ SubPart sub_part(int kind, int rank, int G) {
@@ -212,29 +207,34 @@ __device__ __forceinline__ SubPart sub_part(int kind, int rank, int G) {
     while (j + 1 < 4 && rank >= (j + 1) * G / 4) ++j;
     return SubPart{j * G / 4, (j + 1) * G / 4 - j * G / 4, BAR_Q + 2 * j, 4 + j};
 }
+__device__ __forceinline__ void sub_next_put(lp<int> mem, int kind, unsigned long long v) {
+    lp<int> m = ctx_wave(mem) + CTX_NEXT + 2 * kind;
+    m[0] = (int)(unsigned)v;
+    m[1] = (int)(unsigned)(v >> 32);
+}
 
-// Narrow the context from the whole team `root` to this workgroup's part of
-// kind `kind`.  Only rank 0 of the whole team keeps the profile accumulators
-// (with `part_prof` the part's first workgroup does, so that each part's ops
-// are timed).
-__device__ __forceinline__ void enter_sub(Ctx& c, const SubNext& next, const Team& root, int kind,
-                                          gp<int> words, unsigned long long* part_prof) {
-    const SubPart p = sub_part(kind, root.rank, root.G);
+// Narrow the context from the whole team to this workgroup's part of kind
+// `kind`.  Each part's first workgroup keeps the profile accumulators `prof`,
+// so that each part's ops are timed.
+__device__ __forceinline__ void enter_sub(lp<int> mem, Ctx& c, int kind, gp<int> words, unsigned long long* prof) {
+    ctx_store(mem, c, CTX_ROOT);
+    const SubPart p = sub_part(kind, c.rank, c.G);
+    lp<int> m = ctx_wave(mem) + CTX_NEXT + 2 * kind;
+    c.bar_next = ((unsigned long long)(unsigned)uni(m[1]) << 32) | (unsigned)uni(m[0]);
     c.G = p.size;
-    c.rank = root.rank - p.first;
+    c.rank -= p.first;
     c.gtid = c.rank * NT + c.tid;
     c.gsize = p.size * NT;
     c.bar = (gp<unsigned long long>)(words + p.word);
-    c.bar_next = kind == SUB_REST ? next.rest : kind == SUB_HALF ? next.half : next.quarter;
-    c.tred = root.tred + p.buf * 2 * MAX_TEAM;
+    c.tred += p.buf * 2 * MAX_TEAM;
     c.tpar = 0;
-    c.prof = c.rank == 0 ? part_prof : nullptr;
+    c.prof = c.rank == 0 ? prof : nullptr;
 }
-__device__ __forceinline__ void leave_sub(Ctx& c, SubNext& next, const Team& root, int kind) {
-    next.rest = kind == SUB_REST ? c.bar_next : next.rest;
-    next.half = kind == SUB_HALF ? c.bar_next : next.half;
-    next.quarter = kind == SUB_QUARTER ? c.bar_next : next.quarter;
-    (Team&)c = root;
+// Back to the whole team.
+__device__ __forceinline__ void leave_sub(lp<int> mem, Ctx& c, int kind) {
+    sub_next_put(mem, kind, c.bar_next);
+    c = ctx_load(mem, CTX_ROOT);
+    ctx_store(mem, c);
 }
 
 // XCD of the calling workgroup (hardware register XCC_ID).

@@ -13,11 +13,11 @@
 
 namespace upside {
 
-// Dynamic LDS per workgroup (158 KB of the 160 KB a gfx950 workgroup may
+// Dynamic LDS per workgroup (156 KB of the 160 KB a gfx950 workgroup may
 // hold, the rest being the static reduction scratch and the waves' contexts): staging for pair-graph
 // coefficient tables (the largest, the rotamer pair table, is 20*20*54 floats
 // = 86.4 KB, plus read-past padding), cell grids, and the rotamer solve state.
-constexpr int LDS_FLOATS = 40448;
+constexpr int LDS_FLOATS = 39936;
 // Rotamer statistics words: [0] iterations of the last solve, [1] solves at
 // the iteration limit, [2] total iterations, [3] solves, [4] BP edges, [5]
 // residue-pair candidates, [6] solves held in LDS, [7] warm-started solves,
@@ -205,6 +205,18 @@ struct OpRec {
                            // beside each other (their lists may overflow, so the error words are read)
 };
 
+// What the interpreter goes by, one word per program op side by side (an op
+// record is five cache lines).
+enum : int {
+    FLAG_LANE = 3,         // mask: OpRec::lane
+    FLAG_SOLO = 4,
+    FLAG_EARLY = 8,
+    FLAG_GRAPH = 16,       // has a pair graph
+    FLAG_ROTAMER = 32,
+    FLAG_SECTION = 64,     // starts a section (OpRec::lane_end)
+    FLAG_GATHER = 128      // value op whose graph's sensitivities are summed right after it
+};
+
 struct SysDesc {
     float* arena;          // per-system float arena
     int* iarena;           // per-system int arena
@@ -228,6 +240,7 @@ struct SysDesc {
     float temp0;           // initial temperature (annealing schedule)
     int error;             // int offset of error word (then one per section sub-team)
     int n_lanes;           // lanes of the program's sections (2 or 4)
+    int flags;             // const int offset of the ops' flags (FLAG_*), one word per program op
     int bar;               // int offset (16-byte aligned) of the team barrier words: [0..1] 64-bit
                            // arrival counter, [2] spin-timeout flag, [3] placement report, [4..4+MAX_TEAM)
                            // XCD of each workgroup, [4+MAX_TEAM..+2) 64-bit counter of the sub-team

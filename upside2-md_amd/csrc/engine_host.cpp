@@ -1300,6 +1300,7 @@ struct Program {
     PivotMoves pivots;                       // /input/pivot_moves, if present
     vector<OpRec> prog;                      // the uploaded program (d_ops)
     vector<int> prog_node;                   // node of each program entry
+    int flags_at = 0;                        // the program's flags in the constant ints (SysDesc::flags)
 
     // Parameter vector of a node in the reference's get_param layout, and
     // where it lives here: a pair graph's interaction table (constant floats);
@@ -1676,6 +1677,15 @@ struct Program {
             for (int q = prog[k].kind == OP_ROTAMER ? k + 1 : k; q < e; ++q)
                 if (prog[q].graph >= 0) prog[k].lane_graphs = 1;
         }
+        vector<int> flags;
+        for (int k = 0; k < (int)prog.size(); ++k) {
+            const OpRec& o = prog[k];
+            flags.push_back((k < ng ? o.lane : 0) | (o.solo ? FLAG_SOLO : 0) | (o.early ? FLAG_EARLY : 0) |
+                            (o.graph >= 0 ? FLAG_GRAPH : 0) | (o.kind == OP_ROTAMER ? FLAG_ROTAMER : 0) |
+                            (k < ng && o.lane_end > k ? FLAG_SECTION : 0) |
+                            (o.kind == OP_BACKBONE_PAIRS ? FLAG_GATHER : 0));
+        }
+        flags_at = T.ci_push(flags);
         if (!upload) return;  // lowering only (check_program)
         auto up = [](void** dst, const void* src, size_t bytes, const char* what) {
             hip_check(hipMalloc(dst, std::max(bytes, (size_t)16)), what);
@@ -2015,6 +2025,7 @@ struct Batch {
         d.mom = T.mom;
         d.error = T.err;
         d.n_lanes = P.n_lanes;
+        d.flags = P.flags_at;
         d.bar = T.bar;
         d.tred = T.tred;
         d.seed = base_seed + (uint32_t)k;

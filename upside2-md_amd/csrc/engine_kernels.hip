@@ -760,8 +760,12 @@ __device__ __forceinline__ void backbone_fwd(Ctx& c, SysC& S, OpC& op, GraphC& G
 
 // ---- phases -----------------------------------------------------------------------
 // The outlined functions of the kernel.  Each reads the context from LDS, runs
-// one phase on the current team and gives back the barrier state.
-#define PHASE static __device__ __attribute__((noinline)) PhaseRet
+// one phase on the current team and leaves the barrier state there.  (The
+// interpreter between them keeps next to nothing in registers: what it keeps
+// goes to private memory at each call, and came back from L2.  Its state in
+// LDS, ms per step: 0.47 -> 0.34 for 67 residues on 8 workgroups, 0.94 -> 0.73
+// for 500 on 32.)
+#define PHASE static __device__ __attribute__((noinline)) int
 
 // Bring the cache lines of a record into the scalar cache together: read field
 // by field as the code comes to them, each line costs a trip of its own.
@@ -803,7 +807,7 @@ PHASE ph_lists(lp<int> mem, int at) {
         if (c.gtid == 0) c.I[c.err] = 1;
         team_sync(c);
     }
-    return phase_ret(c, ok);
+    return phase_ret(mem, c, ok);
 }
 
 // Refine the cached slots and evaluate the edges of a graph op.
@@ -813,7 +817,7 @@ PHASE ph_edges(lp<int> mem, int at) {
     unsigned long long t0 = ptick(c);
     pg_edges(c, cmem(c.S->graphs)[op.graph], op);
     pacc(c, PROF_PG_EDGES, t0);
-    return phase_ret(c, 1);
+    return phase_ret(mem, c, 1);
 }
 
 // The body of a value op other than the rotamer (whose graph, if it has one,
@@ -848,7 +852,7 @@ PHASE ph_value(lp<int> mem, int at) {
     }
     if (op.kind == OP_SPRING || op.kind == OP_RAMA_MAP_POT) plan_gather(c, op.plans[0]);
     if (op.kind != OP_BACKBONE_PAIRS) team_sync(c);
-    return phase_ret(c, 0);
+    return phase_ret(mem, c, 0);
 }
 
 // A deriv op: the contributions of each element and their sums in plan order;
@@ -887,7 +891,7 @@ PHASE ph_deriv(lp<int> mem, int at) {
             team_sync(c);
         }
     }
-    return phase_ret(c, 0);
+    return phase_ret(mem, c, 0);
 }
 
 // The sums of a graph op's edges.  Ends with a team barrier.
@@ -899,7 +903,7 @@ PHASE ph_gather(lp<int> mem, int at, int value) {
     touch(G);
     pg_gather(c, G);
     if (!uni(value) && op.kind == OP_PROTEIN_HBOND) protein_hbond_pass(c, op, G);
-    return phase_ret(c, 0);
+    return phase_ret(mem, c, 0);
 }
 
 // ---- rotamer (src/rotamer.cpp:840-850) ----------------------------------------------
@@ -910,19 +914,19 @@ PHASE ph_fill(lp<int> mem, int at) {
     unsigned long long t0 = ptick(c);
     rot_fill(c, cmem(c.S->graphs)[op.graph], cmem(c.S->rots)[op.rot]);
     pacc(c, PROF_ROT_FILL, t0);
-    return phase_ret(c, 0);
+    return phase_ret(mem, c, 0);
 }
 
 // The solve, on this workgroup or on the team; gives the iterations.
 PHASE ph_solve_wg(lp<int> mem, int rot) {
     Ctx c = ctx_load(mem);
     const int it = rot_solve_wg(c, cmem(c.S->rots)[uni(rot)]);
-    return phase_ret(c, it);
+    return phase_ret(mem, c, it);
 }
 PHASE ph_solve_team(lp<int> mem, int rot) {
     Ctx c = ctx_load(mem);
     const int it = rot_solve_team(c, cmem(c.S->rots)[uni(rot)]);
-    return phase_ret(c, it);
+    return phase_ret(mem, c, it);
 }
 
 // After the solve (it: iteration count, on gtid 0): statistics, edge and
@@ -940,21 +944,18 @@ PHASE ph_sens(lp<int> mem, int at, int it) {
         st[BP_HIST + min(it, BP_HIST_BINS - 1)] += 1;
     }
     rot_sens(c, cmem(c.S->graphs)[op.graph], R);
-    return phase_ret(c, 0);
+    return phase_ret(mem, c, 0);
 }
 PHASE ph_free_energy(lp<int> mem, int at) {
     Ctx c = ctx_load(mem);
     OpC& op = cmem(c.S->ops)[uni(at)];
     const float fe = rot_free_energy(c, cmem(c.S->graphs)[op.graph], cmem(c.S->rots)[op.rot]);
     put_pot(c, *c.S, op, fe);
-    return phase_ret(c, 0);
+    return phase_ret(mem, c, 0);
 }
 
 
 // ---- program interpreter ----------------------------------------------------------
-// Run a phase function on the team c.
-#define RUN(call) phase_done(c, (ctx_store(mem, c), call))
-
 // One evaluation: value ops in germ order, then sensitivity pushes in deriv
 // order.  False on a capacity overflow (uniform over the team).
 //
@@ -980,21 +981,24 @@ PHASE ph_free_energy(lp<int> mem, int at) {
 //  * DERIV: the deriv ops (those not already run early) on the whole team.
 enum Where : int { MAIN = 0, SECTION, BESIDE, BESIDE_DERIV, DERIV };
 
-__device__ __forceinline__ bool compute(Ctx& c, SubNext& next, lp<int> mem, gp<int> words, int mode) {
-    SysC& S = *c.S;
-    cp<OpRec> ops = cmem(S.ops);
+// Per op, the bits the interpreter goes by (SysDesc::flags).
+__device__ __forceinline__ bool compute(lp<int> mem, gp<int> words, int mode) {
+    SysC& S = *ctx_load(mem).S;
+    cp<int> flags = cmem((const int*)S.ci) + S.flags;
     const int ng = S.n_germ, nd = S.n_germ + S.n_deriv;
-    c.cur_op = nd;  // outside the ops
-    for (int r = 0; r < S.sens_zero_cnt; ++r) {
-        cp<int> zr = (cp<int>)(c.I + S.sens_zero + 2 * r);  // written once, by the host
-        gp<float> p = c.A + zr[0];
-        const int n = zr[1];
-        for (int i = c.gtid; i < n; i += c.gsize) p[i] = 0.f;
+    {
+        Ctx c = ctx_load(mem);
+        c.cur_op = nd;  // outside the ops
+        for (int r = 0; r < S.sens_zero_cnt; ++r) {
+            cp<int> zr = (cp<int>)(c.I + S.sens_zero + 2 * r);  // written once, by the host
+            gp<float> p = c.A + zr[0];
+            const int n = zr[1];
+            for (int i = c.gtid; i < n; i += c.gsize) p[i] = 0.f;
+        }
+        team_sync(c);
+        ctx_store(mem, c);
     }
-    team_sync(c);
-
-    Team root = c;              // the whole team, while c is narrowed to a part of it
-    int sub = -1;               // kind of the part (SubTeam), -1: the whole team
+    int sub = -1;               // kind of the part the context is narrowed to (SubTeam), -1: the whole team
     int where = MAIN, k = 0, end = ng;
     unsigned lanes = 0;         // SECTION: lanes this part runs
     int section = 0;            // SECTION: its first op
@@ -1011,25 +1015,27 @@ __device__ __forceinline__ bool compute(Ctx& c, SubNext& next, lp<int> mem, gp<i
         where = uni(where); k = uni(k); end = uni(end); sub = uni(sub); lanes = (unsigned)uni((int)lanes);
         rot_graph = uni(rot_graph); rot_k = uni(rot_k); solo_of = uni(solo_of); section = uni(section);
         rot_ready = uni(rot_ready); post = uni(post) != 0; early_done = uni(early_done) != 0;
+        Ctx c = ctx_load(mem);
         // the next op of the range that is this team's
         if (rot_graph < 0 && !post) {
             if (where == SECTION)
-                while (k < end && !((lanes >> ops[k].lane) & 1u)) ++k;
+                while (k < end && !((lanes >> (flags[k] & FLAG_LANE)) & 1u)) ++k;
             else if (where == BESIDE_DERIV)
-                while (k < end && !ops[k].early) ++k;
+                while (k < end && !(flags[k] & FLAG_EARLY)) ++k;
             else if (where == DERIV && early_done)
-                while (k < end && ops[k].early) ++k;
+                while (k < end && (flags[k] & FLAG_EARLY)) ++k;
         }
         const int at = uni(rot_graph >= 0 ? rot_graph : post ? rot_k : k);
         const bool done = rot_graph < 0 && !post && k >= end;
-        OpC& op = ops[done ? 0 : at];
-        const bool starts_section = !done && where == MAIN && !post && op.lane_end > k && (solo_of ? solo_of : c.G) >= 4;
-        const bool solo = !done && !post && rot_graph < 0 && !starts_section && op.solo && (solo_of || c.G > 1);
+        const int fl = done ? 0 : flags[at];
+        const bool starts_section = (fl & FLAG_SECTION) && where == MAIN && !post && (solo_of ? solo_of : c.G) >= 4;
+        const bool solo = (fl & FLAG_SOLO) && !post && rot_graph < 0 && !starts_section && (solo_of || c.G > 1);
         if (solo_of && !solo) {  // a run of solo ops ends
             c.G = solo_of;
             c.gsize = c.G * NT;
             solo_of = 0;
             team_sync(c);
+            ctx_store(mem, c);
         }
         if (done) {
             if (where == MAIN) {
@@ -1037,16 +1043,18 @@ __device__ __forceinline__ bool compute(Ctx& c, SubNext& next, lp<int> mem, gp<i
                 k = ng;
                 end = nd;
             } else if (where == SECTION) {
-                leave_sub(c, next, root, sub);
+                leave_sub(mem, c, sub);
                 sub = -1;
                 team_sync(c);
-                OpC& first = ops[section];
+                sync_store(mem, c);
+                OpC& first = cmem(S.ops)[section];
                 if (first.lane_graphs) {  // the join made every part's error word readable
                     int e = 0;
                     for (int q = 1; q <= MAX_LANES; ++q) e |= c.I[S.error + q];
                     if (uni(e)) {
                         if (c.gtid == 0) c.I[c.err] = 1;
                         team_sync(c);
+                        sync_store(mem, c);
                         return false;
                     }
                 }
@@ -1064,9 +1072,10 @@ __device__ __forceinline__ bool compute(Ctx& c, SubNext& next, lp<int> mem, gp<i
                     if (S.prof && c.gtid == 0)
                         __hip_atomic_fetch_add(S.prof + c.pbase + PROF_BESIDE, wall_clock64() - t_beside,
                                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    leave_sub(c, next, root, sub);
+                    leave_sub(mem, c, sub);
                     sub = -1;
                     team_sync(c);
+                    sync_store(mem, c);
                 }
                 pacc(c, PROF_BP, t_bp);
                 post = true;
@@ -1078,13 +1087,14 @@ __device__ __forceinline__ bool compute(Ctx& c, SubNext& next, lp<int> mem, gp<i
             continue;
         }
         if (starts_section) {
-            root = c;
+            OpC& op = cmem(S.ops)[at];
             sub = (S.n_lanes == 4 && c.G >= 8 && c.args->lane_split == 4) ? SUB_QUARTER : SUB_HALF;
             const SubPart p = sub_part(sub, c.rank, c.G);
             const int j = sub == SUB_QUARTER ? (p.word - BAR_Q) / 2 : (p.first ? 1 : 0);
             lanes = (sub == SUB_QUARTER || S.n_lanes == 2) ? (1u << j) : ((1u << j) | (1u << (j + 2)));
-            enter_sub(c, next, root, sub, words, S.prof);
+            enter_sub(mem, c, sub, words, S.prof);
             c.err = S.error + 1 + j;
+            ctx_store(mem, c);
             section = k;
             where = SECTION;
             end = op.lane_end;
@@ -1094,29 +1104,38 @@ __device__ __forceinline__ bool compute(Ctx& c, SubNext& next, lp<int> mem, gp<i
         if (solo) {
             if (!solo_of) {
                 solo_of = c.G;
-                if (c.rank == 0) { c.G = 1; c.gsize = NT; }
+                if (c.rank == 0) {
+                    c.G = 1;
+                    c.gsize = NT;
+                    ctx_store(mem, c);
+                }
             }
             if (c.rank != 0) { ++k; continue; }
         }
-        c.cur_op = at;
+        if (c.prof) {  // barriers are counted per op
+            c.cur_op = at;
+            ctx_store(mem, c);
+        }
         const bool value = where <= BESIDE;
-        const bool rot = op.kind == OP_ROTAMER;
-        unsigned long long t0 = ptick(c);
-        if (value && op.graph >= 0 && !post && at != rot_ready) {
-            if (!RUN(ph_lists(mem, at))) {
+        const bool rot = (fl & FLAG_ROTAMER) != 0;
+        const unsigned long long t0 = ptick(c);
+        if (value && (fl & FLAG_GRAPH) && !post && at != rot_ready) {
+            if (!uni(ph_lists(mem, at))) {
                 if (where == MAIN) return false;
                 rot_graph = -1;  // to the join
                 if (where == BESIDE) where = BESIDE_DERIV;
                 k = end = 0;
                 continue;
             }
-            RUN(ph_edges(mem, at));
+            ph_edges(mem, at);
             if (rot_graph >= 0) { rot_graph = -1; continue; }
         }
         if (rot && !post) {
-            RotC& R = cmem(S.rots)[op.rot];
             t_rot = t0;
-            RUN(ph_fill(mem, at));
+            ph_fill(mem, at);
+            c = ctx_load(mem);
+            OpC& op = cmem(S.ops)[at];
+            RotC& R = cmem(S.rots)[op.rot];
             t_bp = ptick(c);
             rot_k = k;
             const bool ranged = where == MAIN && op.overlap_end > k;
@@ -1126,23 +1145,32 @@ __device__ __forceinline__ bool compute(Ctx& c, SubNext& next, lp<int> mem, gp<i
             // whole team (or its rank 0), and the range follows
             bool solve = !wg || c.rank == 0;
             if (ranged && c.G > 1 && (wg || (c.bp_layout != 1 && c.G >= 4))) {
-                root = c;
                 sub = wg ? SUB_REST : SUB_HALF;
                 solve = wg ? c.rank == 0 : c.rank < c.G / 2;
-                if (!wg || c.rank != 0) enter_sub(c, next, root, sub, words, S.prof);
+                if (!wg || c.rank != 0) {
+                    enter_sub(mem, c, sub, words, S.prof);
+                    ctx_store(mem, c);
+                }
                 t_beside = S.prof ? wall_clock64() : 0ull;
             }
-            if (solve) it = wg ? RUN(ph_solve_wg(mem, op.rot)) : RUN(ph_solve_team(mem, op.rot));
+            if (solve) {
+                it = wg ? ph_solve_wg(mem, op.rot) : ph_solve_team(mem, op.rot);
+                c = ctx_load(mem);
+            }
             if (sub >= 0 && solve) {  // join; an error in the range is read after the rotamer
-                if (!wg) leave_sub(c, next, root, sub);
+                if (!wg) leave_sub(mem, c, sub);
                 sub = -1;
                 team_sync(c);
+                sync_store(mem, c);
                 pacc(c, PROF_BP, t_bp);
                 post = true;
                 early_done = true;
                 continue;
             }
-            if (sub < 0 && wg && c.G > 1) team_sync(c);
+            if (sub < 0 && wg && c.G > 1) {
+                team_sync(c);
+                sync_store(mem, c);
+            }
             if (ranged) {
                 early_done = true;
                 where = BESIDE;
@@ -1156,10 +1184,11 @@ __device__ __forceinline__ bool compute(Ctx& c, SubNext& next, lp<int> mem, gp<i
         }
         // the op's body, then the sums it leaves
         if (post) {
-            RUN(ph_sens(mem, at, it));
-            RUN(ph_gather(mem, at, 1));
-            if (mode) RUN(ph_free_energy(mem, at));
-            else put_pot(c, S, op, 0.f);
+            ph_sens(mem, at, it);
+            ph_gather(mem, at, 1);
+            if (mode) ph_free_energy(mem, at);
+            OpC& op = cmem(S.ops)[at];
+            if (!mode) put_pot(c, S, op, 0.f);
             prof_op(c, at, t_rot);
             if (op.lane_graphs && uni(c.I[c.err])) return false;
             post = false;
@@ -1167,11 +1196,11 @@ __device__ __forceinline__ bool compute(Ctx& c, SubNext& next, lp<int> mem, gp<i
             continue;
         }
         if (value) {
-            RUN(ph_value(mem, at));
-            if (op.kind == OP_BACKBONE_PAIRS) RUN(ph_gather(mem, at, 1));
+            ph_value(mem, at);
+            if (fl & FLAG_GATHER) ph_gather(mem, at, 1);
         } else {
-            RUN(ph_deriv(mem, at));
-            if (op.graph >= 0) RUN(ph_gather(mem, at, 0));
+            ph_deriv(mem, at);
+            if (fl & FLAG_GRAPH) ph_gather(mem, at, 0);
         }
         prof_op(c, at, t0);
         ++k;
@@ -1241,6 +1270,7 @@ __device__ __forceinline__ double anneal_temperature(UPS_CONST const RunArgs& a,
 PHASE ph_thermostat(lp<int> mem, float noise_scale, uint64_t inv) {
     Ctx c = ctx_load(mem);
     SysC& S = *c.S;
+    const unsigned long long t0 = ptick(c);
     auto mom = c.A + S.mom;
     for (int a = c.gtid; a < S.n_atom; a += c.gsize) {
         float n[3];
@@ -1248,7 +1278,28 @@ PHASE ph_thermostat(lp<int> mem, float noise_scale, uint64_t inv) {
         for (int k = 0; k < 3; ++k)
             mom[a * 3 + k] = __fmaf_rn(noise_scale, n[k], __fmul_rn(S.mom_scale, mom[a * 3 + k]));
     }
-    return phase_ret(c, 0);
+    pacc(c, PROF_THERMO, t0);
+    return phase_ret(mem, c, 0);
+}
+
+// One symplectic-Euler stage (src/deriv_engine.cpp:317-331).
+PHASE ph_integrate(lp<int> mem) {
+    Ctx c = ctx_load(mem);
+    SysC& S = *c.S;
+    auto pos = c.A + S.pos_out;
+    auto der = c.A + S.pos_sens;
+    auto mom = c.A + S.mom;
+    const float dt = c.args->dt;
+    const unsigned long long t0 = ptick(c);
+    c.cur_op = c.pbase;
+    for (int i = c.gtid; i < S.n_atom * 3; i += c.gsize) {
+        float p = mom[i] - dt * der[i];
+        mom[i] = p;
+        pos[i] += dt * p;
+    }
+    team_sync(c);
+    pacc(c, PROF_INTEGRATE, t0);
+    return phase_ret(mem, c, 0);
 }
 
 __device__ __forceinline__ float total_potential(Ctx& c, SysC& S) {
@@ -1350,7 +1401,7 @@ PHASE ph_exchange(lp<int> mem, int sys_, long long done) {
         for (int i = c.gtid; i < S.n_atom * 3; i += c.gsize) pos[i] = st[i];
     }
     team_sync(c);
-    return phase_ret(c, 0);
+    return phase_ret(mem, c, 0);
 }
 
 // One launch evaluates or integrates every system of a batch; system s is
@@ -1394,36 +1445,33 @@ __device__ __forceinline__ void engine_body(SysDesc* systems, lp<float> red, lp<
     c.bar = (gp<unsigned long long>)words;  // 16-byte aligned words
     c.bar_flag = (gp<unsigned>)(words + 2);
     c.bar_next = 0;
-    SubNext next = {0, 0, 0};
     if (G > 1) {
         // read before this workgroup's first arrival at any of them
         auto first = [&](int kind) {
             const SubPart p = sub_part(kind, rank, G);
-            return bar_first((gp<unsigned long long>)(words + p.word), p.size);
+            sub_next_put(mem, kind, bar_first((gp<unsigned long long>)(words + p.word), p.size));
         };
         c.bar_next = bar_first(c.bar, G);
-        if (rank > 0) next.rest = first(SUB_REST);
-        if (G >= 4) next.half = first(SUB_HALF);
-        if (G >= 8) next.quarter = first(SUB_QUARTER);
+        if (rank > 0) first(SUB_REST);
+        if (G >= 4) first(SUB_HALF);
+        if (G >= 8) first(SUB_QUARTER);
     }
     c.tred = c.A + S.tred;
     c.tpar = 0;
     c.bp_layout = args.bp_layout;
     c.args = &args;
     team_place(c, words + 4);
+    ctx_store(mem, c);
     uint64_t inv = S.n_invocations;  // thermostat applications so far (kept here, stored after each one)
     SysDesc& D = systems[sys];
     if (args.n_round < 0) {  // thermostat application only (fresh-start thermalisation)
-        RUN(ph_thermostat(mem, S.noise_scale, inv));
+        ph_thermostat(mem, S.noise_scale, inv);
         if (c.gtid == 0) D.n_invocations = inv + 1;
         return;
     }
     // one evaluation at a time: the frame a round may start with, its three
     // integration stages, the replica exchange it may end with
     enum { EV_SINGLE, EV_FRAME, EV_STAGE, EV_REX };
-    auto pos = c.A + S.pos_out;
-    auto der = c.A + S.pos_sens;
-    auto mom = c.A + S.mom;
     int nf = 0, rr = 0, stage = 0;
     bool start_round = args.n_round > 0, framed = false;
     int ev = EV_SINGLE;
@@ -1433,7 +1481,6 @@ __device__ __forceinline__ void engine_body(SysDesc* systems, lp<float> red, lp<
             if (!framed && args.frame_interval > 0 && round % args.frame_interval == 0) {
                 ev = EV_FRAME;
             } else {
-                unsigned long long t0 = ptick(c);
                 if (args.thermostat_interval > 0 && round % args.thermostat_interval == 0) {
                     float ns = S.noise_scale;
                     if (args.anneal) {  // set_temperature then the update_parameters of src/thermostat.h:9-12
@@ -1441,37 +1488,30 @@ __device__ __forceinline__ void engine_body(SysDesc* systems, lp<float> red, lp<
                         const float temp = (float)anneal_temperature(args, (double)S.temp0, (double)time);
                         ns = sqrtf(temp * (1.f - S.mom_scale * S.mom_scale));
                     }
-                    RUN(ph_thermostat(mem, ns, inv));
+                    ph_thermostat(mem, ns, inv);
                     ++inv;
-                    if (c.gtid == 0) D.n_invocations = inv;
+                    if (rank == 0 && threadIdx.x == 0) D.n_invocations = inv;
                 }
-                pacc(c, PROF_THERMO, t0);
                 ev = EV_STAGE;
                 stage = 0;
                 start_round = false;
             }
         }
-        const bool ok = compute(c, next, mem, words, ev == EV_STAGE ? 0 : ev == EV_SINGLE ? args.mode : 1);
+        const bool ok = compute(mem, words, ev == EV_STAGE ? 0 : ev == EV_SINGLE ? args.mode : 1);
         if (!ok && ev != EV_REX) return;  // capacity overflow: the host repeats the run
         if (ev == EV_SINGLE) return;
         if (ev == EV_FRAME) {
+            c = ctx_load(mem);
             if (args.frame_pot && c.gtid == 0 && nf < args.n_frames)
                 args.frame_pot[sys * args.n_frames + nf] = total_potential(c, S);
             ++nf;
             framed = true;
             team_sync(c);
+            sync_store(mem, c);
             continue;
         }
         if (ev == EV_STAGE) {
-            unsigned long long t0 = ptick(c);
-            c.cur_op = S.n_germ + S.n_deriv;
-            for (int i = c.gtid; i < S.n_atom * 3; i += c.gsize) {
-                float p = mom[i] - args.dt * der[i];
-                mom[i] = p;
-                pos[i] += args.dt * p;
-            }
-            team_sync(c);
-            pacc(c, PROF_INTEGRATE, t0);
+            ph_integrate(mem);
             if (++stage < 3) continue;
             // replica exchange where a segment of the reference's loop ends
             // (src/main.cpp:991-997): after this round the count of completed
@@ -1481,7 +1521,7 @@ __device__ __forceinline__ void engine_body(SysDesc* systems, lp<float> red, lp<
                 continue;
             }
         } else {
-            RUN(ph_exchange(mem, sys, (long long)round + 1));
+            ph_exchange(mem, sys, (long long)round + 1);
             if (!ok) return;
         }
         if (++rr >= args.n_round) return;
@@ -1494,7 +1534,7 @@ __device__ __forceinline__ void engine_body(SysDesc* systems, lp<float> red, lp<
 __global__ void __launch_bounds__(NT) engine_step_kernel(SysDesc* systems, RunArgs args) {
     __shared__ float red[NWAVE];
     __shared__ int ired[NWAVE];
-    __shared__ __attribute__((aligned(16))) int ctx[NWAVE * CTX_WORDS];
+    __shared__ __attribute__((aligned(16))) int ctx[NWAVE * CTX_WAVE];
     extern __shared__ float lds[];
     engine_body(systems, (lp<float>)red, (lp<int>)ired, (lp<int>)ctx, (lp<float>)lds);
 }
@@ -1503,7 +1543,7 @@ __global__ void __launch_bounds__(NT) engine_step_kernel(SysDesc* systems, RunAr
 __global__ void __launch_bounds__(NT) engine_eval_kernel(SysDesc* systems, RunArgs args) {
     __shared__ float red[NWAVE];
     __shared__ int ired[NWAVE];
-    __shared__ __attribute__((aligned(16))) int ctx[NWAVE * CTX_WORDS];
+    __shared__ __attribute__((aligned(16))) int ctx[NWAVE * CTX_WAVE];
     extern __shared__ float lds[];
     engine_body(systems, (lp<float>)red, (lp<int>)ired, (lp<int>)ctx, (lp<float>)lds);
 }
