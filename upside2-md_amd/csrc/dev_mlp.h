@@ -37,9 +37,10 @@ constexpr int MLP_OFF_B2 = MLP_OFF_W2 + MLP_H * MLP_H;
 constexpr int MLP_OFF_W3 = MLP_OFF_B2 + MLP_H;
 constexpr int MLP_OFF_B3 = MLP_OFF_W3 + MLP_OUT * MLP_H;
 constexpr int MLP_NPARAM = MLP_OFF_B3 + MLP_OUT;
-// Workgroups of the gradient kernel (each writes one partial gradient; the
-// partials are summed in workgroup order).
+// Fewest and most workgroups of the gradient kernel (each writes one partial
+// gradient; the partials are summed in workgroup order).
 constexpr int MLP_PARTS = 32;
+constexpr int MLP_MAX_PARTS = 256;
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));

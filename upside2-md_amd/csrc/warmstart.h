@@ -12,13 +12,14 @@ hipError_t upside_mlp_launch_partial(const upside::MlpDev& w, const float* feat,
                                      int row0, int n_batch, float inv_n, float* partial, int n_part,
                                      hipStream_t s);
 hipError_t upside_mlp_launch_reduce(const float* partial, int n_part, float* master, float* m1, float* m2,
-                                    float* grad_out, int adam, float lr, float beta1, float beta2, float eps,
-                                    float bc1, float bc2, hipStream_t s);
+                                    float* grad_out, float* loss_out, int adam, float lr, float beta1, float beta2,
+                                    float eps, float bc1, float bc2, const upside::MlpDev& w, hipStream_t s);
 hipError_t upside_mlp_launch_pack(const float* master, __bf16* w1, __bf16* w2p, __bf16* w3p, __bf16* w3tp,
                                   __bf16* w2tp, float* b1, float* b2, float* b3, hipStream_t s);
 hipError_t upside_mlp_launch_forward(const upside::MlpDev& w, const float* feat, int n, float* out,
                                      hipStream_t s);
 int upside_mlp_partial_size();
+int upside_mlp_parts(int n_batch);
 
 namespace upside {
 

@@ -86,9 +86,10 @@ struct UpsideMlp {
     float* grad = nullptr;     // MLP_NPARAM + 1 (loss last)
     float* feat = nullptr;     // [n_rows][MLP_IN]
     float* tgt = nullptr;      // [n_rows][8]
-    float* partial = nullptr;  // [n_part][MLP_NPARAM + 1]
+    float* partial = nullptr;  // [MLP_MAX_PARTS][MLP_NPARAM + 1]
     int n_rows = 0;
-    int n_part = MLP_PARTS;    // workgroups of the gradient kernel
+    float* losses = nullptr;   // [loss_cap] of a training call
+    int loss_cap = 0;
     long long step = 0;
     hipStream_t stream = nullptr;
 
@@ -99,7 +100,7 @@ struct UpsideMlp {
         check(hipMemset(m1, 0, MLP_NPARAM * 4), "adam");
         check(hipMemset(m2, 0, MLP_NPARAM * 4), "adam");
         check(hipMalloc((void**)&grad, (MLP_NPARAM + 1) * 4), "gradient");
-        check(hipMalloc((void**)&partial, (size_t)n_part * upside_mlp_partial_size() * 4), "partials");
+        check(hipMalloc((void**)&partial, (size_t)MLP_MAX_PARTS * upside_mlp_partial_size() * 4), "partials");
         // He-normal hidden layers, zero output layer (the untrained network
         // leaves the first-pass beliefs unchanged), zero biases
         std::vector<float> p(MLP_NPARAM, 0.f);
@@ -109,7 +110,7 @@ struct UpsideMlp {
         params.set(p.data(), stream);
     }
     ~UpsideMlp() {
-        (void)hipFree(m1); (void)hipFree(m2); (void)hipFree(grad); (void)hipFree(partial);
+        (void)hipFree(m1); (void)hipFree(m2); (void)hipFree(grad); (void)hipFree(partial); (void)hipFree(losses);
         (void)hipFree(feat); (void)hipFree(tgt);
         (void)hipStreamDestroy(stream);
     }
@@ -128,9 +129,10 @@ struct UpsideMlp {
     }
 
     // gradient of the mean loss over rows [row0, row0 + nb) (mod n_rows);
-    // with adam, one Adam step
-    void gradient(int row0, int nb, bool adam, float lr) {
+    // with adam, one Adam step; loss (device, may be null) receives the loss
+    void gradient(int row0, int nb, bool adam, float lr, float* loss) {
         if (!n_rows) throw std::runtime_error("no training data set");
+        const int n_part = upside_mlp_parts(nb);
         check(upside_mlp_launch_partial(params.dev, feat, tgt, n_rows, row0, nb, 1.f / (float)nb, partial, n_part,
                                         stream), "warm-start gradient");
         float bc1 = 1.f, bc2 = 1.f;
@@ -139,9 +141,8 @@ struct UpsideMlp {
             bc1 = 1.f - (float)std::pow(0.9, (double)step);
             bc2 = 1.f - (float)std::pow(0.999, (double)step);
         }
-        check(upside_mlp_launch_reduce(partial, n_part, params.master, m1, m2, grad, adam ? 1 : 0, lr, 0.9f, 0.999f,
-                                       1e-8f, bc1, bc2, stream), "warm-start reduce");
-        if (adam) params.pack(stream);
+        check(upside_mlp_launch_reduce(partial, n_part, params.master, m1, m2, grad, loss, adam ? 1 : 0, lr, 0.9f,
+                                       0.999f, 1e-8f, bc1, bc2, params.dev, stream), "warm-start reduce");
     }
 };
 
@@ -189,7 +190,7 @@ int upside_mlp_set_data(UpsideMlp* m, const float* feat, const float* target, in
 
 int upside_mlp_loss_grad(UpsideMlp* m, float* loss, float* grad) {
     MLP_TRY
-    m->gradient(0, m->n_rows, false, 0.f);
+    m->gradient(0, m->n_rows, false, 0.f, nullptr);
     std::vector<float> g(MLP_NPARAM + 1);
     check(hipMemcpyAsync(g.data(), m->grad, g.size() * 4, hipMemcpyDeviceToHost, m->stream), "gradient");
     check(hipStreamSynchronize(m->stream), "gradient");
@@ -204,17 +205,20 @@ int upside_mlp_train(UpsideMlp* m, int n_steps, int batch_rows, float lr, float*
     if (n_steps < 0 || batch_rows <= 0 || !(lr > 0.f)) throw std::runtime_error("bad training arguments");
     if (!m->n_rows) throw std::runtime_error("no training data set");
     const int nb = batch_rows < m->n_rows ? batch_rows : m->n_rows;
-    long long row0 = 0;
-    for (int k = 0; k < n_steps; ++k) {
-        m->gradient((int)(row0 % m->n_rows), nb, true, lr);
-        row0 += nb;
-        if (losses) {
-            float l;
-            check(hipMemcpyAsync(&l, m->grad + MLP_NPARAM, 4, hipMemcpyDeviceToHost, m->stream), "loss");
-            check(hipStreamSynchronize(m->stream), "loss");
-            losses[k] = l;
-        }
+    if (losses && n_steps > m->loss_cap) {
+        (void)hipFree(m->losses);
+        m->losses = nullptr;
+        m->loss_cap = 0;
+        check(hipMalloc((void**)&m->losses, (size_t)n_steps * 4), "losses");
+        m->loss_cap = n_steps;
     }
+    long long row0 = 0;
+    for (int k = 0; k < n_steps; ++k) {  // the steps follow each other on the stream
+        m->gradient((int)(row0 % m->n_rows), nb, true, lr, losses ? m->losses + k : nullptr);
+        row0 += nb;
+    }
+    if (losses && n_steps > 0)
+        check(hipMemcpyAsync(losses, m->losses, (size_t)n_steps * 4, hipMemcpyDeviceToHost, m->stream), "losses");
     check(hipStreamSynchronize(m->stream), "training");
     return 0;
     MLP_CATCH(1)
