@@ -224,6 +224,8 @@ struct SysDesc {
     int n_germ, n_deriv;
     const PairGraph* graphs;
     const RotamerDev* rots;
+    int n_graph;
+    int snap;              // float offset of this system in the batch's snapshot buffer (positions, momenta)
     const float* cf;       // constant float arena (parameters)
     const int* ci;         // constant int arena (index arrays)
     int n_atom;
@@ -329,6 +331,12 @@ struct RunArgs {
     RexDev rex;            // replica exchange between rounds of this launch
 };
 
+// What the host reads after a launch, one record of STATUS_WORDS + n_pot words
+// per system in pinned host memory (status_kernel): [0] a list outgrew its
+// capacity, [2..3] thermostat applications, then the team words, then the
+// potential of every potential node.
+constexpr int STATUS_TEAM = 4;
+
 constexpr int MAX_TEAM = 64;
 // Team words: [0..1] the team's 64-bit arrival counter, [2] spin-timeout flag,
 // [3] placement report, [4..4+MAX_TEAM) XCD of each workgroup, then the
@@ -336,6 +344,7 @@ constexpr int MAX_TEAM = 64;
 // ranks G/2..G-1, and the four quarters [j*G/4, (j+1)*G/4) (each stays a
 // multiple of its own size).
 constexpr int BAR_WORDS = 4 + MAX_TEAM + 14;
+constexpr int STATUS_WORDS = STATUS_TEAM + BAR_WORDS;
 constexpr int BAR_SUB1 = 4 + MAX_TEAM, BAR_LO = 4 + MAX_TEAM + 2, BAR_HI = 4 + MAX_TEAM + 4;
 constexpr int BAR_Q = 4 + MAX_TEAM + 6;
 // Lanes of a program's sections (OpRec::lane < MAX_LANES); error words

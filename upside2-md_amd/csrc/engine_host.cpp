@@ -33,6 +33,11 @@ hipError_t upside_launch_engine(upside::SysDesc* d_systems, int n_sys, upside::R
 hipError_t upside_launch_param_deriv(const upside::ParamDerivArgs& args, int n_rows, hipStream_t stream);
 hipError_t upside_launch_coupling_param_deriv(const upside::CouplingDerivArgs& args, hipStream_t stream);
 hipError_t upside_launch_recenter(float* pos, int n_atom, int xy_only, hipStream_t stream);
+hipError_t upside_launch_status(const upside::SysDesc* systems, int n_sys, int* out, int stride, float* deriv,
+                                hipStream_t stream);
+hipError_t upside_launch_snapshot(const upside::SysDesc* systems, int n_sys, float* snap, int restore,
+                                  hipStream_t stream);
+hipError_t upside_launch_positions(const upside::SysDesc* systems, const float* pos, hipStream_t stream);
 int upside_max_resident_blocks();
 
 namespace upside {
@@ -1862,11 +1867,22 @@ static vector<int> plan_balanced_teams(const vector<int>& atoms, int budget, int
     return t;
 }
 
+// A team whose workgroups were not all running in time (each wait is bounded).
+struct BarrierTimeout : std::runtime_error {
+    using std::runtime_error::runtime_error;
+};
+
 struct Batch {
     vector<std::shared_ptr<Program>> progs;
     vector<System> sys;
     vector<SysDesc> desc;        // host mirror
     SysDesc* d_desc = nullptr;
+    int* status = nullptr;       // pinned: one record per system (STATUS_WORDS)
+    int status_stride = 0;
+    bool pots_fresh = false;     // the records hold the potentials of the last evaluation
+    float* d_snap = nullptr;     // positions and momenta at the start of a run
+    vector<int> snap_at;         // each system's offset there
+    float* stage = nullptr;      // pinned positions and derivative of a one-system engine
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     float last_ms = 0.f;
@@ -1984,6 +2000,9 @@ struct Batch {
         (void)hipFree(d_blockmap);
         for (auto p : prof) (void)hipFree(p);
         (void)hipFree(d_desc);
+        (void)hipFree(d_snap);
+        (void)hipHostFree(status);
+        (void)hipHostFree(stage);
         if (ev0) (void)hipEventDestroy(ev0);
         if (ev1) (void)hipEventDestroy(ev1);
         if (stream) (void)hipStreamDestroy(stream);
@@ -2013,6 +2032,8 @@ struct Batch {
         d.n_deriv = P.n_deriv();
         d.graphs = P.d_graphs;
         d.rots = P.d_rots;
+        d.n_graph = (int)T.graphs.size();
+        d.snap = snap_at[k];
         d.cf = P.d_cf;
         d.ci = P.d_ci;
         d.n_atom = T.n_atom;
@@ -2067,6 +2088,17 @@ struct Batch {
             sys.push_back(s);
         }
         for (auto& s : sys) alloc_system(s);
+        size_t snap_len = 0;
+        int n_pot = 0;
+        for (auto& s : sys) {
+            if (snap_len > 0x7fffffffull) fail("too many atoms in one batch");
+            snap_at.push_back((int)snap_len);
+            snap_len += 6 * (size_t)s.prog->T.n_atom;
+            n_pot = std::max(n_pot, s.prog->T.n_pot);
+        }
+        hip_check(hipMalloc((void**)&d_snap, std::max(snap_len, (size_t)4) * sizeof(float)), "snapshot");
+        status_stride = STATUS_WORDS + n_pot;
+        hip_check(hipHostMalloc((void**)&status, sys.size() * status_stride * sizeof(int), hipHostMallocDefault), "status");
         desc.clear();
         for (size_t k = 0; k < sys.size(); ++k) desc.push_back(make_desc((int)k));
         hip_check(hipMalloc((void**)&d_desc, desc.size() * sizeof(SysDesc)), "descriptors");
@@ -2084,17 +2116,12 @@ struct Batch {
         hip_check(hipMemcpy(desc.data(), d_desc, desc.size() * sizeof(SysDesc), hipMemcpyDeviceToHost), "descriptors");
     }
 
-    bool overflowed() {
-        bool of = false;
-        for (auto& s : sys) {
-            const Topology& T = s.prog->T;
-            for (auto& G : T.graphs) {
-                int st[4];
-                hip_check(hipMemcpy(st, s.iarena + G.state, sizeof(st), hipMemcpyDeviceToHost), "graph state");
-                if (st[1]) of = true;
-            }
-        }
-        return of;
+    // What the last launch left in pinned host memory (status_kernel).
+    const int* status_of(size_t s) const { return status + s * status_stride; }
+    bool overflowed() const {
+        for (size_t s = 0; s < sys.size(); ++s)
+            if (status_of(s)[0]) return true;
+        return false;
     }
 
     // Re-lower every program with larger list capacities, keeping positions,
@@ -2290,7 +2317,10 @@ struct Batch {
         }
     }
 
-    void launch(const RunArgs& a0) {
+    // Run the engine kernel and wait for it; the status records are then
+    // current.  deriv: pinned memory that receives the derivative of a
+    // one-system engine.
+    void launch(const RunArgs& a0, float* deriv = nullptr) {
         RunArgs a = a0;
         a.team = team;
         a.lane_split = lane_split;
@@ -2304,23 +2334,25 @@ struct Batch {
         a.bp_budget = bp_budget;
         a.bp_klocal = bp_klocal;
         if (mlp) a.mlp = mlp->dev;
+        pots_fresh = false;
         hip_check(hipEventRecord(ev0, stream), "event");
         hip_check(upside_launch_engine(d_desc, (int)sys.size(), a, stream), "engine launch");
         hip_check(hipEventRecord(ev1, stream), "event");
+        hip_check(upside_launch_status(d_desc, (int)sys.size(), status, status_stride, deriv, stream), "status launch");
         hip_check(hipStreamSynchronize(stream), "engine run");
         (void)hipEventElapsedTime(&last_ms, ev0, ev1);
+        for (size_t s = 0; s < sys.size(); ++s)
+            desc[s].n_invocations = (uint64_t)(uint32_t)status_of(s)[2] | ((uint64_t)(uint32_t)status_of(s)[3] << 32);
         if (team > 1) team_local = true;
         if (team > 1)
             for (size_t s = 0; s < sys.size(); ++s) {
-                const System& sy = sys[s];
                 if (team_of(s) < 2) continue;
-                unsigned w[BAR_WORDS];
-                hip_check(hipMemcpy(w, sy.iarena + sy.prog->T.bar, sizeof(w), hipMemcpyDeviceToHost), "barrier");
+                const unsigned* w = (const unsigned*)status_of(s) + STATUS_TEAM;
                 auto word64 = [&](int k) { return (unsigned long long)w[k] | ((unsigned long long)w[k + 1] << 32); };
                 const unsigned long long g = (unsigned long long)team_of(s), lo = g / 2, hi = g - g / 2;
-                if (w[2]) fail("team barrier wait timed out: results of this run are void");
+                if (w[2]) throw BarrierTimeout("team barrier wait timed out: results of this run are void");
                 bool quarters_ok = true;
-                if (sy.prog->n_lanes == 4 && g >= 8)
+                if (sys[s].prog->n_lanes == 4 && g >= 8)
                     for (unsigned long long j = 0; j < 4; ++j)
                         quarters_ok = quarters_ok && word64(BAR_Q + 2 * (int)j) % ((j + 1) * g / 4 - j * g / 4) == 0;
                 if (word64(0) % g || (g > 2 && word64(BAR_SUB1) % (g - 1)) || (g >= 4 && word64(BAR_LO) % lo) ||
@@ -2328,32 +2360,36 @@ struct Batch {
                     fail("team barrier arrivals unbalanced at the end of a launch: results of this run are void");
                 team_local = team_local && w[3] != 0;
             }
+        pots_fresh = a.n_round == 0 && a.mode == 1;
     }
 
     // Evaluate potential and derivative of every system at its positions.
-    void evaluate(int mode) {
+    void evaluate(int mode, float* deriv = nullptr) {
         RunArgs a;
         std::memset(&a, 0, sizeof(a));
         a.mode = mode;
         for (;;) {  // grow() fails once a capacity reaches its limit
-            launch(a);
+            launch(a, deriv);
             if (!overflowed()) break;
             grow();
         }
     }
 
+    // The one-system engine: evaluate at pos (through pinned memory, so that
+    // the call waits for the GPU once) and give back the derivative (null: not).
+    void evaluate_at(const float* pos, float* deriv) {
+        const size_t n = 3 * (size_t)sys[0].prog->T.n_atom;
+        if (!stage) hip_check(hipHostMalloc((void**)&stage, 2 * n * sizeof(float), hipHostMallocDefault), "staging");
+        std::memcpy(stage, pos, n * sizeof(float));
+        hip_check(upside_launch_positions(d_desc, stage, stream), "pos");
+        evaluate(1, deriv ? stage + n : nullptr);
+        if (deriv) std::memcpy(deriv, stage + n, n * sizeof(float));
+    }
+
     void run(int n_round, int frame_interval, float* frame_pot, int n_frames, int first_round) {
         // snapshot for a retry after list overflow
-        vector<vector<float>> pos(sys.size()), mom(sys.size());
-        pull_desc();
+        hip_check(upside_launch_snapshot(d_desc, (int)sys.size(), d_snap, 0, stream), "snapshot");
         vector<SysDesc> saved = desc;
-        for (size_t k = 0; k < sys.size(); ++k) {
-            const Topology& T = sys[k].prog->T;
-            pos[k].resize(T.n_atom * 3);
-            mom[k].resize(T.n_atom * 3);
-            hip_check(hipMemcpy(pos[k].data(), sys[k].arena + T.nodes[0].out, pos[k].size() * 4, hipMemcpyDeviceToHost), "pos");
-            hip_check(hipMemcpy(mom[k].data(), sys[k].arena + T.mom, mom[k].size() * 4, hipMemcpyDeviceToHost), "mom");
-        }
         float* d_frames = nullptr;
         if (frame_pot && n_frames > 0)
             hip_check(hipMalloc((void**)&d_frames, sys.size() * n_frames * sizeof(float)), "frames");
@@ -2387,19 +2423,14 @@ struct Batch {
             }
             if (!overflowed()) break;
             grow();
-            for (size_t k = 0; k < sys.size(); ++k) {
-                const Topology& T = sys[k].prog->T;
-                hip_check(hipMemcpy(sys[k].arena + T.nodes[0].out, pos[k].data(), pos[k].size() * 4, hipMemcpyHostToDevice), "pos");
-                hip_check(hipMemcpy(sys[k].arena + T.mom, mom[k].data(), mom[k].size() * 4, hipMemcpyHostToDevice), "mom");
-                desc[k].n_invocations = saved[k].n_invocations;
-            }
+            for (size_t k = 0; k < sys.size(); ++k) desc[k].n_invocations = saved[k].n_invocations;
             push_desc();
+            hip_check(upside_launch_snapshot(d_desc, (int)sys.size(), d_snap, 1, stream), "snapshot");
         }
         if (d_frames) {
             hip_check(hipMemcpy(frame_pot, d_frames, sys.size() * n_frames * sizeof(float), hipMemcpyDeviceToHost), "frames");
             (void)hipFree(d_frames);
         }
-        pull_desc();
     }
 
     // Checkpoint of the whole device state: a header, then per system its
@@ -2553,7 +2584,8 @@ struct Batch {
     float potential(int k) {
         const Topology& T = sys[k].prog->T;
         vector<float> p(std::max(T.n_pot, 1));
-        hip_check(hipMemcpy(p.data(), sys[k].arena + T.pot, p.size() * 4, hipMemcpyDeviceToHost), "potential");
+        if (pots_fresh) std::memcpy(p.data(), status_of(k) + STATUS_WORDS, T.n_pot * sizeof(float));
+        else hip_check(hipMemcpy(p.data(), sys[k].arena + T.pot, p.size() * 4, hipMemcpyDeviceToHost), "potential");
         float e = 0.f;
         for (int i = 0; i < T.n_pot; ++i) e += p[i];
         return e;
@@ -2589,6 +2621,11 @@ using namespace upside;
 struct DerivEngine {
     Batch batch;
     bool evaluated = false;   // an evaluation has set every node's outputs and sensitivities
+
+    void evaluate(const float* pos, float* deriv) {
+        batch.evaluate_at(pos, deriv);
+        evaluated = true;
+    }
 };
 // /output logger of one system: the basic-level datasets of the reference's
 // simulation loop (src/main.cpp:807-831 pos, mom, kinetic, potential, time;
@@ -3090,9 +3127,7 @@ void free_deriv_engine(DerivEngine* engine) { delete engine; }
 
 int evaluate_energy(float* energy, DerivEngine* engine, const float* pos) {
     ABI_TRY
-    engine->batch.copy_pos_in(0, pos);
-    engine->batch.evaluate(1);
-    engine->evaluated = true;
+    engine->evaluate(pos, nullptr);
     *energy = engine->batch.potential(0);
     return 0;
     ABI_CATCH(1)
@@ -3100,12 +3135,7 @@ int evaluate_energy(float* energy, DerivEngine* engine, const float* pos) {
 
 int evaluate_deriv(float* deriv, DerivEngine* engine, const float* pos) {
     ABI_TRY
-    auto& B = engine->batch;
-    B.copy_pos_in(0, pos);
-    B.evaluate(1);
-    engine->evaluated = true;
-    const Topology& T = B.sys[0].prog->T;
-    hip_check(hipMemcpy(deriv, B.sys[0].arena + T.nodes[0].sens, T.n_atom * 3 * sizeof(float), hipMemcpyDeviceToHost), "deriv");
+    engine->evaluate(pos, deriv);
     return 0;
     ABI_CATCH(1)
 }

@@ -1548,6 +1548,48 @@ __global__ void __launch_bounds__(NT) engine_eval_kernel(SysDesc* systems, RunAr
     engine_body(systems, (lp<float>)red, (lp<int>)ired, (lp<int>)ctx, (lp<float>)lds);
 }
 
+// ---- around a launch --------------------------------------------------------------
+// One workgroup per system gathers what the host reads after a launch into
+// pinned host memory, and with deriv != null (one system) the derivative: one
+// small kernel and one synchronisation instead of a copy per pair graph, team
+// and array (about 10 us each).
+__global__ void __launch_bounds__(NT) status_kernel(const SysDesc* systems, int* out, int stride, float* deriv) {
+    const SysDesc& S = systems[blockIdx.x];
+    int* w = out + (size_t)blockIdx.x * stride;
+    int over = 0;
+    for (int g = threadIdx.x; g < S.n_graph; g += NT) over |= S.iarena[S.graphs[g].state + 1] != 0;
+    over = __syncthreads_or(over);
+    if (threadIdx.x == 0) {
+        w[0] = over;
+        w[2] = (int)(uint32_t)S.n_invocations;
+        w[3] = (int)(uint32_t)(S.n_invocations >> 32);
+    }
+    for (int k = threadIdx.x; k < BAR_WORDS; k += NT) w[STATUS_TEAM + k] = S.iarena[S.bar + k];
+    for (int k = threadIdx.x; k < S.n_pot; k += NT) w[STATUS_WORDS + k] = __float_as_int(S.arena[S.pot + k]);
+    if (deriv)
+        for (int i = threadIdx.x; i < 3 * S.n_atom; i += NT) deriv[i] = S.arena[S.pos_sens + i];
+}
+
+// Positions and momenta of every system into the batch's snapshot buffer, or
+// back (a run that outgrew a list capacity is repeated from it); grid.y
+// workgroups share a system.
+__global__ void __launch_bounds__(NT) snapshot_kernel(const SysDesc* systems, float* snap, int restore) {
+    const SysDesc& S = systems[blockIdx.x];
+    float* b = snap + S.snap;
+    const int n = 3 * S.n_atom;
+    for (int i = blockIdx.y * NT + threadIdx.x; i < 2 * n; i += gridDim.y * NT) {
+        float* p = S.arena + (i < n ? S.pos_out + i : S.mom + i - n);
+        if (restore) *p = b[i];
+        else b[i] = *p;
+    }
+}
+
+// Positions from pinned host memory into the first system.
+__global__ void __launch_bounds__(NT) positions_kernel(const SysDesc* systems, const float* pos) {
+    const SysDesc& S = systems[0];
+    for (int i = blockIdx.x * NT + threadIdx.x; i < 3 * S.n_atom; i += gridDim.x * NT) S.arena[S.pos_out + i] = pos[i];
+}
+
 // ---- parameter derivatives of spline pair graphs ------------------------------
 // Weights of the four coefficients of a uniform cubic B-spline at x >= 1 and
 // the first coefficient they multiply: the derivative of the value with
@@ -1740,6 +1782,25 @@ __global__ void __launch_bounds__(NT) recenter_kernel(float* pos, int n_atom, in
 }
 
 }  // namespace upside
+
+hipError_t upside_launch_status(const upside::SysDesc* systems, int n_sys, int* out, int stride, float* deriv,
+                                hipStream_t stream) {
+    if (n_sys <= 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(upside::status_kernel, dim3(n_sys), dim3(upside::NT), 0, stream, systems, out, stride, deriv);
+    return hipGetLastError();
+}
+
+hipError_t upside_launch_snapshot(const upside::SysDesc* systems, int n_sys, float* snap, int restore,
+                                  hipStream_t stream) {
+    if (n_sys <= 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(upside::snapshot_kernel, dim3(n_sys, 4), dim3(upside::NT), 0, stream, systems, snap, restore);
+    return hipGetLastError();
+}
+
+hipError_t upside_launch_positions(const upside::SysDesc* systems, const float* pos, hipStream_t stream) {
+    hipLaunchKernelGGL(upside::positions_kernel, dim3(4), dim3(upside::NT), 0, stream, systems, pos);
+    return hipGetLastError();
+}
 
 hipError_t upside_launch_recenter(float* pos, int n_atom, int xy_only, hipStream_t stream) {
     if (n_atom <= 0) return hipErrorInvalidValue;
