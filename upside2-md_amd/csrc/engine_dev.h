@@ -104,18 +104,20 @@ struct ParamDerivArgs {
     const int* loc2;
     const int* type1;
     const int* type2;
+    int n1, n2;            // elements of the two sides
+    const int* off;        // rows: slots [off[i], off[i+1]) of side-1 element i
     const int* row;        // slot -> side-1 element
     const int* nbr;        // slot -> side-2 element
+    const int* toff;       // transposed rows: entries [toff[j], toff[j+1]) of side-2 element j
+    const int* tslot;      // transposed entry -> slot
     const int* act;        // slot refined in (edge present)
     const float* es;       // slot edge sensitivity
-    int n_slot;
     const float* param;    // (n_type1*n_type2, n_param)
     int n_type2, n_param, sym, kind;
     float* out;            // (n_type1*n_type2, n_param)
 };
 
-// Parameter derivative of a sigmoid coupling node after an evaluation
-// (one workgroup; one output entry per thread at a time).
+// Parameter derivative of a sigmoid coupling node after an evaluation.
 struct CouplingDerivArgs {
     int kind;              // OP_SIGMOID_COUPLING or OP_BB_SIGMOID_COUPLING
     int n_res, nt, n_indep;

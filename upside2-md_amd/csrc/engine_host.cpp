@@ -1883,6 +1883,20 @@ struct Batch {
     float* d_snap = nullptr;     // positions and momenta at the start of a run
     vector<int> snap_at;         // each system's offset there
     float* stage = nullptr;      // pinned positions and derivative of a one-system engine
+    float* param_out = nullptr;  // pinned: a parameter derivative
+    size_t param_cap = 0;
+    // Pinned memory for n floats of parameter derivatives (the kernels write
+    // there: no allocation and no copy per call).
+    float* param_out_for(size_t n) {
+        if (n > param_cap) {
+            (void)hipHostFree(param_out);
+            param_out = nullptr;
+            param_cap = 0;
+            hip_check(hipHostMalloc((void**)&param_out, n * sizeof(float), hipHostMallocDefault), "param deriv");
+            param_cap = n;
+        }
+        return param_out;
+    }
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     float last_ms = 0.f;
@@ -2003,6 +2017,7 @@ struct Batch {
         (void)hipFree(d_snap);
         (void)hipHostFree(status);
         (void)hipHostFree(stage);
+        (void)hipHostFree(param_out);
         if (ev0) (void)hipEventDestroy(ev0);
         if (ev1) (void)hipEventDestroy(ev1);
         if (stream) (void)hipStreamDestroy(stream);
@@ -3264,14 +3279,10 @@ int get_param_deriv(int n_param, float* deriv, DerivEngine* engine, const char* 
         }
         if (n_param != a.n_out)
             fail("Wrong number of parameters, expected " + std::to_string(a.n_out) + " but got " + std::to_string(n_param));
-        float* d_out = nullptr;
-        hip_check(hipMalloc((void**)&d_out, (size_t)a.n_out * sizeof(float)), "param deriv");
-        a.out = d_out;
-        hipError_t e = upside_launch_coupling_param_deriv(a, B.stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(B.stream);
-        if (e == hipSuccess) e = hipMemcpy(deriv, d_out, (size_t)a.n_out * sizeof(float), hipMemcpyDeviceToHost);
-        (void)hipFree(d_out);
-        hip_check(e, "param deriv");
+        a.out = B.param_out_for(a.n_out);
+        hip_check(upside_launch_coupling_param_deriv(a, B.stream), "param deriv");
+        hip_check(hipStreamSynchronize(B.stream), "param deriv");
+        std::memcpy(deriv, a.out, (size_t)a.n_out * sizeof(float));
         return 0;
     }
     for (size_t g = 0; g < T.graphs.size(); ++g) {
@@ -3307,26 +3318,24 @@ int get_param_deriv(int n_param, float* deriv, DerivEngine* engine, const char* 
         a.loc2 = P.d_ci + G.loc2;
         a.type1 = P.d_ci + G.type1;
         a.type2 = P.d_ci + G.type2;
+        a.n1 = G.n1;
+        a.n2 = G.n2;
+        a.off = s.iarena + G.off;
+        a.toff = s.iarena + G.toff;
+        a.tslot = s.iarena + G.tslot;
         a.row = s.iarena + G.row;
         a.nbr = s.iarena + G.nbr;
         a.act = s.iarena + G.act;
         a.es = s.arena + G.esens;
-        int st[4];
-        hip_check(hipMemcpy(st, s.iarena + G.state, sizeof(st), hipMemcpyDeviceToHost), "state");
-        a.n_slot = st[3];
         a.param = P.d_cf + G.param;
         a.n_type2 = G.n_type2;
         a.n_param = G.n_param;
         a.sym = G.sym;
         a.kind = G.kind;
-        float* d_out = nullptr;
-        hip_check(hipMalloc((void**)&d_out, (size_t)size * sizeof(float)), "param deriv");
-        a.out = d_out;
-        hipError_t e = upside_launch_param_deriv(a, rows, B.stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(B.stream);
-        if (e == hipSuccess) e = hipMemcpy(deriv, d_out, (size_t)size * sizeof(float), hipMemcpyDeviceToHost);
-        (void)hipFree(d_out);
-        hip_check(e, "param deriv");
+        a.out = B.param_out_for(size);
+        hip_check(upside_launch_param_deriv(a, rows, B.stream), "param deriv");
+        hip_check(hipStreamSynchronize(B.stream), "param deriv");
+        std::memcpy(deriv, a.out, (size_t)size * sizeof(float));
         return 0;
     }
     fail(string("get_param_deriv: no parameters exposed for node ") + node_name);

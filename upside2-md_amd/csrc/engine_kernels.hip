@@ -1649,43 +1649,68 @@ __device__ void quadspline_param_deriv(const float* p, const float* x1, const fl
     for (int i = 0; i < 4; ++i) acc[NKA + b + i] += scale * (a1 * nn * w[i]);
 }
 
-// One workgroup per interaction-table row t: every thread walks the slots in
-// a fixed stride, adds the derivative of each present edge whose type pair is
-// t (or, in a symmetric graph, whose transposed pair is t) into its own LDS
-// row, and the rows are summed in thread order, so the result is the same on
-// every run.  In a symmetric graph an edge is taken with its lower element
-// first, the orientation the reference's pair list gives it
-// (src/interaction_graph.h:134-145).
+// One workgroup per interaction-table row t = (ta, tb): the present edges with
+// side-1 type ta and side-2 type tb, found through the rows of the elements of
+// type ta (in a symmetric graph, whose rows hold the edge's lower element first
+// as the reference's pair list does, src/interaction_graph.h:134-145, also the
+// edges of types (tb, ta), through the transposed rows).  A wave tests 64
+// elements at a time and takes the slots of each hit with its 64 lanes; a lane
+// adds into its own LDS row, and the rows are summed in thread order, so the
+// result is the same on every run.  Bound by memory trips per slot step and
+// the summing of the rows.  A whole call for the rotamer table (20 x 20 pairs):
+// 82 us at 210 residues and 157 at 400; 102 and 209 when every type pair
+// scanned every slot of the graph.
 __global__ void __launch_bounds__(NT) param_deriv_kernel(ParamDerivArgs a) {
     extern __shared__ float lds[];
-    const int t = blockIdx.x;
     const int np = a.n_param;
-    float* acc = lds + threadIdx.x * np;
-    for (int d = 0; d < np; ++d) acc[d] = 0.f;
-    for (int s = threadIdx.x; s < a.n_slot; s += NT) {
-        if (!a.act[s]) continue;
-        int i = a.row[s], j = a.nbr[s];
-        if (a.sym && j < i) { int k = i; i = j; j = k; }
-        const int t1 = a.type1[i], t2 = a.type2[j];
-        const int m = (t1 * a.n_type2 + t2 == t) + (a.sym && t2 * a.n_type2 + t1 == t);
-        if (!m) continue;
-        const float* x1 = a.x1 + a.loc1[i] * a.w1;
-        const float* x2 = a.x2 + a.loc2[j] * a.w2;
-        const float* p = a.param + (t1 * a.n_type2 + t2) * np;
-        for (int k = 0; k < m; ++k) {
-            if (a.kind == EDGE_ROTAMER) {
-                quadspline_param_deriv<15, 12>(p, x1, x2, 6.f, 1.f / 0.7f, a.es[s], acc);
-            } else {  // hbond coverage: (1 - hb)^2 times the spline (src/hbond.cpp:286-291)
-                const float om = 1.f - x1[6];
-                quadspline_param_deriv<15, 10>(p, x1, x2, 6.f, 1.f / 0.625f, a.es[s] * (om * om), acc);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int ta = blockIdx.x / a.n_type2, tb = blockIdx.x % a.n_type2;
+    for (int d = tid; d < NT * np; d += NT) lds[d] = 0.f;
+    float* acc = lds + tid * np;
+    __syncthreads();
+    for (int pass = 0; pass < (a.sym ? 2 : 1); ++pass) {
+        const int n = pass ? a.n2 : a.n1;
+        const int* type = pass ? a.type2 : a.type1;
+        const int* off = pass ? a.toff : a.off;
+        const int* other_type = pass ? a.type1 : a.type2;
+        for (int base = wave * 64; base < n; base += NT) {
+            const int e = base + lane;
+            unsigned long long hits = __ballot(e < n && type[e] == ta);
+            while (hits) {
+                const int el = base + __builtin_ctzll(hits);
+                hits &= hits - 1;
+                const int k1 = off[el + 1];
+                for (int k = off[el] + lane; k < k1; k += 64) {
+                    const int s = pass ? a.tslot[k] : k;
+                    if (!a.act[s]) continue;
+                    const int i = pass ? a.row[s] : el, j = pass ? el : a.nbr[s];
+                    if (other_type[pass ? i : j] != tb) continue;
+                    const float* x1 = a.x1 + a.loc1[i] * a.w1;
+                    const float* x2 = a.x2 + a.loc2[j] * a.w2;
+                    const float* p = a.param + (pass ? tb * a.n_type2 + ta : ta * a.n_type2 + tb) * np;
+                    if (a.kind == EDGE_ROTAMER) {
+                        quadspline_param_deriv<15, 12>(p, x1, x2, 6.f, 1.f / 0.7f, a.es[s], acc);
+                    } else {  // hbond coverage: (1 - hb)^2 times the spline (src/hbond.cpp:286-291)
+                        const float om = 1.f - x1[6];
+                        quadspline_param_deriv<15, 10>(p, x1, x2, 6.f, 1.f / 0.625f, a.es[s] * (om * om), acc);
+                    }
+                }
             }
         }
     }
     __syncthreads();
-    for (int d = threadIdx.x; d < np; d += NT) {
+    // each wave's rows, then the waves in order (the sums go where rows of the
+    // wave itself were, once it has read them all)
+    for (int d = lane; d < np; d += 64) {
         float sum = 0.f;
-        for (int k = 0; k < NT; ++k) sum += lds[k * np + d];
-        a.out[t * np + d] = sum;
+        for (int k = 0; k < 64; ++k) sum += lds[(wave * 64 + k) * np + d];
+        lds[wave * 64 * np + d] = sum;  // entry d of the first row: read by this lane alone
+    }
+    __syncthreads();
+    for (int d = tid; d < np; d += NT) {
+        float sum = 0.f;
+        for (int w = 0; w < NWAVE; ++w) sum += lds[w * 64 * np + d];
+        a.out[blockIdx.x * np + d] = sum;
     }
 }
 
@@ -1695,72 +1720,112 @@ __global__ void __launch_bounds__(NT) param_deriv_kernel(ParamDerivArgs a) {
 // node has independent weights (400: per coupling type and amino acid; 20: per
 // amino acid, repeated).  Backbone sigmoid coupling
 // (BackboneSigmoidCoupling::get_param_deriv, :1118-1134): only d/dscale.
-// Each thread owns output entries and sums over residues in residue order.
+// Residues are spread over the threads and summed in a fixed order (sigmoid
+// coupling: COUPLING_OUT entries per workgroup, the residues' sigmoids in LDS,
+// COUPLING_PARTS threads per entry over contiguous ranges of residues).  A
+// thread per entry walking all residues from memory is bound by that chain: 382
+// us for the sigmoid coupling of 210 residues and 170 for the hydrogen-bond
+// energy, now 31 and 17.
+constexpr int COUPLING_OUT = 64, COUPLING_PARTS = NT / COUPLING_OUT, COUPLING_RES = 2048;
+
 __global__ void __launch_bounds__(NT) coupling_param_deriv_kernel(CouplingDerivArgs a) {
-    const int nt = a.nt;
-    for (int j = threadIdx.x; j < a.n_out; j += NT) {
+    __shared__ float red[NT * 4];
+    const int nt = a.nt, tid = threadIdx.x;
+    if (a.kind == OP_SIGMOID_COUPLING) {
+        __shared__ float rv[COUPLING_RES], rd[COUPLING_RES], rdc[COUPLING_RES];
+        __shared__ int rct[COUPLING_RES];
+        const int j = blockIdx.x * COUPLING_OUT + tid % COUPLING_OUT, part = tid / COUPLING_OUT;
+        const int cs = 3 * nt;
+        const int q = j < cs ? j / nt : 3;
+        const int want_ct = j < cs ? j % nt : (a.n_indep == 400 ? (j - cs) / nt : -1);
+        const int want_aa = j < cs ? -1 : (j - cs) % nt;
+        const bool live = j < a.n_out && (j < cs || a.n_indep > 1);
         float acc = 0.f;
-        if (a.kind == OP_HBOND_ENERGY) {
-            // HBondEnergy::get_param_deriv (src/hbond.cpp:655-720): [0..2] hbonds of
-            // each residue times its helix, sheet and turn scores, [3] the bias
-            // term of each peptide; the shape parameters [4..11] stay zero
-            const float* P = a.hp;
-            if (j < 3) {
-                for (int i = 0; i < a.n_res; ++i) {
-                    const float phi = a.rama[i * a.wr], psi = a.rama[i * a.wr + 1];
-                    float p1, d1, p2, d2, s1, e1, s2, e2;
-                    compact_sigmoid(phi - P[4], P[5], p1, d1);
-                    compact_sigmoid(phi - P[6], P[7], p2, d2);
-                    compact_sigmoid(psi - P[8], P[9], s1, e1);
-                    compact_sigmoid(psi - P[10], P[11], s2, e2);
-                    const float turn = (float)((1. - (double)p1) * p2);
-                    const float psis = (float)((1. - (double)s1) * s2);
-                    const float nturn = (float)(1. - (double)turn), npsi = (float)(1. - (double)psis);
-                    const float score = j == 0 ? nturn * psis : (j == 1 ? nturn * npsi : turn);
-                    float hb = 0.f;
-                    for (int k = a.h1o[i]; k < a.h1o[i + 1]; ++k) hb += a.pp[a.h1i[k] * a.wp + 6];
-                    acc += hb * score;
-                }
-            } else if (j == 3) {
-                for (int i = 0; i + 1 < a.n_res; ++i) {
-                    float hb = 0.f;
-                    for (int k = a.h2o[i]; k < a.h2o[i + 1]; ++k) hb += a.pp[a.h2i[k] * a.wp + 6];
-                    float v, d;
-                    compact_sigmoid(1.5f - hb, 2.0f, v, d);
-                    acc += v;
-                }
+        for (int r0 = 0; r0 < a.n_res; r0 += COUPLING_RES) {
+            const int n = min(COUPLING_RES, a.n_res - r0);
+            __syncthreads();  // the previous chunk has been read
+            for (int k = tid; k < n; k += NT) {
+                const int r = r0 + k, ct = a.ctype[r];
+                float w = 0.f;
+                for (int aa = 0; aa < nt; ++aa) w += a.weights[ct * nt + aa] * a.cov[r * nt + aa];
+                const float dc = w - a.center[ct];
+                float v, d;
+                compact_sigmoid(dc, a.sharp[ct], v, d);
+                rct[k] = ct;
+                rv[k] = v;
+                rd[k] = d;
+                rdc[k] = dc;
             }
-        } else if (a.kind == OP_BB_SIGMOID_COUPLING) {
-            if (j == 0)
-                for (int r = 0; r < a.n_res; ++r) {
-                    float bl = 0.f;
-                    for (int aa = 0; aa < nt; ++aa) bl += a.weights[aa] * a.cov[r * nt + aa];
-                    bl += a.bb_hbond_weight * a.cov_hb[r];
-                    float v, d;
-                    compact_sigmoid(bl - a.bb_center, a.bb_sharp, v, d);
-                    acc += v;
-                }
-        } else {
-            const int cs = 3 * nt;
-            const int q = j < cs ? j / nt : 3;
-            const int want_ct = j < cs ? j % nt : (a.n_indep == 400 ? (j - cs) / nt : -1);
-            const int want_aa = j < cs ? -1 : (j - cs) % nt;
-            if (j < cs || a.n_indep > 1)
-                for (int r = 0; r < a.n_res; ++r) {
-                    const int ct = a.ctype[r];
+            __syncthreads();
+            const int per = (n + COUPLING_PARTS - 1) / COUPLING_PARTS, e = min(n, (part + 1) * per);
+            if (live)
+                for (int k = part * per; k < e; ++k) {
+                    const int ct = rct[k];
                     if (want_ct >= 0 && ct != want_ct) continue;
-                    float w = 0.f;
-                    for (int aa = 0; aa < nt; ++aa) w += a.weights[ct * nt + aa] * a.cov[r * nt + aa];
-                    const float dc = w - a.center[ct];
-                    float v, d;
-                    compact_sigmoid(dc, a.sharp[ct], v, d);
-                    if (q == 0) acc += v;
-                    else if (q == 1) acc += -a.scale[ct] * d;
-                    else if (q == 2) acc += a.scale[ct] * dc * d / a.sharp[ct];
-                    else acc += (d * a.scale[ct]) * a.cov[r * nt + want_aa];
+                    if (q == 0) acc += rv[k];
+                    else if (q == 1) acc += -a.scale[ct] * rd[k];
+                    else if (q == 2) acc += a.scale[ct] * rdc[k] * rd[k] / a.sharp[ct];
+                    else acc += (rd[k] * a.scale[ct]) * a.cov[(r0 + k) * nt + want_aa];
                 }
         }
-        a.out[j] = acc;
+        red[tid] = acc;
+        __syncthreads();
+        if (part == 0 && j < a.n_out) {
+            float sum = 0.f;
+            for (int p = 0; p < COUPLING_PARTS; ++p) sum += red[p * COUPLING_OUT + tid];
+            a.out[j] = sum;
+        }
+        return;
+    }
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    if (a.kind == OP_HBOND_ENERGY) {
+        // HBondEnergy::get_param_deriv (src/hbond.cpp:655-720): [0..2] hbonds of
+        // each residue times its helix, sheet and turn scores, [3] the bias
+        // term of each peptide; the shape parameters [4..11] stay zero
+        const float* P = a.hp;
+        for (int i = tid; i < a.n_res; i += NT) {
+            const float phi = a.rama[i * a.wr], psi = a.rama[i * a.wr + 1];
+            float p1, d1, p2, d2, s1, e1, s2, e2;
+            compact_sigmoid(phi - P[4], P[5], p1, d1);
+            compact_sigmoid(phi - P[6], P[7], p2, d2);
+            compact_sigmoid(psi - P[8], P[9], s1, e1);
+            compact_sigmoid(psi - P[10], P[11], s2, e2);
+            const float turn = (float)((1. - (double)p1) * p2);
+            const float psis = (float)((1. - (double)s1) * s2);
+            const float nturn = (float)(1. - (double)turn), npsi = (float)(1. - (double)psis);
+            float hb = 0.f;
+            for (int k = a.h1o[i]; k < a.h1o[i + 1]; ++k) hb += a.pp[a.h1i[k] * a.wp + 6];
+            acc[0] += hb * (nturn * psis);
+            acc[1] += hb * (nturn * npsi);
+            acc[2] += hb * turn;
+            if (i + 1 < a.n_res) {
+                float hb2 = 0.f;
+                for (int k = a.h2o[i]; k < a.h2o[i + 1]; ++k) hb2 += a.pp[a.h2i[k] * a.wp + 6];
+                float v, d;
+                compact_sigmoid(1.5f - hb2, 2.0f, v, d);
+                acc[3] += v;
+            }
+        }
+    } else {
+        for (int r = tid; r < a.n_res; r += NT) {
+            float bl = 0.f;
+            for (int aa = 0; aa < nt; ++aa) bl += a.weights[aa] * a.cov[r * nt + aa];
+            bl += a.bb_hbond_weight * a.cov_hb[r];
+            float v, d;
+            compact_sigmoid(bl - a.bb_center, a.bb_sharp, v, d);
+            acc[0] += v;
+        }
+    }
+    for (int q = 0; q < 4; ++q) {
+        const float w = wave_sum(acc[q]);
+        if ((tid & 63) == 0) red[q * NWAVE + (tid >> 6)] = w;
+    }
+    __syncthreads();
+    if (tid < a.n_out) {
+        float sum = 0.f;
+        if (tid < 4)
+            for (int w = 0; w < NWAVE; ++w) sum += red[tid * NWAVE + w];
+        a.out[tid] = sum;
     }
 }
 
@@ -1812,7 +1877,10 @@ hipError_t upside_launch_coupling_param_deriv(const upside::CouplingDerivArgs& a
     if (args.n_out <= 0 || args.nt <= 0) return hipErrorInvalidValue;
     upside::CouplingDerivArgs a = args;
     void* kargs[] = {&a};
-    return hipLaunchKernel((const void*)upside::coupling_param_deriv_kernel, dim3(1), dim3(upside::NT), kargs, 0,
+    const int wgs = args.kind == upside::OP_SIGMOID_COUPLING
+                        ? (args.n_out + upside::COUPLING_OUT - 1) / upside::COUPLING_OUT : 1;
+    if (wgs == 1 && args.n_out > upside::NT) return hipErrorInvalidValue;
+    return hipLaunchKernel((const void*)upside::coupling_param_deriv_kernel, dim3(wgs), dim3(upside::NT), kargs, 0,
                            stream);
 }
 
