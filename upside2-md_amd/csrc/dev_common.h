@@ -30,6 +30,78 @@ using GraphC = UPS_CONST const PairGraph;
 using RotC = UPS_CONST const RotamerDev;
 using SysC = UPS_CONST const SysDesc;
 
+// Arena pointers.  What one workgroup of a team writes to the system's arenas,
+// the others read after the next team barrier.  Every load from an arena goes
+// past the CU's L1 to the L2 of its XCD (buffer loads with sc1, agent scope:
+// 90 ns against 52 for an L1 hit and the same as an L1 miss, measured by a
+// pointer chase), so a barrier does not have to invalidate L1 (see team_sync).
+// A pointer is a buffer resource that starts at its array (so that only one
+// array, not an arena, has to be smaller than 4 GB; as fast as one resource an
+// arena with a scalar offset) and a lane's offset.
+constexpr int AUX_SC1 = 16;                   // cache policy bits of a buffer access
+constexpr int RSRC_FLAGS = 0x00027000;        // raw buffer of 32-bit data
+template <class T> struct Unconst { using type = T; };
+template <class T> struct Unconst<const T> { using type = T; };
+template <class T> struct ap {
+    using V = typename Unconst<T>::type;
+    gp<V> p;
+    __amdgpu_buffer_rsrc_t r;
+    int o;
+    __device__ __forceinline__ V load() const {
+        return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b32(r, o * 4, 0, AUX_SC1));
+    }
+    struct Ref {
+        ap a;
+        __device__ __forceinline__ operator V() const { return a.load(); }
+        __device__ __forceinline__ V operator=(V v) const { *a.ptr() = v; return v; }
+        __device__ __forceinline__ V operator=(const Ref& b) const { return *this = (V)b; }
+        __device__ __forceinline__ V operator+=(V v) const { return *this = a.load() + v; }
+    };
+    // for atomics and stores
+    __device__ __forceinline__ gp<V> ptr() const { return p + o; }
+    __device__ __forceinline__ ap operator+(int k) const { ap q = *this; q.o += k; return q; }
+    __device__ __forceinline__ Ref operator[](int k) const { return Ref{*this + k}; }
+    __device__ __forceinline__ operator ap<const V>() const { return ap<const V>{p, r, o}; }
+    // N consecutive elements, and added to.  (A load is not moved across a store
+    // to an arena, so elements are loaded together before any is stored.)
+    template <int N> __device__ __forceinline__ void get(V* v) const {
+#pragma unroll
+        for (int k = 0; k < N; ++k) v[k] = (*this + k).load();
+    }
+    template <int N> __device__ __forceinline__ void add(const V* v) const {
+        V x[N];
+        get<N>(x);
+#pragma unroll
+        for (int k = 0; k < N; ++k) (*this)[k] = x[k] + v[k];
+    }
+};
+// Read only: an element is its value.
+template <class T> struct ap<const T> {
+    gp<T> p;
+    __amdgpu_buffer_rsrc_t r;
+    int o;
+    __device__ __forceinline__ ap operator+(int k) const { ap q = *this; q.o += k; return q; }
+    __device__ __forceinline__ T operator[](int k) const {
+        return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, (o + k) * 4, 0, AUX_SC1));
+    }
+    template <int N> __device__ __forceinline__ void get(T* v) const {
+#pragma unroll
+        for (int k = 0; k < N; ++k) v[k] = (*this)[k];
+    }
+};
+// A whole arena; offsets added to it are uniform.
+template <class T> struct Arena {
+    gp<T> p;
+    __device__ __forceinline__ ap<T> operator+(int k) const {
+        return ap<T>{p + k, __builtin_amdgcn_make_buffer_rsrc((T*)(p + k), 0, -1, RSRC_FLAGS), 0};
+    }
+    __device__ __forceinline__ typename ap<T>::Ref operator[](int k) const { return (*this + k)[0]; }
+    // Data at k that nobody writes while it is read, through L1: only after
+    // l1_drop.  For records of a few cache lines read piece by piece (an edge's
+    // matrix): past L1 every 16-byte piece is a request to L2 of its own.
+    __device__ __forceinline__ gp<const T> cached(int k) const { return p + k; }
+};
+
 // A value every lane holds alike, as a scalar.
 __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
 __device__ __forceinline__ float unif(float v) { return __int_as_float(uni(__float_as_int(v))); }
@@ -62,8 +134,8 @@ struct Team {
 // Measured with the program records in scalar registers, ms per step: 0.55 ->
 // 0.47 for 67 residues on 8 workgroups, 1.03 -> 0.95 for 500 on 32.)
 struct Ctx : Team {
-    gp<float> A;           // per-system float arena
-    gp<int> I;             // per-system int arena
+    Arena<float> A;        // per-system float arena
+    Arena<int> I;          // per-system int arena
     gp<const float> CF;    // constant float arena
     gp<const int> CI;      // constant int arena
     cp<SysDesc> S;         // the system
@@ -137,10 +209,11 @@ __device__ __forceinline__ void pacc(const Ctx& c, int slot, unsigned long long 
 //   Memory ordering: a team spread over XCDs (separate L2s) needs
 // device-scope fences (write back L2 before arriving, invalidate after the
 // wait).  A team on one XCD shares its L2: every wave waits for its stores to
-// be acknowledged by L2 before the workgroup barrier (no L2 write-back), and
-// after the wait a device-scope invalidate drops the CU's L1.  (A
-// workgroup-scope invalidate does not reach L1 outside thread-group-split
-// mode.)
+// be acknowledged by L2 before the workgroup barrier, and loads of what others
+// wrote go to L2 (ap).  Nothing is invalidated: a device-scope invalidate of L1
+// after the wait, with plain loads, is served by the shared L2 one CU after
+// the other (a barrier of 2, 8, 16, 32 workgroups and reads of three others'
+// data: 1.07, 1.38, 1.82, 2.92 us with it; 0.95, 0.92, 0.93, 1.12 without).
 //   The wait is bounded: after ~1 s of spinning the workgroup records a
 // timeout and proceeds, so a launch always drains; the host then reports the
 // run as failed.
@@ -179,15 +252,23 @@ __device__ __forceinline__ void team_sync(Ctx& c) {
                     break;
                 }
             }
-            if (c.local) asm volatile("buffer_inv sc1" ::: "memory");  // L1 (no L2 write-back)
-            else __threadfence();
+            if (!c.local) __threadfence();
         }
         __syncthreads();
+        asm volatile("" ::: "memory");  // no load of an arena is moved up or reused across
         // profiling: team barriers per op, after the fixed slots
         if (c.prof && c.tid == 0)
             __hip_atomic_fetch_add(c.prof + c.pbase + PROF_EXTRA + c.cur_op, 1ull, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
     }
+}
+
+// Drop the CU's L1, which may hold lines of the arenas from before other
+// workgroups wrote them, ahead of cached reads.  All threads of the workgroup.
+__device__ __forceinline__ void l1_drop(Ctx& c) {
+    if (c.G == 1) return;  // nobody else writes this system's arenas
+    if (c.tid == 0) asm volatile("buffer_inv sc1" ::: "memory");
+    __syncthreads();
 }
 
 // Sub-teams: parts of a team that run beside each other, each with an arrival
@@ -291,12 +372,13 @@ __device__ __forceinline__ float block_max(Ctx& c, float v) {
 // memory trip and combined from registers; a loop over them in memory pays a
 // trip per unrolled group of ranks.
 static_assert(MAX_TEAM <= 64, "one lane per rank");
-__device__ __forceinline__ gp<float> team_partials(Ctx& c, float t) {
+// The partial of rank min(lane, G - 1), after all ranks have stored theirs.
+__device__ __forceinline__ float team_partial(Ctx& c, float t) {
     gp<float> buf = c.tred + c.tpar * c.G;
     c.tpar ^= 1;
     if (c.tid == 0) buf[c.rank] = t;
     team_sync(c);
-    return buf;
+    return __hip_atomic_load(buf + min(c.tid & 63, c.G - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ float lane_value(float v, int lane) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
@@ -304,8 +386,7 @@ __device__ __forceinline__ float lane_value(float v, int lane) {
 __device__ __forceinline__ float team_sum(Ctx& c, float v) {
     float t = block_sum(c, v);
     if (c.G == 1) return t;
-    gp<float> buf = team_partials(c, t);
-    const float x = buf[min(c.tid & 63, c.G - 1)];
+    const float x = team_partial(c, t);
     float s = 0.f;
     for (int r = 0; r < c.G; ++r) s += lane_value(x, r);
     return unif(s);
@@ -313,14 +394,12 @@ __device__ __forceinline__ float team_sum(Ctx& c, float v) {
 __device__ __forceinline__ float team_max(Ctx& c, float v) {
     float t = block_max(c, v);
     if (c.G == 1) return t;
-    gp<float> buf = team_partials(c, t);
-    return unif(wave_max(buf[min(c.tid & 63, c.G - 1)]));
+    return unif(wave_max(team_partial(c, t)));
 }
 __device__ __forceinline__ int team_or(Ctx& c, int v) {
     int t = uni(__syncthreads_or(v));
     if (c.G == 1) return t;
-    gp<float> buf = team_partials(c, t ? 1.f : 0.f);
-    return __any(buf[min(c.tid & 63, c.G - 1)] > 0.f) ? 1 : 0;
+    return __any(team_partial(c, t ? 1.f : 0.f) > 0.f) ? 1 : 0;
 }
 
 // In-place exclusive scan of the ints a[0..n) (any memory); returns the
@@ -366,9 +445,9 @@ __device__ __forceinline__ int team_exscan(Ctx& c, P a, int n) {
     int b = min(c.rank * per, n), e = min(b + per, n);
     int tot = uni(block_exscan(c, a + b, e - b));
     if (c.G == 1) return tot;
-    gp<float> buf = team_partials(c, __int_as_float(tot));
     const int lane = c.tid & 63;
-    const int x = lane < c.G ? __float_as_int(buf[lane]) : 0;
+    const int part = __float_as_int(team_partial(c, __int_as_float(tot)));
+    const int x = lane < c.G ? part : 0;
     int v = x;  // inclusive scan over the ranks
     for (int o = 1; o < 64; o <<= 1) {
         const int t = __shfl_up(v, o, 64);
@@ -474,8 +553,8 @@ __device__ __forceinline__ void quat_to_rot(P q, float* U) {
 // plan order, as one component at a time would).  Called by all threads of
 // the team; no barrier at the end.
 template <int CW>
-__device__ __forceinline__ void plan_gather_w(Ctx& c, gp<const int> off, gp<const int> idx, gp<float> sens,
-                                              gp<const float> con, int nt, int ss, int col, int cs) {
+__device__ __forceinline__ void plan_gather_w(Ctx& c, gp<const int> off, gp<const int> idx, ap<float> sens,
+                                              ap<const float> con, int nt, int ss, int col, int cs) {
     for (int t = c.gtid; t < nt; t += c.gsize) {
         const int b = off[t], e = off[t + 1];
         if (b == e) continue;
@@ -484,12 +563,11 @@ __device__ __forceinline__ void plan_gather_w(Ctx& c, gp<const int> off, gp<cons
         for (int k = 0; k < CW; ++k) acc[k] = 0.f;
 #pragma unroll 2
         for (int j = b; j < e; ++j) {
-            gp<const float> q = con + idx[j] * cs;
+            ap<const float> q = con + idx[j] * cs;
 #pragma unroll
             for (int k = 0; k < CW; ++k) acc[k] += q[k];
         }
-#pragma unroll
-        for (int k = 0; k < CW; ++k) sens[t * ss + col + k] += acc[k];
+        (sens + (t * ss + col)).template add<CW>(acc);
     }
 }
 
@@ -498,8 +576,8 @@ __device__ __forceinline__ void plan_gather(Ctx& c, int plan) {
     int nt = h[0], cw = h[1], so = h[2], ss = h[3], col = h[4], cb = h[5], cs = h[6];
     gp<const int> off = c.CI + plan + PLAN_HDR;
     gp<const int> idx = off + nt + 1;
-    gp<float> sens = c.A + so;
-    gp<const float> con = c.A + cb;
+    ap<float> sens = c.A + so;
+    ap<const float> con = c.A + cb;
     switch (cw) {
     case 1: plan_gather_w<1>(c, off, idx, sens, con, nt, ss, col, cs); break;
     case 2: plan_gather_w<2>(c, off, idx, sens, con, nt, ss, col, cs); break;

@@ -32,7 +32,7 @@ __device__ __forceinline__ bool pg_accept(GraphC& G, int a, int b) {
     return d > G.excl || -d > G.excl;
 }
 
-__device__ __forceinline__ gp<const float> pg_side2(const Ctx& c, GraphC& G) {
+__device__ __forceinline__ ap<const float> pg_side2(const Ctx& c, GraphC& G) {
     return c.A + G.pos_pack + (G.sym ? 0 : G.n1 * 3);
 }
 
@@ -41,18 +41,19 @@ __device__ __forceinline__ gp<const float> pg_side2(const Ctx& c, GraphC& G) {
 __device__ __forceinline__ bool pg_pack_and_check(Ctx& c, GraphC& G) {
     gp<const int> loc1 = c.CI + G.loc1;
     gp<const int> loc2 = c.CI + G.loc2;
-    gp<const float> P1 = c.A + G.out1;
-    gp<const float> P2 = c.A + G.out2;
-    gp<float> pack = c.A + G.pos_pack;
-    gp<const float> cache = c.A + G.cache_pos;
+    ap<const float> P1 = c.A + G.out1;
+    ap<const float> P2 = c.A + G.out2;
+    ap<float> pack = c.A + G.pos_pack;
+    ap<const float> cache = c.A + G.cache_pos;
     int n = G.sym ? G.n1 : G.n1 + G.n2;
     int valid = c.I[G.state];
     int moved = 0;
     for (int i = c.gtid; i < n; i += c.gsize) {
-        gp<const float> src = (i < G.n1) ? P1 + loc1[i] * G.w1 : P2 + loc2[i - G.n1] * G.w2;
-        float x = src[0], y = src[1], z = src[2];
+        ap<const float> src = (i < G.n1) ? P1 + loc1[i] * G.w1 : P2 + loc2[i - G.n1] * G.w2;
+        float x = src[0], y = src[1], z = src[2], old[3];
+        (cache + i * 3).get<3>(old);
         pack[i * 3 + 0] = x; pack[i * 3 + 1] = y; pack[i * 3 + 2] = z;
-        float dx = x - cache[i * 3 + 0], dy = y - cache[i * 3 + 1], dz = z - cache[i * 3 + 2];
+        float dx = x - old[0], dy = y - old[1], dz = z - old[2];
         if (!(dx * dx + dy * dy + dz * dz <= G.drift2)) moved = 1;  // NaN also forces a rebuild
     }
     int any = team_or(c, moved | (valid ? 0 : 1));
@@ -94,8 +95,8 @@ __device__ __forceinline__ GroupLanes group_lanes(const Ctx& c) {
 // cur + (hits of the lower lanes), so hits keep candidate order.  Every lane of
 // the group calls it.
 template <bool FILL>
-__device__ __forceinline__ int group_emit(const GroupLanes& L, bool hit, int cur, int q, int j, gp<int> nbr,
-                                         gp<int> row) {
+__device__ __forceinline__ int group_emit(const GroupLanes& L, bool hit, int cur, int q, int j, ap<int> nbr,
+                                         ap<int> row) {
     unsigned long long m = __ballot(hit) & L.gmask;
     if (FILL && hit) {
         int p = cur + __popcll(m & L.below);
@@ -116,7 +117,7 @@ __device__ __forceinline__ void el_put(lp<float> el, int k, float x, float y, fl
 }
 
 // Stage elements [t0, t0+n) of side pts (ids in id) as (x, y, z, id).
-__device__ __forceinline__ void stage_tile(Ctx& c, gp<const float> pts, gp<const int> id, int t0, int n) {
+__device__ __forceinline__ void stage_tile(Ctx& c, ap<const float> pts, gp<const int> id, int t0, int n) {
     lp<float> tile = c.lds;
     for (int k = c.tid; k < n; k += NT) {  // every workgroup stages its own copy
         int j = t0 + k;
@@ -130,9 +131,9 @@ __device__ __forceinline__ void stage_tile(Ctx& c, gp<const float> pts, gp<const
 // acceptable (SYM: also j > q).  !FILL adds row q's hits to off[q].  FILL
 // writes them at the cursor cur[q] (advanced).
 template <bool SYM, bool FILL>
-__device__ __forceinline__ void tile_rows(Ctx& c, GraphC& G, gp<const float> qp, gp<const int> qid, int nq,
-                          gp<const float> ep, gp<const int> eid, int ne, gp<int> off, gp<int> cur_arr, gp<int> nbr,
-                          gp<int> row) {
+__device__ __forceinline__ void tile_rows(Ctx& c, GraphC& G, ap<const float> qp, gp<const int> qid, int nq,
+                          ap<const float> ep, gp<const int> eid, int ne, ap<int> off, ap<int> cur_arr, ap<int> nbr,
+                          ap<int> row) {
     lp<const float> tile = (lp<const float>)c.lds;
     const float cc2 = G.cache_cut2;
     const GroupLanes L = group_lanes(c);
@@ -199,7 +200,7 @@ __device__ __forceinline__ bool lgrid_fits(int m) {
 
 // Build the grid of the m points pts (stride 3) in this workgroup's LDS
 // (every workgroup of a team builds its own copy).  All threads of the workgroup.
-__device__ __forceinline__ LGrid lgrid_build(Ctx& c, GraphC& G, gp<const float> pts, gp<const int> ids, int m) {
+__device__ __forceinline__ LGrid lgrid_build(Ctx& c, GraphC& G, ap<const float> pts, gp<const int> ids, int m) {
     float mn0 = 3.0e38f, mn1 = 3.0e38f, mn2 = 3.0e38f;
     for (int i = c.tid; i < m; i += NT) {
         mn0 = fminf(mn0, pts[i * 3]);
@@ -261,8 +262,8 @@ __device__ __forceinline__ LGrid lgrid_build(Ctx& c, GraphC& G, gp<const float> 
 // Rows against the grid; same hit rule as tile_rows.  !FILL: off[q] = hits of
 // row q.  FILL: row q's hits are written from off[q] on.
 template <bool SYM, bool FILL>
-__device__ __forceinline__ void grid_rows(Ctx& c, GraphC& G, const LGrid& g, gp<const float> qp, gp<const int> qid, int nq,
-                          gp<int> off, gp<int> nbr, gp<int> row) {
+__device__ __forceinline__ void grid_rows(Ctx& c, GraphC& G, const LGrid& g, ap<const float> qp, gp<const int> qid, int nq,
+                          ap<int> off, ap<int> nbr, ap<int> row) {
     const float cc2 = G.cache_cut2;
     const GroupLanes L = group_lanes(c);
     const int grp = c.gtid / SG, ngrp = c.gsize / SG;
@@ -303,10 +304,10 @@ __device__ __forceinline__ void grid_rows(Ctx& c, GraphC& G, const LGrid& g, gp<
 // among the team's workgroups; each workgroup stages runs of whole columns in
 // LDS.  All threads of the team.
 __device__ __forceinline__ void pg_order_columns(Ctx& c, GraphC& G, int n2) {
-    gp<const int> toff = c.I + G.toff;
-    gp<const int> tmp = c.I + G.tmp;
-    gp<const int> nbr = c.I + G.nbr;
-    gp<int> tslot = c.I + G.tslot;
+    ap<const int> toff = c.I + G.toff;
+    ap<const int> tmp = c.I + G.tmp;
+    ap<const int> nbr = c.I + G.nbr;
+    ap<int> tslot = c.I + G.tslot;
     lp<int> sl = (lp<int>)c.lds;
     const int CAP = LDS_FLOATS;
     int per = (n2 + c.G - 1) / c.G;
@@ -358,17 +359,17 @@ __device__ __forceinline__ bool pg_rebuild(Ctx& c, GraphC& G) {
     gp<const int> id1 = c.CI + G.id1;
     const bool sym = G.sym != 0;
     gp<const int> id2 = sym ? id1 : c.CI + G.id2;
-    gp<const float> pack = c.A + G.pos_pack;
-    gp<float> cache = c.A + G.cache_pos;
-    gp<const float> p1 = pack;
-    gp<const float> p2 = pg_side2(c, G);
+    ap<const float> pack = c.A + G.pos_pack;
+    ap<float> cache = c.A + G.cache_pos;
+    ap<const float> p1 = pack;
+    ap<const float> p2 = pg_side2(c, G);
     const int n1 = G.n1, n2 = sym ? G.n1 : G.n2;
-    gp<int> off = c.I + G.off;
-    gp<int> nbr = c.I + G.nbr;
-    gp<int> row = c.I + G.row;
-    gp<int> toff = c.I + G.toff;
-    gp<int> tmp = c.I + G.tmp;
-    gp<int> tcur = c.I + G.tcur;
+    ap<int> off = c.I + G.off;
+    ap<int> nbr = c.I + G.nbr;
+    ap<int> row = c.I + G.row;
+    ap<int> toff = c.I + G.toff;
+    ap<int> tmp = c.I + G.tmp;
+    ap<int> tcur = c.I + G.tcur;
     int npack = sym ? n1 : n1 + n2;
     for (int i = c.gtid; i < npack * 3; i += c.gsize) cache[i] = pack[i];
     for (int i = c.gtid; i <= n1; i += c.gsize) off[i] = 0;
@@ -418,12 +419,12 @@ __device__ __forceinline__ bool pg_rebuild(Ctx& c, GraphC& G) {
     pacc(c, PROF_RB_FILL, t0);
     t0 = ptick(c);
     // transposed rows: column counts, arrival-order placement, slot order
-    for (int s = c.gtid; s < E; s += c.gsize) atomicAdd((int*)(toff + nbr[s]), 1);
+    for (int s = c.gtid; s < E; s += c.gsize) atomicAdd((int*)(toff + nbr[s]).ptr(), 1);
     team_sync(c);
     team_exscan(c, toff, n2 + 1);
     for (int j = c.gtid; j < n2; j += c.gsize) tcur[j] = toff[j];
     team_sync(c);
-    for (int s = c.gtid; s < E; s += c.gsize) tmp[atomicAdd((int*)(tcur + nbr[s]), 1)] = s;
+    for (int s = c.gtid; s < E; s += c.gsize) tmp[atomicAdd((int*)(tcur + nbr[s]).ptr(), 1)] = s;
     team_sync(c);
     pg_order_columns(c, G, n2);
     pacc(c, PROF_RB_MAP, t0);
@@ -555,7 +556,7 @@ __device__ __forceinline__ void cross3_rn(const float* a, const float* b, float*
 // repulsion between the placed backbone atoms (at most 4) of two residues;
 // derivatives are (force, torque) on each residue frame.
 __device__ __forceinline__ float backbone_edge(const Ctx& c, OpC& op, int r1, int r2, float* d1, float* d2) {
-    gp<const float> aff = c.A + op.in_out[0];
+    ap<const float> aff = c.A + op.in_out[0];
     int w = op.in_w[0];
     gp<const float> ref = c.CF + op.ia[1];
     gp<const int> nat = c.CI + op.ia[2];
@@ -624,32 +625,32 @@ __device__ __forceinline__ float backbone_edge(const Ctx& c, OpC& op, int r1, in
 // param is the coefficient table (LDS or memory).
 template <int KIND, int DD1, int DD2, class P>
 __device__ __forceinline__ void pg_edges_impl(Ctx& c, GraphC& G, OpC& op, P param) {
-    gp<const int> nbr = c.I + G.nbr;
-    gp<const int> row = c.I + G.row;
-    gp<int> act = c.I + G.act;
-    gp<float> val = c.A + G.val;
-    gp<float> D1 = c.A + G.d1;
-    gp<float> D2 = c.A + G.d2;
-    gp<const float> pack = c.A + G.pos_pack;
-    gp<const float> pk2 = pg_side2(c, G);
+    ap<const int> nbr = c.I + G.nbr;
+    ap<const int> row = c.I + G.row;
+    ap<int> act = c.I + G.act;
+    ap<float> val = c.A + G.val;
+    ap<float> D1 = c.A + G.d1;
+    ap<float> D2 = c.A + G.d2;
+    ap<const float> pack = c.A + G.pos_pack;
+    ap<const float> pk2 = pg_side2(c, G);
     gp<const int> loc1 = c.CI + G.loc1;
     gp<const int> loc2 = c.CI + G.loc2;
     gp<const int> t1 = c.CI + G.type1;
     gp<const int> t2 = c.CI + G.type2;
-    gp<const float> P1 = c.A + G.out1;
-    gp<const float> P2 = c.A + G.out2;
+    ap<const float> P1 = c.A + G.out1;
+    ap<const float> P2 = c.A + G.out2;
     const int E = uni(c.I[G.state + 3]);
     const int cap = G.ecap;
     for (int s = c.gtid; s < E; s += c.gsize) {
         int i1 = row[s], j = nbr[s];
-        gp<const float> xp = pack + i1 * 3;
-        gp<const float> yp = pk2 + j * 3;
+        ap<const float> xp = pack + i1 * 3;
+        ap<const float> yp = pk2 + j * 3;
         float d2 = refine_dist2(xp[0] - yp[0], xp[1] - yp[1], xp[2] - yp[2]);
         int a = d2 < G.cutoff2;
         act[s] = a;
         if (!a) { val[s] = 0.f; continue; }
-        gp<const float> x1 = P1 + loc1[i1] * G.w1;
-        gp<const float> x2 = P2 + loc2[j] * G.w2;
+        ap<const float> x1 = P1 + loc1[i1] * G.w1;
+        ap<const float> x2 = P2 + loc2[j] * G.w2;
         P p = param + (t1[i1] * G.n_type2 + t2[j]) * G.n_param;
         float e1[7], e2[7];
         float v = 0.f;
@@ -715,17 +716,17 @@ static_assert(GW <= 32 && (GW & (GW - 1)) == 0, "a lane group is a power of two 
 
 template <int D1N, int D2N>
 __device__ __forceinline__ void pg_gather_t(Ctx& c, GraphC& G) {
-    gp<const int> off = c.I + G.off;
-    gp<const int> toff = c.I + G.toff;
-    gp<const int> tslot = c.I + G.tslot;
-    gp<const int> act = c.I + G.act;
-    gp<const float> es = c.A + G.esens;
-    gp<const float> D1 = c.A + G.d1;
-    gp<const float> D2 = c.A + G.d2;
+    ap<const int> off = c.I + G.off;
+    ap<const int> toff = c.I + G.toff;
+    ap<const int> tslot = c.I + G.tslot;
+    ap<const int> act = c.I + G.act;
+    ap<const float> es = c.A + G.esens;
+    ap<const float> D1 = c.A + G.d1;
+    ap<const float> D2 = c.A + G.d2;
     gp<const int> loc1 = c.CI + G.loc1;
     gp<const int> loc2 = c.CI + G.loc2;
-    gp<float> S1 = c.A + G.sens1;
-    gp<float> S2 = c.A + G.sens2;
+    ap<float> S1 = c.A + G.sens1;
+    ap<float> S2 = c.A + G.sens2;
     const int cap = G.ecap;
     int grp = c.gtid / GW, gl = c.gtid % GW;
     const int NG = c.gsize / GW;
@@ -765,9 +766,8 @@ __device__ __forceinline__ void pg_gather_t(Ctx& c, GraphC& G) {
 #pragma unroll
         for (int q = 0; q < D1N; ++q) acc[q] = group_sum<GW>(acc[q]);
         if (ok && gl == 0) {
-            gp<float> dst = S1 + loc1[i] * G.w1;
-#pragma unroll
-            for (int q = 0; q < D1N; ++q) dst[q] += acc[q];
+            ap<float> dst = S1 + loc1[i] * G.w1;
+            dst.template add<D1N>(acc);
         }
     }
     // both sides in one phase unless they accumulate into shared producer rows
@@ -794,9 +794,8 @@ __device__ __forceinline__ void pg_gather_t(Ctx& c, GraphC& G) {
 #pragma unroll
         for (int q = 0; q < D2N; ++q) acc[q] = group_sum<GW>(acc[q]);
         if (ok && gl == 0) {
-            gp<float> dst = S2 + loc2[j] * G.w2;
-#pragma unroll
-            for (int q = 0; q < D2N; ++q) dst[q] += acc[q];
+            ap<float> dst = S2 + loc2[j] * G.w2;
+            dst.template add<D2N>(acc);
         }
     }
     team_sync(c);
@@ -816,9 +815,9 @@ __device__ __forceinline__ void pg_gather(Ctx& c, GraphC& G) {
 // (side 2), in slot order: out[k*stride] = sum.  Groups of 16 lanes.
 template <class O>
 __device__ __forceinline__ void pg_row_sums(Ctx& c, GraphC& G, bool side2, O out, int stride) {
-    gp<const int> off = c.I + (side2 ? G.toff : G.off);
-    gp<const int> tslot = c.I + G.tslot;
-    gp<const float> val = c.A + G.val;
+    ap<const int> off = c.I + (side2 ? G.toff : G.off);
+    ap<const int> tslot = c.I + G.tslot;
+    ap<const float> val = c.A + G.val;
     int n = side2 ? G.n2 : G.n1;
     int grp = c.gtid / GW, gl = c.gtid % GW;
     for (int base = 0; base < n; base += c.gsize / GW) {

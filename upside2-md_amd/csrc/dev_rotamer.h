@@ -27,8 +27,8 @@ namespace upside {
 
 struct RotView {
     gp<const int> nrot, bead0, brot, bnode;
-    gp<int> coff, ca, cb, scand, ioff, iinc, eidx, bpc, bpf, bps, ninc, binc, stats;
-    gp<float> P, msg, marg, e1x, nprob, ncur, nold, noff, feat, nprev;
+    ap<int> coff, ca, cb, scand, ioff, iinc, eidx, bpc, bpf, bps, ninc, binc, stats;
+    ap<float> P, msg, marg, e1x, nprob, ncur, nold, noff, feat, nprev;
     int cap;
 };
 
@@ -141,10 +141,10 @@ __device__ __forceinline__ bool rot_candidate_lists(Ctx& c, GraphC& G, RotC& R, 
 // capacity overflow.
 __device__ __forceinline__ bool rot_rebuild(Ctx& c, GraphC& G, RotC& R) {
     RotView v = rot_view(c, R);
-    gp<const float> pack = c.A + G.pos_pack;
-    gp<float> cen = c.A + R.ncen;
-    gp<const int> row = c.I + G.row;
-    gp<const int> nbr = c.I + G.nbr;
+    ap<const float> pack = c.A + G.pos_pack;
+    ap<float> cen = c.A + R.ncen;
+    ap<const int> row = c.I + G.row;
+    ap<const int> nbr = c.I + G.nbr;
     const int n = R.n_node;
     for (int a = c.gtid; a < n; a += c.gsize) {
         int b0 = v.bead0[a], b1 = v.bead0[a + 1];
@@ -168,7 +168,7 @@ __device__ __forceinline__ bool rot_rebuild(Ctx& c, GraphC& G, RotC& R) {
         __syncthreads();
         ok = rot_candidate_lists(c, G, R, v, (lp<const float>)L);
     } else {
-        ok = rot_candidate_lists(c, G, R, v, (gp<const float>)cen);
+        ok = rot_candidate_lists(c, G, R, v, (ap<const float>)cen);
     }
     if (!ok) return false;
     // candidate of every bead slot
@@ -195,13 +195,13 @@ __device__ __forceinline__ bool rot_rebuild(Ctx& c, GraphC& G, RotC& R) {
 // Node probabilities, BP-edge compaction and edge matrices for this evaluation.
 __device__ __forceinline__ void rot_fill(Ctx& c, GraphC& G, RotC& R) {
     RotView v = rot_view(c, R);
-    gp<const int> off = c.I + G.off;
-    gp<const int> nbr = c.I + G.nbr;
-    gp<const int> row = c.I + G.row;
-    gp<const int> toff = c.I + G.toff;
-    gp<const int> tslot = c.I + G.tslot;
-    gp<const int> act = c.I + G.act;
-    gp<const float> val = c.A + G.val;
+    ap<const int> off = c.I + G.off;
+    ap<const int> nbr = c.I + G.nbr;
+    ap<const int> row = c.I + G.row;
+    ap<const int> toff = c.I + G.toff;
+    ap<const int> tslot = c.I + G.tslot;
+    ap<const int> act = c.I + G.act;
+    ap<const float> val = c.A + G.val;
     gp<const int> loc1 = c.CI + G.loc1;
     const int E = uni(c.I[G.state + 3]);
     const int C = uni(v.coff[R.n_node]);
@@ -235,7 +235,7 @@ __device__ __forceinline__ void rot_fill(Ctx& c, GraphC& G, RotC& R) {
         for (int k = 0; k < 6; ++k) {
             float s = 0.f;
             if (k < nr) {
-                for (int q = 0; q < R.n_prob; ++q) s += c.A[R.prob_out[q] + loc1[b0 + k] * R.prob_w[q]];
+                for (int q = 0; q < R.n_prob; ++q) s += (c.A + R.prob_out[q])[loc1[b0 + k] * R.prob_w[q]];
                 mn = fminf(mn, s);
             }
             e[k] = s;
@@ -327,18 +327,18 @@ struct BpMem {
     static constexpr bool AOS = !__is_same(F, lp<float>);
     F msg;             // component (side*6 + r) of edge e at msg[mi(side*6 + r, e)]
     int ms;
-    gp<const float> P; // edge matrices (memory), entry (i, j) of edge e at P[pi(i*6 + j, e)]
+    gp<const float> P; // edge matrices (memory, unchanged during the solve: through L1), entry (i, j) of edge e at P[pi(i*6 + j, e)]
     int ps;
     __device__ __forceinline__ int mi(int r, int e) const { return AOS ? e * 12 + r : r * ms + e; }
     __device__ __forceinline__ int pi(int q, int e) const { return AOS ? e * 36 + q : q * ps + e; }
     __device__ __forceinline__ int cs() const { return AOS ? 1 : ms; }  // stride of a message's components
-    gp<const float> prob;  // node probabilities [n*6]
+    gp<const float> prob;  // node probabilities [n*6], likewise
     I ends;            // edge endpoints: first | second << 16 (rows, columns of P)
     I ioff, ninc;      // node incidences inc[ioff[x] + t], t < ninc[x]
     J inc;             // incidence: edge*2 + side
     gp<const int> nrot;
     int c1, c2;        // edges [0,c1) are 3x3, [c1,c2) 3x6, the rest 6x6 (unsorted: c1 = c2 = 0)
-    gp<const int> pos; // position of BP edge e in this order (null: the order of the BP edges)
+    gp<const int> pos; // LDS: position of BP edge e in this order (memory: the order of the BP edges)
 };
 
 // Who runs a BP pass: one workgroup (TEAM = false: threads c.tid of NT,
@@ -482,8 +482,11 @@ __device__ __forceinline__ void bp_node_store(int x, const float* pr, const floa
         for (int r = 0; r < 6; ++r) mx = fmaxf(mx, b[r]);
         float im = 1.f / mx;
         const float w = __fmul_rn(1.f - damping, im);
+        float o[6];
 #pragma unroll
-        for (int r = 0; r < 6; ++r) ncur_[x * 6 + r] = __fmaf_rn(damping, nold_[x * 6 + r], __fmul_rn(w, b[r]));
+        for (int r = 0; r < 6; ++r) o[r] = nold_[x * 6 + r];  // before the first store
+#pragma unroll
+        for (int r = 0; r < 6; ++r) ncur_[x * 6 + r] = __fmaf_rn(damping, o[r], __fmul_rn(w, b[r]));
     }
 }
 
@@ -567,7 +570,7 @@ __device__ __forceinline__ void rot_node_pass(Ctx& c, const BpMem<F, I, J>& m, i
 // need one team barrier instead of two.  Results equal rot_edge_pass +
 // rot_node_pass.
 template <class F, class I, class J>
-__device__ __forceinline__ void rot_fused_pass(Ctx& c, const BpMem<F, I, J>& m, gp<const float> min_, gp<float> mout, int n_node,
+__device__ __forceinline__ void rot_fused_pass(Ctx& c, const BpMem<F, I, J>& m, ap<const float> min_, ap<float> mout, int n_node,
                                F ncur_, F nold_, float damping, bool swap_first) {
     const int t = c.gtid, gl = t % NODE_LANES;
     for (int x = t / NODE_LANES; x < n_node; x += c.gsize / NODE_LANES) {  // uniform in a group
@@ -635,8 +638,8 @@ __device__ __forceinline__ void rot_fused_pass(Ctx& c, const BpMem<F, I, J>& m, 
 //   rest 0.
 // Nodes with one state get a row of zeros.
 template <bool TEAM, class F, class I, class J>
-__device__ __forceinline__ void bp_features(Ctx& c, const BpMem<F, I, J>& m, int n_node, F b0, gp<const float> prev,
-                            gp<float> feat) {
+__device__ __forceinline__ void bp_features(Ctx& c, const BpMem<F, I, J>& m, int n_node, F b0, ap<const float> prev,
+                            ap<float> feat) {
     for (int x = bp_t<TEAM>(c); x < n_node; x += bp_nt<TEAM>(c)) {
         float f[MLP_IN];
 #pragma unroll
@@ -689,7 +692,7 @@ __device__ __forceinline__ void bp_features(Ctx& c, const BpMem<F, I, J>& m, int
 // states (max-normalised, as the damped update leaves beliefs), into cur.
 template <bool TEAM, class F, class I, class J>
 __device__ __forceinline__ void bp_warm_beliefs(Ctx& c, const BpMem<F, I, J>& m, const MlpDev& w, int n_node,
-                                gp<const float> feat, F cur) {
+                                ap<const float> feat, F cur) {
     const int t = bp_t<TEAM>(c), nw = bp_nt<TEAM>(c) / 64;
     const int l = t & 63, g = l >> 4, cl = l & 15;
     for (int tile = t / 64; tile * 16 < n_node; tile += nw) {  // uniform over the wave
@@ -815,7 +818,7 @@ __device__ __forceinline__ int bp_iterate(Ctx& c, RotC& R, const RotView& v, con
         unsigned long long t0 = ptick(c);
         if constexpr (TEAM) {
             if (!swap_first) {
-                rot_fused_pass(c, mm, (gp<const float>)mm.msg, (gp<float>)other, n, cur_, old_, damping, false);
+                rot_fused_pass(c, mm, (ap<const float>)mm.msg, (ap<float>)other, n, cur_, old_, damping, false);
                 F tt = mm.msg; mm.msg = other; other = tt;
                 pacc(c, PROF_BP_NODE, t0);
                 return;
@@ -830,11 +833,11 @@ __device__ __forceinline__ int bp_iterate(Ctx& c, RotC& R, const RotView& v, con
     for (;;) {
         iterate(cur, old, 0.f, true);
         if (mode > 0 && total == 0)  // old: the first pass's product
-            bp_features<TEAM>(c, mm, n, old, (gp<const float>)v.nprev, v.feat);
+            bp_features<TEAM>(c, mm, n, old, (ap<const float>)v.nprev, v.feat);
         if (warm) {
             const auto& w = c.args->mlp;
             const MlpDev net = {w.w1, w.w2p, w.w3p, w.w3tp, w.w2tp, w.b1, w.b2, w.b3};
-            bp_warm_beliefs<TEAM>(c, mm, net, n, (gp<const float>)v.feat, cur);
+            bp_warm_beliefs<TEAM>(c, mm, net, n, (ap<const float>)v.feat, cur);
             bp_local_messages<TEAM>(c, mm, nbp, cur, c.args->bp_klocal);
         }
         const float tol = resid || (mode == 3 && c.args->bp_residual > 0.f) ? c.args->bp_residual : R.tol;
@@ -874,7 +877,7 @@ __device__ __forceinline__ int bp_iterate(Ctx& c, RotC& R, const RotView& v, con
     unsigned long long t0 = ptick(c);
     // node marginals (:283-290) into memory and into `old` (free now; cur and
     // old are always distinct buffers)
-    gp<float> ncur = v.ncur;
+    ap<float> ncur = v.ncur;
     for (int x = t; x < n; x += nt) {
         int nr = m.nrot[x];
         float b[6];
@@ -889,9 +892,9 @@ __device__ __forceinline__ int bp_iterate(Ctx& c, RotC& R, const RotView& v, con
     }
     bp_sync<TEAM>(c);
     // edge marginals (:425-449), written in the order of the BP edges
-    gp<float> marg = v.marg;
+    ap<float> marg = v.marg;
     for (int e = t; e < nbp; e += nt) {
-        const int k = m.pos ? m.pos[e] : e;
+        const int k = m.AOS ? e : m.pos[e];
         const int ends = m.ends[k];
         const int f = ends & 0xFFFF, s = ends >> 16;
         float b1[6], b2[6];
@@ -940,6 +943,7 @@ __device__ __forceinline__ bool bp_fits_lds(int nbp, int n, int cap) {
 // iteration count.
 __device__ __forceinline__ int rot_solve_wg(Ctx& c, RotC& R) {
     RotView v = rot_view(c, R);
+    l1_drop(c);
     const int nbp = uni(v.stats[4]);
     const int n = R.n_node;
     const int cap = v.cap;
@@ -948,7 +952,7 @@ __device__ __forceinline__ int rot_solve_wg(Ctx& c, RotC& R) {
         if (c.tid == 0) v.stats[6] += 1;  // solves held in LDS
         lp<float> L = c.lds;
         BpMem<lp<float>, lp<int>, lp<unsigned short>> m;
-        m.nrot = v.nrot; m.prob = (gp<const float>)v.nprob;
+        m.nrot = v.nrot; m.prob = c.A.cached(R.nprob);
         m.msg = L; m.ms = nbp; L += 12 * nbp;
         lp<float> cur = L; L += 6 * n;
         lp<float> old = L; L += 6 * n;
@@ -981,8 +985,9 @@ __device__ __forceinline__ int rot_solve_wg(Ctx& c, RotC& R) {
         block_exscan(c, S + 2 * nbp, nbp);
         m.c1 = n0;
         m.c2 = n0 + n1;
-        gp<float> Ps = v.msg;  // matrices in class order, stride nbp
-        gp<int> gpos = v.bpc;  // position of every BP edge (endpoints now staged)
+        gp<const float> P0 = c.A.cached(R.P);
+        ap<float> Ps = v.msg;  // matrices in class order, stride nbp
+        ap<int> gpos = v.bpc;  // position of every BP edge (endpoints now staged)
         for (int e = c.tid; e < nbp; e += NT) {
             const int en = stash[e];
             const int nf = v.nrot[en & 0xFFFF], ns = v.nrot[en >> 16];
@@ -992,7 +997,7 @@ __device__ __forceinline__ int rot_solve_wg(Ctx& c, RotC& R) {
             posl[e] = k;
             gpos[e] = k;
 #pragma unroll 4
-            for (int q = 0; q < 36; ++q) Ps[q * nbp + k] = v.P[e * 36 + q];
+            for (int q = 0; q < 36; ++q) Ps[q * nbp + k] = P0[e * 36 + q];
         }
         __syncthreads();
         for (int x = c.tid; x < n; x += NT) {
@@ -1003,7 +1008,7 @@ __device__ __forceinline__ int rot_solve_wg(Ctx& c, RotC& R) {
             }
         }
         __syncthreads();  // the scratch is overwritten by the messages next
-        m.P = (gp<const float>)Ps; m.ps = nbp; m.pos = (gp<const int>)gpos;
+        m.P = c.A.cached(R.msg); m.ps = nbp; m.pos = c.I.cached(R.bpc);
         m.ends = ends; m.ioff = ioff; m.ninc = ninc; m.inc = inc;
         // initial messages = 1, old beliefs = prob (:1110-1133)
         for (int e = c.tid; e < nbp; e += NT)
@@ -1013,12 +1018,11 @@ __device__ __forceinline__ int rot_solve_wg(Ctx& c, RotC& R) {
         pacc(c, PROF_BP_SETUP, t0);
         return bp_iterate<false>(c, R, v, m, nbp, cur, old);
     }
-    BpMem<gp<float>, gp<int>, gp<int>> m;
-    m.P = (gp<const float>)v.P; m.ps = 0; m.nrot = v.nrot; m.prob = (gp<const float>)v.nprob;
+    BpMem<ap<float>, gp<const int>, gp<const int>> m;
+    m.P = c.A.cached(R.P); m.ps = 0; m.nrot = v.nrot; m.prob = c.A.cached(R.nprob);
     m.msg = v.msg; m.ms = 0;
-    m.ends = v.bpc; m.ioff = v.ioff; m.ninc = v.ninc; m.inc = v.binc;
+    m.ends = c.I.cached(R.bpc); m.ioff = c.I.cached(R.ioff); m.ninc = c.I.cached(R.ninc); m.inc = c.I.cached(R.binc);
     m.c1 = m.c2 = 0;
-    m.pos = nullptr;
     for (int i = c.tid; i < n * 6; i += NT) v.nold[i] = v.nprob[i];
     for (int e = c.tid; e < nbp; e += NT)
 #pragma unroll
@@ -1034,15 +1038,15 @@ __device__ __forceinline__ int rot_solve_wg(Ctx& c, RotC& R) {
 // iteration count.
 __device__ __forceinline__ int rot_solve_team(Ctx& c, RotC& R) {
     RotView v = rot_view(c, R);
+    l1_drop(c);
     const int nbp = uni(v.stats[4]);
     const int n = R.n_node;
     unsigned long long t0 = ptick(c);
-    BpMem<gp<float>, gp<int>, gp<int>> m;
-    m.P = (gp<const float>)v.P; m.ps = 0; m.nrot = v.nrot; m.prob = (gp<const float>)v.nprob;
+    BpMem<ap<float>, gp<const int>, gp<const int>> m;
+    m.P = c.A.cached(R.P); m.ps = 0; m.nrot = v.nrot; m.prob = c.A.cached(R.nprob);
     m.msg = v.msg; m.ms = 0;
-    m.ends = v.bpc; m.ioff = v.ioff; m.ninc = v.ninc; m.inc = v.binc;
+    m.ends = c.I.cached(R.bpc); m.ioff = c.I.cached(R.ioff); m.ninc = c.I.cached(R.ninc); m.inc = c.I.cached(R.binc);
     m.c1 = m.c2 = 0;
-    m.pos = nullptr;
     for (int i = c.gtid; i < n * 6; i += c.gsize) v.nold[i] = v.nprob[i];
     for (int e = c.gtid; e < nbp; e += c.gsize)
 #pragma unroll
@@ -1090,10 +1094,10 @@ __device__ __forceinline__ float rot_free_energy(Ctx& c, GraphC& G, RotC& R) {
         en += e;
     }
     // 1-rotamer pairs: -log P with P the probability of their single bead pair
-    gp<const int> row = c.I + G.row;
-    gp<const int> nbr = c.I + G.nbr;
-    gp<const int> act = c.I + G.act;
-    gp<const float> val = c.A + G.val;
+    ap<const int> row = c.I + G.row;
+    ap<const int> nbr = c.I + G.nbr;
+    ap<const int> act = c.I + G.act;
+    ap<const float> val = c.A + G.val;
     const int E = uni(c.I[G.state + 3]);
     for (int s = c.gtid; s < E; s += c.gsize)
         if (act[s] && v.nrot[v.bnode[row[s]]] == 1 && v.nrot[v.bnode[nbr[s]]] == 1) en += -logf(expf(-val[s]));
@@ -1116,10 +1120,10 @@ __device__ __forceinline__ float rot_free_energy(Ctx& c, GraphC& G, RotC& R) {
 // sensitivities (:1074-1085).
 __device__ __forceinline__ void rot_sens(Ctx& c, GraphC& G, RotC& R) {
     RotView v = rot_view(c, R);
-    gp<const int> row = c.I + G.row;
-    gp<const int> nbr = c.I + G.nbr;
-    gp<const int> act = c.I + G.act;
-    gp<float> es = c.A + G.esens;
+    ap<const int> row = c.I + G.row;
+    ap<const int> nbr = c.I + G.nbr;
+    ap<const int> act = c.I + G.act;
+    ap<float> es = c.A + G.esens;
     gp<const int> loc1 = c.CI + G.loc1;
     const int E = uni(c.I[G.state + 3]);
     const int cap = v.cap;
@@ -1142,7 +1146,7 @@ __device__ __forceinline__ void rot_sens(Ctx& c, GraphC& G, RotC& R) {
     }
     for (int b = c.gtid; b < G.n1; b += c.gsize) {
         float m = v.ncur[v.bnode[b] * 6 + v.brot[b]];
-        for (int q = 0; q < R.n_prob; ++q) c.A[R.prob_sens[q] + loc1[b] * R.prob_w[q]] += m;
+        for (int q = 0; q < R.n_prob; ++q) (c.A + R.prob_sens[q])[loc1[b] * R.prob_w[q]] += m;
     }
     team_sync(c);
 }

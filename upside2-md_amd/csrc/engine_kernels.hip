@@ -48,10 +48,11 @@ __device__ __forceinline__ void dist3d_bwd(Ctx& c, OpC& op) {
     auto der = c.A + op.scratch;
     auto con = c.A + op.ia[1];
     for (int e = c.gtid; e < op.n_elem; e += c.gsize) {
-        float s = SENS(op)[e];
+        float s = SENS(op)[e], d[3];
+        (der + e * 3).get<3>(d);
         for (int k = 0; k < 3; ++k) {
-            con[(e * 2 + 0) * 3 + k] = s * der[e * 3 + k];
-            con[(e * 2 + 1) * 3 + k] = -s * der[e * 3 + k];
+            con[(e * 2 + 0) * 3 + k] = s * d[k];
+            con[(e * 2 + 1) * 3 + k] = -s * d[k];
         }
     }
 }
@@ -84,9 +85,10 @@ __device__ __forceinline__ void angle_bwd(Ctx& c, OpC& op) {
     auto der = c.A + op.scratch;
     auto con = c.A + op.ia[1];
     for (int e = c.gtid; e < op.n_elem; e += c.gsize) {
-        float s = SENS(op)[e];
+        float s = SENS(op)[e], d[6];
+        (der + e * 6).get<6>(d);
         for (int k = 0; k < 3; ++k) {
-            float d1 = s * der[e * 6 + k], d2 = s * der[e * 6 + 3 + k];
+            float d1 = s * d[k], d2 = s * d[3 + k];
             con[(e * 3 + 0) * 3 + k] = d1;
             con[(e * 3 + 1) * 3 + k] = d2;
             con[(e * 3 + 2) * 3 + k] = -d1 - d2;
@@ -143,8 +145,9 @@ __device__ __forceinline__ void dihedral_bwd(Ctx& c, OpC& op) {
     auto jac = c.A + op.scratch;
     auto con = c.A + op.ia[1];
     for (int e = c.gtid; e < op.n_elem; e += c.gsize) {
-        float s = SENS(op)[e];
-        for (int k = 0; k < 12; ++k) con[e * 12 + k] = s * jac[e * 12 + k];
+        float s = SENS(op)[e], d[12];
+        (jac + e * 12).get<12>(d);
+        for (int k = 0; k < 12; ++k) con[e * 12 + k] = s * d[k];
     }
 }
 
@@ -178,8 +181,9 @@ __device__ __forceinline__ void rama_coord_fwd(Ctx& c, OpC& op) {
     auto i1 = CIA(op, 0);
     auto i2 = CIA(op, 1);
     for (int e = c.gtid; e < op.n_elem; e += c.gsize) {
-        OUT(op)[2 * e] = IN(op, 0)[i1[e] * op.in_w[0]];
-        OUT(op)[2 * e + 1] = IN(op, 1)[i2[e] * op.in_w[1]];
+        const float phi = IN(op, 0)[i1[e] * op.in_w[0]], psi = IN(op, 1)[i2[e] * op.in_w[1]];
+        OUT(op)[2 * e] = phi;
+        OUT(op)[2 * e + 1] = psi;
     }
 }
 __device__ __forceinline__ void cat_pos_fwd(Ctx& c, OpC& op) {
@@ -208,7 +212,7 @@ __device__ __forceinline__ void rama_map_fwd(Ctx& c, SysC& S, OpC& op) {
         float v, dx, dy;
         bicubic(coef + ((size_t)(mid[e] * nx + xb) * nx + yb) * 16, x - xb, y - yb, v, dx, dy);
         pot += v;
-        c.A[op.scratch + 2 * n + e] = v;  // per-residue potential (logging)
+        (c.A + op.scratch)[2 * n + e] = v;  // per-residue potential (logging)
         con[2 * e] = dx * scale;
         con[2 * e + 1] = dy * scale;
     }
@@ -359,19 +363,25 @@ __device__ __forceinline__ void affine_bwd(Ctx& c, OpC& op) {
     auto ec = c.A + op.scratch + 4 * op.n_elem;
     auto con = c.A + op.ia[2];
     for (int r = c.gtid; r < op.n_elem; r += c.gsize) {
-        auto s = SENS(op) + r * 7;
-        auto E = ec + r * 16;
-        auto q = E;
+        float s[7], E[16], w[4];
+        (SENS(op) + r * 7).get<7>(s);
+        (ec + r * 16).get<16>(E);
+        (ev + r * 4).get<4>(w);
+        const float* q = E;
         float t0 = s[3], t1 = s[4], t2 = s[5];
-        float qs[4] = {2.f * (-t0 * q[1] - t1 * q[2] - t2 * q[3]), 2.f * (t0 * q[0] + t1 * q[3] - t2 * q[2]),
-                       2.f * (t1 * q[0] + t2 * q[1] - t0 * q[3]), 2.f * (t2 * q[0] + t0 * q[2] - t1 * q[1])};
+        // roundings fixed, here and for dv: which product of a sum is fused otherwise depends on how
+        // the compiler ordered the operands
+        float qs[4] = {2.f * __fmaf_rn(-t2, q[3], __fmaf_rn(-t0, q[1], -__fmul_rn(t1, q[2]))),
+                       2.f * __fmaf_rn(-t2, q[2], __fmaf_rn(t1, q[3], __fmul_rn(t0, q[0]))),
+                       2.f * __fmaf_rn(-t0, q[3], __fmaf_rn(t2, q[1], __fmul_rn(t1, q[0]))),
+                       2.f * __fmaf_rn(-t1, q[1], __fmaf_rn(t0, q[2], __fmul_rn(t2, q[0])))};
         float qsd[4], inv[4];
         for (int dd = 0; dd < 4; ++dd) {
             float acc = 0.f;
             for (int i = 0; i < 4; ++i) acc += qs[i] * E[dd * 4 + i];
             qsd[dd] = acc;
         }
-        for (int k = 1; k < 4; ++k) inv[k] = 1.f / (ev[r * 4] - ev[r * 4 + k]);
+        for (int k = 1; k < 4; ++k) inv[k] = 1.f / (w[0] - w[k]);
         for (int na = 0; na < 3; ++na) {
             auto g = ref + r * 9 + na * 3;
             float gx = g[0], gy = g[1], gz = g[2];
@@ -380,7 +390,7 @@ __device__ __forceinline__ void affine_bwd(Ctx& c, OpC& op) {
                               {gy, -gz, 0.f, gx, -gy, gx, 0.f, gy, gz, -gy},
                               {gz, gy, -gx, 0.f, -gz, 0.f, gx, -gz, gy, gz}};
             for (int j = 0; j < 3; ++j) {
-                float dv = (1.f / 3.f) * s[j];
+                float dv = 0.f;
                 for (int k = 1; k < 4; ++k) {
                     float t = 0.f;
                     for (int a = 0; a < 4; ++a)
@@ -389,7 +399,8 @@ __device__ __forceinline__ void affine_bwd(Ctx& c, OpC& op) {
                             float term = a == b ? E[k * 4 + a] * E[b] : E[k * 4 + a] * E[b] + E[k * 4 + b] * E[a];
                             t += fab * term;
                         }
-                    dv += inv[k] * t * qsd[k];
+                    const float it = __fmul_rn(inv[k], t);
+                    dv = k == 1 ? __fmaf_rn(1.f / 3.f, s[j], __fmul_rn(it, qsd[k])) : __fmaf_rn(it, qsd[k], dv);
                 }
                 con[(r * 3 + na) * 3 + j] = dv;
             }
@@ -416,11 +427,12 @@ __device__ __forceinline__ void placement_fwd(Ctx& c, OpC& op) {
             float v, dx, dy;
             bicubic(data + ((size_t)(layer[e] * nx + xb) * ny + yb) * 16, x - xb, y - yb, v, dx, dy);
             o[0] = v;
-            c.A[op.scratch + 2 * e] = dx * op.fa[0];
-            c.A[op.scratch + 2 * e + 1] = dy * op.fa[1];
+            (c.A + op.scratch)[2 * e] = dx * op.fa[0];
+            (c.A + op.scratch)[2 * e + 1] = dy * op.fa[1];
             continue;
         }
-        auto a = aff + ares[e] * wa;
+        float a[7];
+        (aff + ares[e] * wa).get<7>(a);
         float U[9];
         quat_to_rot(a + 3, U);
         auto v = data + layer[e] * dim;
@@ -436,9 +448,10 @@ __device__ __forceinline__ void placement_bwd(Ctx& c, OpC& op) {
     auto con = c.A + op.ia[8];
     if (is_rama) {
         for (int e = c.gtid; e < op.n_elem; e += c.gsize) {
-            float s = SENS(op)[e];
-            con[2 * e] = s * c.A[op.scratch + 2 * e];
-            con[2 * e + 1] = s * c.A[op.scratch + 2 * e + 1];
+            float s = SENS(op)[e], d[2];
+            (c.A + op.scratch + 2 * e).get<2>(d);
+            con[2 * e] = s * d[0];
+            con[2 * e + 1] = s * d[1];
         }
         return;
     }
@@ -446,9 +459,10 @@ __device__ __forceinline__ void placement_bwd(Ctx& c, OpC& op) {
     auto aff = IN(op, 0);
     int wa = op.in_w[0];
     for (int e = c.gtid; e < op.n_elem; e += c.gsize) {
-        auto s = SENS(op) + e * op.width;
-        auto x = OUT(op) + e * op.width;
-        auto t = aff + ares[e] * wa;
+        float s[6], x[6], t[3];
+        (SENS(op) + e * op.width).get<6>(s);
+        (OUT(op) + e * op.width).get<6>(x);
+        (aff + ares[e] * wa).get<3>(t);
         float p[3] = {x[0] - t[0], x[1] - t[1], x[2] - t[2]};
         float tq1[3], tq2[3];
         cross3(p, s, tq1);
@@ -470,7 +484,9 @@ __device__ __forceinline__ void infer_fwd(Ctx& c, OpC& op) {
     for (int e = c.gtid; e < op.n_elem; e += c.gsize) {
         auto pc = P + id[3 * e] * w; auto cc = P + id[3 * e + 1] * w; auto nc = P + id[3 * e + 2] * w;
         float pr[3], nx[3], ds[3];
-        for (int k = 0; k < 3; ++k) { pr[k] = pc[k] - cc[k]; nx[k] = nc[k] - cc[k]; }
+        float cx[3];
+        cc.get<3>(cx);
+        for (int k = 0; k < 3; ++k) { pr[k] = pc[k] - cx[k]; nx[k] = nc[k] - cx[k]; }
         float pi = rsqrtf(dot3(pr, pr)), ni = rsqrtf(dot3(nx, nx));
         for (int k = 0; k < 3; ++k) { pr[k] *= pi; nx[k] *= ni; ds[k] = pr[k] + nx[k]; }
         float di = rsqrtf(dot3(ds, ds));
@@ -479,7 +495,7 @@ __device__ __forceinline__ void infer_fwd(Ctx& c, OpC& op) {
         for (int k = 0; k < 3; ++k) { cs[k] = pr[k]; cs[4 + k] = nx[k]; cs[8 + k] = ds[k]; }
         cs[3] = pi; cs[7] = ni; cs[11] = di;
         auto o = OUT(op) + e * 6;
-        for (int k = 0; k < 3; ++k) { o[k] = cc[k] - bl[e] * ds[k]; o[3 + k] = -ds[k]; }
+        for (int k = 0; k < 3; ++k) { o[k] = cx[k] - bl[e] * ds[k]; o[3 + k] = -ds[k]; }
     }
 }
 __device__ __forceinline__ void infer_bwd(Ctx& c, OpC& op) {
@@ -487,8 +503,9 @@ __device__ __forceinline__ void infer_bwd(Ctx& c, OpC& op) {
     auto cache = c.A + op.scratch;
     auto con = c.A + op.ia[2];
     for (int e = c.gtid; e < op.n_elem; e += c.gsize) {
-        auto s = SENS(op) + e * 6;
-        auto cs = cache + e * 12;
+        float s[6], cs[12];
+        (SENS(op) + e * 6).get<6>(s);
+        (cache + e * 12).get<12>(cs);
         float sn[3], sd[3], sp[3], sx[3];
         for (int k = 0; k < 3; ++k) sn[k] = s[3 + k] + bl[e] * s[k];
         float t = dot3(cs + 8, sn);
@@ -520,9 +537,12 @@ __device__ __forceinline__ void protein_hbond_fwd(Ctx& c, OpC& op, GraphC& G) {
         int i = don ? v : v - nd;
         auto src = IN(op, 0) + (don ? loc1[i] : loc2[i]) * op.in_w[0];
         auto o = OUT(op) + v * 7;
+        float x[6];
+        const float sv = ss[v];
+        src.get<6>(x);
 #pragma unroll
-        for (int k = 0; k < 6; ++k) o[k] = src[k];
-        o[6] = 1.f - expf(-ss[v]);
+        for (int k = 0; k < 6; ++k) o[k] = x[k];
+        o[6] = 1.f - expf(-sv);
     }
 }
 __device__ __forceinline__ void protein_hbond_bwd(Ctx& c, OpC& op, GraphC& G) {
@@ -542,13 +562,17 @@ __device__ __forceinline__ void protein_hbond_pass(Ctx& c, OpC& op, GraphC& G) {
     // pass the coordinate sensitivities through to infer_H_O (:419-433)
     auto loc1 = c.CI + G.loc1;
     auto loc2 = c.CI + G.loc2;
-    for (int i = c.gtid; i < G.n1; i += c.gsize)
-#pragma unroll
-        for (int k = 0; k < 6; ++k) INS(op, 0)[loc1[i] * op.in_w[0] + k] += SENS(op)[i * 7 + k];
+    for (int i = c.gtid; i < G.n1; i += c.gsize) {
+        float s[6];
+        (SENS(op) + i * 7).get<6>(s);
+        (INS(op, 0) + loc1[i] * op.in_w[0]).add<6>(s);
+    }
     team_sync(c);
-    for (int j = c.gtid; j < G.n2; j += c.gsize)
-#pragma unroll
-        for (int k = 0; k < 6; ++k) INS(op, 0)[loc2[j] * op.in_w[0] + k] += SENS(op)[(nd + j) * 7 + k];
+    for (int j = c.gtid; j < G.n2; j += c.gsize) {
+        float s[6];
+        (SENS(op) + (nd + j) * 7).get<6>(s);
+        (INS(op, 0) + loc2[j] * op.in_w[0]).add<6>(s);
+    }
     team_sync(c);
 }
 
@@ -626,8 +650,11 @@ __device__ __forceinline__ void weighted_pos_fwd(Ctx& c, OpC& op) {
     for (int e = c.gtid; e < op.n_elem; e += c.gsize) {
         auto p = IN(op, 0) + ip[e] * op.in_w[0];
         auto o = OUT(op) + e * 4;
-        o[0] = p[0]; o[1] = p[1]; o[2] = p[2];
-        o[3] = expf(-IN(op, 1)[iw[e] * op.in_w[1]]);
+        float x[3];
+        p.get<3>(x);
+        const float w = IN(op, 1)[iw[e] * op.in_w[1]];
+        o[0] = x[0]; o[1] = x[1]; o[2] = x[2];
+        o[3] = expf(-w);
     }
 }
 __device__ __forceinline__ void weighted_pos_bwd(Ctx& c, OpC& op) {
@@ -711,7 +738,14 @@ __device__ __forceinline__ void sigmoid_coupling_fwd(Ctx& c, SysC& S, OpC& op) {
         float v, dv;
         compact_sigmoid(wn - ce[t], sh[t], v, dv);
         pot += sc[t] * v;
-        for (int a = 0; a < nt; ++a) xs[r * nt + a] += W[t * nt + a] * sc[t] * dv;
+        for (int a = 0; a < nt; a += 4) {
+            float y[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) y[q] = a + q < nt ? (float)xs[r * nt + a + q] : 0.f;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (a + q < nt) xs[r * nt + a + q] = y[q] + W[t * nt + a + q] * sc[t] * dv;
+        }
     }
     pot = team_sum(c, pot);
     put_pot(c, S, op, pot);
@@ -736,7 +770,14 @@ __device__ __forceinline__ void bb_sigmoid_fwd(Ctx& c, SysC& S, OpC& op) {
         compact_sigmoid(bl - center, sharp, v, dv);
         pot += scale * v;
         float dp = scale * dv;
-        for (int a = 0; a < nt; ++a) scs[r * nt + a] += W[a] * dp;
+        for (int a = 0; a < nt; a += 4) {
+            float y[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) y[q] = a + q < nt ? (float)scs[r * nt + a + q] : 0.f;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (a + q < nt) scs[r * nt + a + q] = y[q] + W[a + q] * dp;
+        }
         hbs[r * op.in_w[1]] += hw * dp;
     }
     pot = team_sum(c, pot);
@@ -990,8 +1031,8 @@ __device__ __forceinline__ bool compute(lp<int> mem, gp<int> words, int mode) {
         Ctx c = ctx_load(mem);
         c.cur_op = nd;  // outside the ops
         for (int r = 0; r < S.sens_zero_cnt; ++r) {
-            cp<int> zr = (cp<int>)(c.I + S.sens_zero + 2 * r);  // written once, by the host
-            gp<float> p = c.A + zr[0];
+            cp<int> zr = cmem((const int*)S.iarena) + S.sens_zero + 2 * r;  // written once, by the host
+            ap<float> p = c.A + zr[0];
             const int n = zr[1];
             for (int i = c.gtid; i < n; i += c.gsize) p[i] = 0.f;
         }
@@ -1275,8 +1316,9 @@ PHASE ph_thermostat(lp<int> mem, float noise_scale, uint64_t inv) {
     for (int a = c.gtid; a < S.n_atom; a += c.gsize) {
         float n[3];
         normal3(S.seed, 0u, (uint32_t)a, inv, n);
-        for (int k = 0; k < 3; ++k)
-            mom[a * 3 + k] = __fmaf_rn(noise_scale, n[k], __fmul_rn(S.mom_scale, mom[a * 3 + k]));
+        float m[3];
+        (mom + a * 3).get<3>(m);
+        for (int k = 0; k < 3; ++k) mom[a * 3 + k] = __fmaf_rn(noise_scale, n[k], __fmul_rn(S.mom_scale, m[k]));
     }
     pacc(c, PROF_THERMO, t0);
     return phase_ret(mem, c, 0);
@@ -1293,9 +1335,10 @@ PHASE ph_integrate(lp<int> mem) {
     const unsigned long long t0 = ptick(c);
     c.cur_op = c.pbase;
     for (int i = c.gtid; i < S.n_atom * 3; i += c.gsize) {
+        const float x = pos[i];
         float p = mom[i] - dt * der[i];
         mom[i] = p;
-        pos[i] += dt * p;
+        pos[i] = x + dt * p;
     }
     team_sync(c);
     pacc(c, PROF_INTEGRATE, t0);
@@ -1432,7 +1475,7 @@ __device__ __forceinline__ void engine_body(SysDesc* systems, lp<float> red, lp<
     SysC& S = cmem(systems)[sys];
     Ctx c;
     c.S = &S;
-    c.A = gmem(S.arena); c.I = gmem(S.iarena); c.CF = gmem(S.cf); c.CI = gmem(S.ci);
+    c.A.p = gmem(S.arena); c.I.p = gmem(S.iarena); c.CF = gmem(S.cf); c.CI = gmem(S.ci);
     c.red = red; c.ired = ired; c.lds = lds;
     c.tid = (int)threadIdx.x;
     c.prof = rank == 0 ? S.prof : nullptr;
@@ -1441,7 +1484,7 @@ __device__ __forceinline__ void engine_body(SysDesc* systems, lp<float> red, lp<
     c.err = S.error;
     c.rank = rank; c.G = G;
     c.gtid = rank * NT + c.tid; c.gsize = G * NT;
-    const gp<int> words = c.I + S.bar;
+    const gp<int> words = gmem(S.iarena) + S.bar;
     c.bar = (gp<unsigned long long>)words;  // 16-byte aligned words
     c.bar_flag = (gp<unsigned>)(words + 2);
     c.bar_next = 0;
@@ -1456,7 +1499,7 @@ __device__ __forceinline__ void engine_body(SysDesc* systems, lp<float> red, lp<
         if (G >= 4) first(SUB_HALF);
         if (G >= 8) first(SUB_QUARTER);
     }
-    c.tred = c.A + S.tred;
+    c.tred = gmem(S.arena) + S.tred;
     c.tpar = 0;
     c.bp_layout = args.bp_layout;
     c.args = &args;
