@@ -280,7 +280,8 @@ int upside_batch_set_lane_split(UpsideBatch* batch, int split);
 int upside_batch_get_lane_split(UpsideBatch* batch);
 /* Where each rotamer BP solve runs (no reference counterpart; the reference
  * solves on its one thread, src/rotamer.cpp:1106-1162): 0 (default) on one
- * workgroup with the BP state in its LDS when it fits (the rest of the team
+ * workgroup with the BP state in its LDS when it fits and the team has fewer
+ * than 16 workgroups or the solve at most 600 edges (the rest of the team
  * meanwhile evaluates the ops that do not depend on the solve), else on
  * several workgroups with the state in memory (with four or more workgroups
  * per system the first half of the team solves while the second half

@@ -1058,25 +1058,24 @@ __device__ __forceinline__ int rot_solve_team(Ctx& c, RotC& R) {
 
 // Where a solve runs: true = rank 0 alone (rot_solve_wg), false = several
 // workgroups (rot_solve_team: the whole team, or its first half beside the
-// independent ops).  bp_layout 0: one workgroup when the state fits LDS or
-// the team has one workgroup, else several; 1: always the whole team; 2:
-// always one workgroup; 3: always several.  Uniform over the team (nbp is
-// read after a team barrier).
+// independent ops).  bp_layout 0: one workgroup if the team has only one, or
+// if the state fits LDS and the team has fewer than BP_TEAM_MIN or the solve at
+// most BP_WG_EDGES edges, else several; 1: always the whole team; 2: always one
+// workgroup; 3: always several.  Uniform over the team (nbp is read after a
+// team barrier).
+//
+// One workgroup's iteration grows with the edges and has no team barrier;
+// several share the edges and pay two.  ms per step, one workgroup / several
+// (edges in brackets): on 16 workgroups 0.336 / 0.357 (285), 0.471 / 0.460
+// (546), 0.637 / 0.609 (825), 0.814 / 0.747 (1287); on 32 0.344 / 0.383 (285),
+// 0.462 / 0.469 (546), 0.599 / 0.584 (825), 0.704 / 0.633 (1287), 0.900 /
+// 0.755 (500 residues).  Half of a team of 8 or 4 never won (67 to 500
+// residues).
+constexpr int BP_TEAM_MIN = 16, BP_WG_EDGES = 600;
 __device__ __forceinline__ bool bp_on_one_wg(const Ctx& c, RotC& R, int nbp, int bp_layout) {
     if (c.G == 1 || bp_layout == 2) return true;
     if (bp_layout == 1 || bp_layout == 3) return false;
-    return bp_fits_lds(nbp, R.n_node, R.ccap);
-}
-
-// Solve by rank 0 of the team while the others wait at the barrier, or by
-// the whole team (see bp_on_one_wg).
-__device__ __forceinline__ int rot_solve(Ctx& c, RotC& R, int bp_layout) {
-    const int nbp = uni(c.I[R.stats + 4]);
-    if (!bp_on_one_wg(c, R, nbp, bp_layout)) return rot_solve_team(c, R);
-    int it = 0;
-    if (c.rank == 0) it = rot_solve_wg(c, R);
-    team_sync(c);
-    return it;
+    return bp_fits_lds(nbp, R.n_node, R.ccap) && (c.G < BP_TEAM_MIN || nbp <= BP_WG_EDGES);
 }
 
 // Bethe free energy (calculate_energy_from_marginals, :915-927).
