@@ -16,6 +16,26 @@ def ue():
     return upside_engine
 
 
+@pytest.mark.parametrize("n_res", [25, 26, 55, 56, 125, 126])
+def test_evaluation_on_a_team(ue, chain_file, monkeypatch, n_res):
+    """Evaluations of a one-system engine, on both sides of each line of the
+    rule for its team, against one workgroup."""
+    import upconfig
+    path = chain_file(n_res, 11)
+    rng = np.random.default_rng(n_res)
+    a = ue.Upside(path, quiet=True)
+    monkeypatch.setenv("UPSIDE_TEAM", "1")
+    b = ue.Upside(path, quiet=True)
+    for _ in range(3):
+        pos = np.ascontiguousarray(upconfig.random_initial_config(n_res, rng), np.float32)
+        np.testing.assert_allclose(a.energy(pos), b.energy(pos), rtol=1e-5)
+        np.testing.assert_array_equal(a.deriv(pos), b.deriv(pos))
+        np.testing.assert_allclose(a.get_output("rotamer"), b.get_output("rotamer"), rtol=1e-5)
+        for node in ("placement_fixed_point_vector_only", "hbond_coverage"):
+            np.testing.assert_array_equal(a.get_output(node), b.get_output(node))
+            np.testing.assert_array_equal(a.get_sens(node), b.get_sens(node))
+
+
 @pytest.mark.parametrize("n_res,team", [(2, 16), (150, 15), (150, 16), (165, 16), (180, 32)])
 def test_rotamer_solve_by_edges(ue, chain_file, n_res, team):
     """The default layout of the rotamer solve around the number of edges where
@@ -31,3 +51,31 @@ def test_rotamer_solve_by_edges(ue, chain_file, n_res, team):
     assert b1.bp_stats(0)["total"] == bt.bp_stats(0)["total"]
     np.testing.assert_array_equal(bt.pos(0), b1.pos(0))
     np.testing.assert_array_equal(bt.mom(0), b1.mom(0))
+
+
+def test_evaluations_in_threads(ue, chain_file):
+    """Engines of several threads, each with its own stream, whose teams ask
+    for the same workgroup slots."""
+    import threading
+
+    import upconfig
+    path = chain_file(126, 11)
+    rng = np.random.default_rng(7)
+    pos = [np.ascontiguousarray(upconfig.random_initial_config(126, rng), np.float32) for _ in range(4)]
+    ref = ue.Upside(path, quiet=True)
+    want = [ref.deriv(p) for p in pos]
+    engines = [ue.Upside(path, quiet=True) for _ in range(4)]
+    bad = []
+
+    def work(k):
+        for i in range(20):
+            p = (i + k) % 4
+            if not np.array_equal(engines[k].deriv(pos[p]), want[p]):
+                bad.append((k, i))
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad

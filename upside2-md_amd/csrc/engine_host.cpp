@@ -2223,6 +2223,17 @@ struct Batch {
         teams.clear();
     }
 
+    // After a barrier timeout: one workgroup per system from here on, nothing
+    // kept of what the abandoned launch left (lists, error words).
+    void drop_teams() {
+        set_team(1);
+        for (auto& sy : sys) {
+            const Topology& T = sy.prog->T;
+            hip_check(hipMemset(sy.iarena + T.err, 0, (2 + MAX_LANES) * sizeof(int)), "error words");
+            for (auto& g : T.graphs) hip_check(hipMemset(sy.iarena + g.state, 0, 2 * sizeof(int)), "list state");
+        }
+    }
+
     bool pack_teams(const vector<int>& t, vector<int>* map) const {
         return plan_team_map(t, upside_max_resident_blocks() / N_XCD, map);
     }
@@ -2638,8 +2649,37 @@ struct DerivEngine {
     bool evaluated = false;   // an evaluation has set every node's outputs and sensitivities
 
     void evaluate(const float* pos, float* deriv) {
-        batch.evaluate_at(pos, deriv);
+        try {
+            batch.evaluate_at(pos, deriv);
+        } catch (const BarrierTimeout&) {
+            // another process's team holds part of the XCD: one workgroup waits for nobody
+            batch.drop_teams();
+            batch.evaluate_at(pos, deriv);
+        }
         evaluated = true;
+    }
+
+    // Workgroups of one evaluation.  Every team gives the same derivative bit
+    // for bit; more workgroups shorten the phases and lengthen their barriers,
+    // and a team's cooperative launch costs 20 us.  us per evaluation with the
+    // derivative, on 1 / 4 / 8 / 16 / 32 workgroups:
+    //   a whole force field (a rotamer solve)
+    //      10 residues  480 /  416 /  421 /  433 /  462
+    //      40           716 /  514 /  503 /  523 /  577
+    //      67          1154 /  658 /  607 /  589 /  619
+    //     101          1445 /  748 /  657 /  643 /  693
+    //     150          2890 / 1226 /  969 /  857 /  832
+    //     500         11227 / 4302 / 2700 / 1927 / 1593
+    //   pair lists, but no rotamer solve (backbone pairs and hydrogen bonds)
+    //     120           210 /  186 /  188 /  197 /  219
+    //     200           266 /  216 /  206 /  213 /  234
+    //     500           600 /  326 /  279 /  262 /  281
+    //   bonded terms only
+    //     500           120 /  141 /  144 /  152 /  166
+    // The lines are drawn where the next team overtakes.
+    static int eval_team(const Topology& T) {
+        if (!T.rots.empty()) return T.n_atom <= 75 ? 4 : T.n_atom <= 165 ? 8 : T.n_atom <= 375 ? 16 : 32;
+        return T.graphs.empty() || T.n_atom < 600 ? 1 : 8;
     }
 };
 // /output logger of one system: the basic-level datasets of the reference's
@@ -3134,6 +3174,8 @@ DerivEngine* construct_deriv_engine(int n_atom, const char* potential_file, bool
     std::unique_ptr<DerivEngine> e(new DerivEngine);
     e->batch.create({string(potential_file)}, {1.f}, n_atom);
     if (e->batch.sys[0].prog->T.n_atom != n_atom) fail("n_atom mismatch");
+    if (!std::getenv("UPSIDE_TEAM"))
+        e->batch.set_team(std::min(DerivEngine::eval_team(e->batch.sys[0].prog->T), e->batch.max_team()));
     return e.release();
     ABI_CATCH(nullptr)
 }
