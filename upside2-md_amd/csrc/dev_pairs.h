@@ -818,7 +818,7 @@ __device__ __forceinline__ void pg_edges_impl(Ctx& c, GraphC& G, OpC& op, P para
 #pragma unroll
         for (int q = 0; q < DD1; ++q) D1[q * cap + s] = e1[q];
 #pragma unroll
-        for (int q = 0; q < DD2; ++q) D2[q * cap + s] = e2[q];
+        for (int q = 0; q < DD2; ++q) D2[s * DD2 + q] = e2[q];
     }
     team_sync(c);
 }
@@ -896,12 +896,10 @@ __device__ __forceinline__ void pg_gather_t(Ctx& c, GraphC& G) {
             for (int t = tb + gl; t < te; t += GW) {
                 int s = tslot[t];
                 bool a = act[s] != 0;
-                float w = es[s];
+                float w = es[s], d[D1N];
+                (D2 + s * D1N).template get<D1N>(d);
 #pragma unroll
-                for (int q = 0; q < D1N; ++q) {
-                    float d = D2[q * cap + s];
-                    acc[q] += a ? w * d : 0.f;
-                }
+                for (int q = 0; q < D1N; ++q) acc[q] += a ? w * d[q] : 0.f;
             }
         }
 #pragma unroll
@@ -925,12 +923,10 @@ __device__ __forceinline__ void pg_gather_t(Ctx& c, GraphC& G) {
         for (int t = tb + gl; t < te; t += GW) {
             int s = tslot[t];
             bool a = act[s] != 0;
-            float w = es[s];
+            float w = es[s], d[D2N];
+            (D2 + s * D2N).template get<D2N>(d);
 #pragma unroll
-            for (int q = 0; q < D2N; ++q) {
-                float d = D2[q * cap + s];
-                acc[q] += a ? w * d : 0.f;
-            }
+            for (int q = 0; q < D2N; ++q) acc[q] += a ? w * d[q] : 0.f;
         }
 #pragma unroll
         for (int q = 0; q < D2N; ++q) acc[q] = group_sum<GW>(acc[q]);
