@@ -311,3 +311,22 @@ def test_warm_start_free_energy_and_forces_match_converged_oracle(ue, chain_file
             assert de < 1e-4 and df < 1e-4, (name, tag, de, df)
     assert rel_rms(got["warm"][1], got["plain"][1]) < 1e-4
     assert got["warm"][3]["warm"] >= 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [33, 2049, 4097, 8300])
+def test_gpu_gradient_row_splits(ue, n):
+    """Loss and gradient where the rows do not fill a workgroup's two chunks,
+    and beyond the rows that the smallest grid takes in one trip: the bars of
+    test_gpu_gradient_matches_oracle."""
+    say("case: warm-start gradient, %d rows" % n)
+    f, t = synthetic_rows(n, 40 + n)
+    p = random_params(22, scale_out=1.0)
+    net = ue.WarmStartNet(seed=1)
+    net.set_params(p)
+    net.set_data(f, t)
+    loss, g = net.loss_grad()
+    loss_o, g_o = M.loss_grad(p.astype(np.float64), f, t)
+    assert abs(loss - loss_o) <= 1e-6 * abs(loss_o)
+    for k, v in block_errors(g.astype(np.float64), g_o).items():
+        assert v < 1e-4, (k, v)
