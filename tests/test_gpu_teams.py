@@ -36,10 +36,12 @@ def test_evaluation_on_a_team(ue, chain_file, monkeypatch, n_res):
             np.testing.assert_array_equal(a.get_sens(node), b.get_sens(node))
 
 
-@pytest.mark.parametrize("n_res,team", [(2, 16), (150, 15), (150, 16), (165, 16), (180, 32)])
+@pytest.mark.parametrize("n_res,team", [(2, 16), (150, 15), (150, 16), (165, 16), (180, 32),
+                                        (256, 16), (257, 16)])
 def test_rotamer_solve_by_edges(ue, chain_file, n_res, team):
     """The default layout of the rotamer solve around the number of edges where
-    it changes from one workgroup to several."""
+    it changes from one workgroup to several, and around the number of nodes
+    that half the team can keep in registers."""
     path = chain_file(n_res, 12)
     b1 = ue.Batch([path], [0.85], seed=6)
     b1.run(3)

@@ -130,7 +130,7 @@ struct Team {
 // the few outlined phase functions of the kernel (PHASE), and within one a
 // context is a set of scalar registers: ctx_load reads it from LDS at the
 // phase's start.  (Passed by reference it lives in private memory, and every
-// phase begins by reloading it from L2, since a team barrier drops L1.
+// phase began by reloading it from L2, when a team barrier still dropped L1.
 // Measured with the program records in scalar registers, ms per step: 0.55 ->
 // 0.47 for 67 residues on 8 workgroups, 1.03 -> 0.95 for 500 on 32.)
 struct Ctx : Team {

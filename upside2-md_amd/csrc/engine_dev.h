@@ -53,8 +53,10 @@ enum EdgeKind : int {
 // by the positions alone.  The transposed rows list, for each i2, the slots
 // naming it, in the same kind of canonical order.  Both orders are canonical, so every sum over slots (energies,
 // sensitivity gathers) runs in a fixed order: bit-reproducible, no float
-// atomics.  Per-slot derivatives are stored structure-of-arrays: component q
-// of slot s at d1[q*ecap + s].
+// atomics.  Per-slot derivatives of side 1, which gathers read in slot order,
+// are stored as a structure of arrays: component q of slot s at d1[q*ecap + s];
+// those of side 2, read by transposed rows in any order, lie together:
+// d2[s*ddim2 + q].
 struct PairGraph {
     int kind;
     int sym;
@@ -85,10 +87,10 @@ struct PairGraph {
     int row;               // int ecap  row of each slot
     int toff;              // int n2+1  transposed row offsets
     int tslot;             // int ecap  slot of each transposed entry
-    int tmp;               // int ecap  transposed entries in arrival order during a rebuild
-    int tcur;              // int max(n1,n2)+1  cursors during a rebuild
+    int tmp;               // int ecap  rows' slabs, then transposed entries in arrival order, during a rebuild
+    int tcur;              // int max(n1,n2)+1  unused: keeps the place of what follows, as saved states have it
     int val;               // float ecap   edge value (0 when inactive)
-    int d1, d2;            // float ddim1*ecap, ddim2*ecap (SoA)
+    int d1, d2;            // float ddim1*ecap (SoA), ddim2*ecap (AoS)
     int esens;             // float ecap   edge sensitivity
     int act;               // int ecap     active flag
     int state;             // int [0]=cache valid, [1]=overflow, [2]=rebuild count, [3]=slots
