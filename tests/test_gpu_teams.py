@@ -81,3 +81,71 @@ def test_evaluations_in_threads(ue, chain_file):
     for t in threads:
         t.join()
     assert not bad
+
+
+@pytest.mark.parametrize("n_res", [26, 126])
+@pytest.mark.parametrize("spins", [0, 2, 4, 8, 30])
+def test_evaluation_whose_team_cannot_meet(ue, chain_file, monkeypatch, capfd, n_res, spins):
+    """Barriers that give up after a few polls (0: at the first workgroup that
+    is not there yet; more: somewhere in the evaluation, or not at all): every
+    workgroup leaves, and the evaluation is repeated on one.  Same bits."""
+    import upconfig
+    path = chain_file(n_res, 11)
+    rng = np.random.default_rng(n_res)
+    pos = [np.ascontiguousarray(upconfig.random_initial_config(n_res, rng), np.float32) for _ in range(4)]
+    with monkeypatch.context() as m:
+        m.setenv("UPSIDE_TEAM", "1")
+        one = ue.Upside(path, quiet=True)
+    with monkeypatch.context() as m:
+        m.setenv("UPSIDE_BARRIER_SPINS", str(spins))
+        eng = ue.Upside(path, quiet=True)
+    want = [(one.deriv(p), one.energy(p)) for p in pos]
+    capfd.readouterr()
+    # 64 evaluations on one workgroup, then the team's second try
+    for k in range(68 if spins == 0 else 4):
+        d, e = want[k % 4]
+        np.testing.assert_array_equal(eng.deriv(pos[k % 4]), d)
+        if k < 4:
+            np.testing.assert_allclose(eng.energy(pos[k]), e, rtol=1e-5)
+    said = capfd.readouterr().err
+    if spins == 0:
+        assert "the next 64 evaluations" in said and "the next 128 evaluations" in said
+
+
+@pytest.mark.parametrize("spins", [0, 8])
+def test_run_whose_team_cannot_meet(ue, chain_file, monkeypatch, spins):
+    """A run on such teams is an error, or (enough polls) the run; after the
+    error the batch evaluates and runs like a new one."""
+    path = chain_file(56, 11)
+    monkeypatch.setenv("UPSIDE_BARRIER_SPINS", str(spins))
+    b = ue.Batch([path], [0.85], seed=4)
+    if b.max_team() < 8:
+        pytest.skip("no team of this size fits")
+    start = b.pos(0), b.mom(0)
+    b.set_team(8)
+    try:
+        b.run(4)
+        assert spins > 0
+    except RuntimeError:
+        pass
+    b.set_team(1)
+    b.set_pos(0, start[0])
+    b.set_mom(0, start[1])
+    new = ue.Batch([path], [0.85], seed=4)
+    np.testing.assert_array_equal(b.energies(), new.energies())
+    np.testing.assert_array_equal(b.deriv(0), new.deriv(0))
+
+
+def test_exchange_whose_systems_cannot_meet(ue, chain_file, monkeypatch):
+    """The same for the barrier of all systems around a replica exchange."""
+    path = chain_file(30, 11)
+    monkeypatch.setenv("UPSIDE_BARRIER_SPINS", "0")
+    temps = [0.8, 0.85, 0.9, 0.95]
+    b = ue.Batch([path] * 4, temps, seed=4)
+    start = [b.pos(s) for s in range(4)]
+    b.set_replica_exchange(2, [[(0, 1), (2, 3)], [(1, 2)]])
+    with pytest.raises(RuntimeError):
+        b.run_logged(6, 0)
+    for s in range(4):
+        b.set_pos(s, start[s])
+    np.testing.assert_array_equal(b.energies(), ue.Batch([path] * 4, temps, seed=4).energies())

@@ -118,8 +118,9 @@ struct Team {
     unsigned long long bar_next;  // count that opens this workgroup's next barrier on `bar`
     int tpar;          // buffer parity of the next reduction
     int rank, G;       // workgroup rank in the team, team size (rank is the fourth word: sync_store)
-    int gtid, gsize;   // thread in the team, team threads
+    int gsize;         // team threads
     int err;           // int arena offset of the error word this team sets
+    lp<int> lost;      // LDS word of the workgroup: a wait of its ended without the others (team_sync)
     gp<unsigned long long> bar;   // arrival counter
     gp<float> tred;    // reduction scratch, 2 buffers of G floats
     unsigned long long* prof;  // wall-clock accumulators (null: profiling off)
@@ -148,7 +149,8 @@ struct Ctx : Team {
     int cur_op;            // program op being run (team barriers are counted per op while profiling)
     int local;             // the whole team runs on one XCD (shares one L2)
     int bp_layout;         // where rotamer solves run (see bp_on_one_wg)
-    int tid;               // thread in the workgroup
+    unsigned spin_limit;   // RunArgs::spin_limit
+    int tid, gtid;         // thread in the workgroup, in the team (not kept in LDS)
 };
 
 // Threads of a team are numbered wave by wave across its workgroups, so that a
@@ -158,20 +160,32 @@ struct Ctx : Team {
 // step, an evaluation of 101 residues 1432 -> 1371 us).
 __device__ __forceinline__ int team_tid(int rank, int G, int tid) { return ((tid >> 6) * G + rank) * 64 + (tid & 63); }
 
+// sync_store keeps the words that barriers advance as the first four.
+static_assert(__builtin_offsetof(Team, bar_next) == 0 && __builtin_offsetof(Team, tpar) == 8 &&
+              __builtin_offsetof(Team, rank) == 12, "first 16 bytes of a context");
+
 // The context in LDS, one copy per wave (no wave waits for another's): the
 // current one, the whole team's while the current one is narrowed to a part of
 // it, and the next barrier counts of the parts this workgroup belongs to.
-constexpr int CTX_WORDS = (sizeof(Ctx) + 15) / 16 * 4;
+constexpr int CTX_BYTES = sizeof(Ctx) - 2 * sizeof(int);
+constexpr int CTX_WORDS = (CTX_BYTES + 15) / 16 * 4;
 constexpr int CTX_ROOT = CTX_WORDS, CTX_NEXT = 2 * CTX_WORDS;
 constexpr int CTX_WAVE = 2 * CTX_WORDS + 8;
+constexpr int CTX_LOST = NWAVE * CTX_WAVE;  // Team::lost, after the waves' copies
+constexpr int CTX_TOTAL = CTX_LOST + 4;
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ lp<int> ctx_wave(lp<int> mem) { return mem + (int)(threadIdx.x >> 6) * CTX_WAVE; }
 __device__ __forceinline__ void ctx_store(lp<int> mem, const Ctx& c, int at = 0) {
     int w[CTX_WORDS] = {};
-    __builtin_memcpy(w, &c, sizeof(Ctx));
+    __builtin_memcpy(w, &c, CTX_BYTES);
     lp<i32x4> m = (lp<i32x4>)(ctx_wave(mem) + at);
 #pragma unroll
     for (int k = 0; k < CTX_WORDS / 4; ++k) m[k] = i32x4{w[4 * k], w[4 * k + 1], w[4 * k + 2], w[4 * k + 3]};
+}
+// A workgroup whose team cannot meet ends here (all its waves: the word is set
+// between two workgroup barriers, and every wave reads it at the same places).
+__device__ __forceinline__ void leave_if(int lost) {
+    if (uni(lost)) __builtin_amdgcn_endpgm();
 }
 __device__ __forceinline__ Ctx ctx_load(lp<int> mem, int at = 0) {
     int w[CTX_WORDS];
@@ -183,7 +197,7 @@ __device__ __forceinline__ Ctx ctx_load(lp<int> mem, int at = 0) {
         for (int q = 0; q < 4; ++q) w[4 * k + q] = uni(v[q]);
     }
     Ctx c;
-    __builtin_memcpy(&c, w, sizeof(Ctx));
+    __builtin_memcpy(&c, w, CTX_BYTES);
     c.tid = (int)threadIdx.x;
     c.gtid = team_tid(c.rank, c.G, c.tid);
     return c;
@@ -221,21 +235,40 @@ __device__ __forceinline__ void pacc(const Ctx& c, int slot, unsigned long long 
 // after the wait, with plain loads, is served by the shared L2 one CU after
 // the other (a barrier of 2, 8, 16, 32 workgroups and reads of three others'
 // data: 1.07, 1.38, 1.82, 2.92 us with it; 0.95, 0.92, 0.93, 1.12 without).
-//   The wait is bounded: after ~1 s of spinning the workgroup records a
-// timeout and proceeds, so a launch always drains; the host then reports the
-// run as failed.
-constexpr unsigned BAR_SPIN_LIMIT = 1u << 24;
+//   The wait is bounded (RunArgs::spin_limit): a workgroup that has polled that
+// often, or sees that another of its team gave up, records a timeout and closes
+// the counter for good (BAR_CLOSED), and so any other that it comes to
+// (enter_sub, leave_sub): nobody passes a barrier on account of what it does
+// without the others.  It goes on, waiting for nobody, to the next place where
+// it reads `lost`, and ends there: where integers that others should have
+// written would be taken as an index, an offset or a count (the pair lists,
+// ahead of the edges, and the edges of a solve: list_sync, team_or,
+// team_exscan; the exchange), and at the start of an evaluation.  In between it
+// may compute floats from what others had not finished, which become an index
+// nowhere there but through a clamp.  So a launch always drains, inside of its
+// arrays; the host then reports the run as failed.  (Reading the word at every
+// barrier, or at the start of every phase, costs up to 6 % of an evaluation of
+// 10 residues or a step of 67.)
 
 // s_waitcnt immediate: vmcnt(0), expcnt and lgkmcnt not waited on.
 constexpr int WAIT_VMEM = 0x0F70;
 
+// Set in a counter: as a signed number it is below every count (counts are
+// compared signed), whoever still arrives.
+constexpr unsigned long long BAR_CLOSED = 1ull << 63;
+
 // Count that opens the first barrier of a team of G on counter `bar`, read
 // before this workgroup's first arrival: fewer than G arrivals of that
 // barrier can precede it (it cannot open without this workgroup), so the
-// count rounded down to a multiple of G is the base.
+// count rounded down to a multiple of G is the base.  (A closed counter: any
+// count that it cannot reach.)
 __device__ __forceinline__ unsigned long long bar_first(gp<unsigned long long> bar, int G) {
-    const unsigned long long v = uni64(__hip_atomic_load(bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    const unsigned long long v = uni64(__hip_atomic_load(bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) & ~BAR_CLOSED;
     return (v / (unsigned long long)G + 1ull) * (unsigned long long)G;
+}
+
+__device__ __forceinline__ void close_bar(Ctx& c) {
+    (void)__hip_atomic_fetch_or(c.bar, BAR_CLOSED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 __device__ __forceinline__ void team_sync(Ctx& c) {
@@ -249,13 +282,16 @@ __device__ __forceinline__ void team_sync(Ctx& c) {
             if (!c.local) __threadfence();
             (void)__hip_atomic_fetch_add(c.bar, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             unsigned spins = 0;
-            while (__hip_atomic_load(c.bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
+            while ((long long)__hip_atomic_load(c.bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < (long long)target) {
                 __builtin_amdgcn_s_sleep(2);
-                // after one timeout anywhere in the team no barrier waits again,
-                // so the launch drains quickly
-                if (++spins > BAR_SPIN_LIMIT ||
-                    __hip_atomic_load(c.bar_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) {
+                // after one timeout anywhere in the team no barrier waits long,
+                // so the launch drains quickly (a poll takes 241 ns with a look
+                // at the flag, 190 without)
+                if (__builtin_expect(++spins > c.spin_limit || (spins % 16 == 0 &&
+                    __hip_atomic_load(c.bar_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u), 0)) {
                     __hip_atomic_store(c.bar_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    close_bar(c);
+                    *c.lost = 1;
                     break;
                 }
             }
@@ -268,6 +304,12 @@ __device__ __forceinline__ void team_sync(Ctx& c) {
             __hip_atomic_fetch_add(c.prof + c.pbase + PROF_EXTRA + c.cur_op, 1ull, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
     }
+}
+
+// A barrier after which offsets or counts that others wrote are read.
+__device__ __forceinline__ void list_sync(Ctx& c) {
+    team_sync(c);
+    if (c.G > 1) leave_if(*c.lost);
 }
 
 // Drop the CU's L1, which may hold lines of the arenas from before other
@@ -317,12 +359,14 @@ __device__ __forceinline__ void enter_sub(lp<int> mem, Ctx& c, int kind, gp<int>
     c.tred += p.buf * 2 * MAX_TEAM;
     c.tpar = 0;
     c.prof = c.rank == 0 ? prof : nullptr;
+    if (uni(*c.lost) && c.tid == 0) close_bar(c);
 }
 // Back to the whole team.
 __device__ __forceinline__ void leave_sub(lp<int> mem, Ctx& c, int kind) {
     sub_next_put(mem, kind, c.bar_next);
     c = ctx_load(mem, CTX_ROOT);
     ctx_store(mem, c);
+    if (uni(*c.lost) && c.tid == 0) close_bar(c);
 }
 
 // XCD of the calling workgroup (hardware register XCC_ID).
@@ -406,7 +450,9 @@ __device__ __forceinline__ float team_max(Ctx& c, float v) {
 __device__ __forceinline__ int team_or(Ctx& c, int v) {
     int t = uni(__syncthreads_or(v));
     if (c.G == 1) return t;
-    return __any(team_partial(c, t ? 1.f : 0.f) > 0.f) ? 1 : 0;
+    const float x = team_partial(c, t ? 1.f : 0.f);
+    leave_if(*c.lost);  // the answer decides whether lists are built
+    return __any(x > 0.f) ? 1 : 0;
 }
 
 // In-place exclusive scan of the ints a[0..n) (any memory); returns the
@@ -454,6 +500,7 @@ __device__ __forceinline__ int team_exscan(Ctx& c, P a, int n) {
     if (c.G == 1) return tot;
     const int lane = c.tid & 63;
     const int part = __float_as_int(team_partial(c, __int_as_float(tot)));
+    leave_if(*c.lost);
     const int x = lane < c.G ? part : 0;
     int v = x;  // inclusive scan over the ranks
     for (int o = 1; o < 64; o <<= 1) {
@@ -463,7 +510,7 @@ __device__ __forceinline__ int team_exscan(Ctx& c, P a, int n) {
     const int all = __builtin_amdgcn_readlane(v, 63);
     const int before = __builtin_amdgcn_readlane(v - x, c.rank);
     for (int i = b + c.tid; i < e; i += NT) a[i] += before;
-    team_sync(c);
+    list_sync(c);
     return all;
 }
 

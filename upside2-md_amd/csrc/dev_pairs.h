@@ -482,7 +482,7 @@ __device__ __forceinline__ void pg_order_columns(Ctx& c, GraphC& G, int n2) {
         }
         jb = je;
     }
-    team_sync(c);
+    list_sync(c);
 }
 
 // Latency bound: a chain of short phases (scan, sums of offsets, fill, columns)
@@ -572,7 +572,7 @@ __device__ __forceinline__ bool pg_rebuild(Ctx& c, GraphC& G) {
         c.I[G.state + 2] += 1;
         c.I[G.state + 3] = E;
     }
-    team_sync(c);
+    list_sync(c);
     pg_order_columns(c, G, n2);
     pacc(c, PROF_RB_MAP, t0);
     return true;

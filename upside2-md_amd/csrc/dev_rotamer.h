@@ -188,7 +188,7 @@ __device__ __forceinline__ bool rot_rebuild(Ctx& c, GraphC& G, RotC& R) {
         return false;
     }
     if (c.gtid == 0) v.stats[5] = v.coff[n];  // candidate count
-    team_sync(c);
+    list_sync(c);
     return true;
 }
 
@@ -308,7 +308,7 @@ __device__ __forceinline__ void rot_fill(Ctx& c, GraphC& G, RotC& R) {
             if (x < R.n_node && gl == 0) v.ninc[x] = k - t0;
         }
     }
-    team_sync(c);
+    list_sync(c);
 }
 
 // Belief-propagation state of one solve.  Messages are updated in place (an

@@ -333,7 +333,10 @@ struct RunArgs {
     int bp_klocal;
     MlpDev mlp;            // warm-start network (bp_mode 2)
     RexDev rex;            // replica exchange between rounds of this launch
+    unsigned spin_limit;   // polls after which a barrier among workgroups gives up (see team_sync)
 };
+// 192 ns a poll: about 3 s.
+constexpr unsigned BAR_SPIN_LIMIT = 1u << 24;
 
 // What the host reads after a launch, one record of STATUS_WORDS + n_pot words
 // per system in pinned host memory (status_kernel): [0] a list outgrew its

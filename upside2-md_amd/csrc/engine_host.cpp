@@ -1929,6 +1929,7 @@ struct Batch {
         const float time = 3.f * dt * (float)(nr + 1);
         for (auto& s : sys) s.temperature = (float)anneal_temp((double)s.temp0, (double)time);
     }
+    unsigned spin_limit = BAR_SPIN_LIMIT;  // RunArgs::spin_limit
     bool profile = false;
     vector<unsigned long long*> prof;
     // wall-clock ticks per op, fixed slots, then team barriers per op (+1: outside the ops)
@@ -2084,6 +2085,8 @@ struct Batch {
             double v = std::atof(e);
             if (v > 0.0 && v <= 64.0) cap_scale = v;
         }
+        // UPSIDE_BARRIER_SPINS: polls after which a barrier gives up (0: at the first one not yet met)
+        if (const char* e = std::getenv("UPSIDE_BARRIER_SPINS")) spin_limit = (unsigned)std::strtoul(e, nullptr, 10);
         hip_check(hipStreamCreate(&stream), "stream");
         hip_check(hipEventCreate(&ev0), "event");
         hip_check(hipEventCreate(&ev1), "event");
@@ -2223,10 +2226,11 @@ struct Batch {
         teams.clear();
     }
 
-    // After a barrier timeout: one workgroup per system from here on, nothing
-    // kept of what the abandoned launch left (lists, error words).
-    void drop_teams() {
-        set_team(1);
+    // After a barrier timeout: nothing of what the abandoned launch left is
+    // read again (barrier words, lists, error words; the kernel has stored
+    // nothing outside of its own arrays).
+    void forget_launch() {
+        reset_barriers();
         for (auto& sy : sys) {
             const Topology& T = sy.prog->T;
             hip_check(hipMemset(sy.iarena + T.err, 0, (2 + MAX_LANES) * sizeof(int)), "error words");
@@ -2359,6 +2363,7 @@ struct Batch {
         a.bp_residual = bp_residual;
         a.bp_budget = bp_budget;
         a.bp_klocal = bp_klocal;
+        a.spin_limit = spin_limit;
         if (mlp) a.mlp = mlp->dev;
         pots_fresh = false;
         hip_check(hipEventRecord(ev0, stream), "event");
@@ -2376,7 +2381,10 @@ struct Batch {
                 const unsigned* w = (const unsigned*)status_of(s) + STATUS_TEAM;
                 auto word64 = [&](int k) { return (unsigned long long)w[k] | ((unsigned long long)w[k + 1] << 32); };
                 const unsigned long long g = (unsigned long long)team_of(s), lo = g / 2, hi = g - g / 2;
-                if (w[2]) throw BarrierTimeout("team barrier wait timed out: results of this run are void");
+                if (w[2]) {
+                    forget_launch();
+                    throw BarrierTimeout("team barrier wait timed out: results of this run are void");
+                }
                 bool quarters_ok = true;
                 if (sys[s].prog->n_lanes == 4 && g >= 8)
                     for (unsigned long long j = 0; j < 4; ++j)
@@ -2647,13 +2655,23 @@ using namespace upside;
 struct DerivEngine {
     Batch batch;
     bool evaluated = false;   // an evaluation has set every node's outputs and sensitivities
+    int team = 1;             // workgroups of an evaluation
+    int alone = 0;            // evaluations left on one workgroup since a team could not meet
+    int pause = 0;            // how many they were
 
     void evaluate(const float* pos, float* deriv) {
+        if (alone > 0 && --alone == 0) batch.set_team(team);
         try {
             batch.evaluate_at(pos, deriv);
+            if (!alone) pause = 0;
         } catch (const BarrierTimeout&) {
-            // another process's team holds part of the XCD: one workgroup waits for nobody
-            batch.drop_teams();
+            // another launch holds part of the XCD: one workgroup waits for
+            // nobody.  The team is tried again after 64 evaluations, then 128, ...
+            team = batch.team;
+            alone = pause = std::min(std::max(2 * pause, 64), 4096);
+            fprintf(stderr, "WARNING: the %d workgroups of an evaluation could not meet; the next %d evaluations "
+                    "run on one\n", team, alone);
+            batch.set_team(1);
             batch.evaluate_at(pos, deriv);
         }
         evaluated = true;
@@ -3176,6 +3194,8 @@ DerivEngine* construct_deriv_engine(int n_atom, const char* potential_file, bool
     if (e->batch.sys[0].prog->T.n_atom != n_atom) fail("n_atom mismatch");
     if (!std::getenv("UPSIDE_TEAM"))
         e->batch.set_team(std::min(DerivEngine::eval_team(e->batch.sys[0].prog->T), e->batch.max_team()));
+    // an evaluation can be repeated on one workgroup: it need not wait as long as a run (0.8 s)
+    if (!std::getenv("UPSIDE_BARRIER_SPINS")) e->batch.spin_limit = BAR_SPIN_LIMIT / 4;
     return e.release();
     ABI_CATCH(nullptr)
 }

@@ -1029,6 +1029,7 @@ __device__ __forceinline__ bool compute(lp<int> mem, gp<int> words, int mode) {
     const int ng = S.n_germ, nd = S.n_germ + S.n_deriv;
     {
         Ctx c = ctx_load(mem);
+        leave_if(mem[CTX_LOST]);
         c.cur_op = nd;  // outside the ops
         for (int r = 0; r < S.sens_zero_cnt; ++r) {
             cp<int> zr = cmem((const int*)S.iarena) + S.sens_zero + 2 * r;  // written once, by the host
@@ -1354,9 +1355,10 @@ __device__ __forceinline__ float total_potential(Ctx& c, SysC& S) {
 // Barrier over every workgroup of the launch that takes part in replica
 // exchange (teams on different XCDs: device-scope fences on both sides), on a
 // monotonic arrival counter as team_sync.  Bounded: a timeout sets the flag,
-// which the host turns into an error, and no later wait blocks.
+// which the host turns into an error, and the workgroups leave.
 __device__ __forceinline__ void grid_sync(Ctx& c, UPS_CONST const RexDev& x) {
     __syncthreads();
+    leave_if(*c.lost);
     if (c.tid == 0) {
         __threadfence();
         unsigned long long old = __hip_atomic_fetch_add(x.grid_bar, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1364,15 +1366,17 @@ __device__ __forceinline__ void grid_sync(Ctx& c, UPS_CONST const RexDev& x) {
         unsigned spins = 0;
         while (__hip_atomic_load(x.grid_bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
             __builtin_amdgcn_s_sleep(2);
-            if (++spins > BAR_SPIN_LIMIT ||
+            if (++spins > c.spin_limit ||
                 __hip_atomic_load(x.grid_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) {
                 __hip_atomic_store(x.grid_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                *c.lost = 1;
                 break;
             }
         }
         __threadfence();
     }
     __syncthreads();
+    leave_if(*c.lost);
 }
 
 // One replica-exchange attempt after `done` completed rounds (see RexDev):
@@ -1477,6 +1481,9 @@ __device__ __forceinline__ void engine_body(SysDesc* systems, lp<float> red, lp<
     c.S = &S;
     c.A.p = gmem(S.arena); c.I.p = gmem(S.iarena); c.CF = gmem(S.cf); c.CI = gmem(S.ci);
     c.red = red; c.ired = ired; c.lds = lds;
+    c.lost = mem + CTX_LOST;
+    if (threadIdx.x == 0) *c.lost = 0;
+    __syncthreads();
     c.tid = (int)threadIdx.x;
     c.prof = rank == 0 ? S.prof : nullptr;
     c.pbase = S.n_germ + S.n_deriv;
@@ -1502,6 +1509,7 @@ __device__ __forceinline__ void engine_body(SysDesc* systems, lp<float> red, lp<
     c.tred = gmem(S.arena) + S.tred;
     c.tpar = 0;
     c.bp_layout = args.bp_layout;
+    c.spin_limit = args.spin_limit;
     c.args = &args;
     team_place(c, words + 4);
     ctx_store(mem, c);
@@ -1573,11 +1581,13 @@ __device__ __forceinline__ void engine_body(SysDesc* systems, lp<float> red, lp<
     }
 }
 
+static_assert((LDS_FLOATS + CTX_TOTAL + 2 * NWAVE) * 4 <= 160 * 1024, "LDS of a workgroup");
+
 // Integration rounds (args.n_round > 0).
 __global__ void __launch_bounds__(NT) engine_step_kernel(SysDesc* systems, RunArgs args) {
     __shared__ float red[NWAVE];
     __shared__ int ired[NWAVE];
-    __shared__ __attribute__((aligned(16))) int ctx[NWAVE * CTX_WAVE];
+    __shared__ __attribute__((aligned(16))) int ctx[CTX_TOTAL];
     extern __shared__ float lds[];
     engine_body(systems, (lp<float>)red, (lp<int>)ired, (lp<int>)ctx, (lp<float>)lds);
 }
@@ -1586,7 +1596,7 @@ __global__ void __launch_bounds__(NT) engine_step_kernel(SysDesc* systems, RunAr
 __global__ void __launch_bounds__(NT) engine_eval_kernel(SysDesc* systems, RunArgs args) {
     __shared__ float red[NWAVE];
     __shared__ int ired[NWAVE];
-    __shared__ __attribute__((aligned(16))) int ctx[NWAVE * CTX_WAVE];
+    __shared__ __attribute__((aligned(16))) int ctx[CTX_TOTAL];
     extern __shared__ float lds[];
     engine_body(systems, (lp<float>)red, (lp<int>)ired, (lp<int>)ctx, (lp<float>)lds);
 }
