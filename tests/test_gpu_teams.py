@@ -149,3 +149,25 @@ def test_exchange_whose_systems_cannot_meet(ue, chain_file, monkeypatch):
     for s in range(4):
         b.set_pos(s, start[s])
     np.testing.assert_array_equal(b.energies(), ue.Batch([path] * 4, temps, seed=4).energies())
+
+
+def test_every_evaluation_in_threads(ue, chain_file):
+    """As test_evaluations_in_threads, where an evaluation that fails is a
+    failure too: all of them are counted."""
+    import concurrent.futures
+
+    import upconfig
+    path = chain_file(126, 11)
+    rng = np.random.default_rng(8)
+    pos = [np.ascontiguousarray(upconfig.random_initial_config(126, rng), np.float32) for _ in range(4)]
+    ref = ue.Upside(path, quiet=True)
+    want = [ref.deriv(p) for p in pos]
+    engines = [ue.Upside(path, quiet=True) for _ in range(4)]
+
+    def work(k):
+        for i in range(20):
+            np.testing.assert_array_equal(engines[k].deriv(pos[(i + k) % 4]), want[(i + k) % 4])
+        return 20
+
+    with concurrent.futures.ThreadPoolExecutor(4) as pool:
+        assert sum(f.result() for f in [pool.submit(work, k) for k in range(4)]) == 80
