@@ -229,12 +229,12 @@ __device__ __forceinline__ void pacc(const Ctx& c, int slot, unsigned long long 
 // starts polling.  A stale poll can only prolong a wait.
 //   Memory ordering: a team spread over XCDs (separate L2s) needs
 // device-scope fences (write back L2 before arriving, invalidate after the
-// wait).  A team on one XCD shares its L2: every wave waits for its stores to
-// be acknowledged by L2 before the workgroup barrier, and loads of what others
-// wrote go to L2 (ap).  Nothing is invalidated: a device-scope invalidate of L1
-// after the wait, with plain loads, is served by the shared L2 one CU after
-// the other (a barrier of 2, 8, 16, 32 workgroups and reads of three others'
-// data: 1.07, 1.38, 1.82, 2.92 us with it; 0.95, 0.92, 0.93, 1.12 without).
+// wait).  A team on one XCD shares its L2, and loads of what others wrote go to
+// L2 (ap).  Either way every wave waits for its stores to be acknowledged by L2
+// before the workgroup barrier, which does not wait for them.  On one XCD
+// nothing is invalidated: a device-scope invalidate of L1 after the wait, with
+// plain loads, is served by the shared L2 one CU after the other (a barrier of
+// 2, 8, 16, 32 workgroups and reads of three others' data: 1.07, 1.38, 1.82, 2.92 us with it; 0.95, 0.92, 0.93, 1.12 without).
 //   The wait is bounded (RunArgs::spin_limit): a workgroup that has polled that
 // often, or sees that another of its team gave up, records a timeout and closes
 // the counter for good (BAR_CLOSED), and so any other that it comes to
@@ -273,7 +273,7 @@ __device__ __forceinline__ void close_bar(Ctx& c) {
 
 __device__ __forceinline__ void team_sync(Ctx& c) {
     // every wave's stores acknowledged by L2 before the team can observe the arrival
-    if (c.G > 1 && c.local) __builtin_amdgcn_s_waitcnt(WAIT_VMEM);
+    if (c.G > 1) __builtin_amdgcn_s_waitcnt(WAIT_VMEM);
     __syncthreads();
     if (c.G > 1) {
         const unsigned long long target = c.bar_next;
@@ -310,6 +310,34 @@ __device__ __forceinline__ void team_sync(Ctx& c) {
 __device__ __forceinline__ void list_sync(Ctx& c) {
     team_sync(c);
     if (c.G > 1) leave_if(*c.lost);
+}
+
+// Barrier over every workgroup of the launch that takes part in replica
+// exchange (teams on different XCDs: device-scope fences on both sides), on a
+// monotonic arrival counter as team_sync.  Bounded: a timeout sets the flag,
+// which the host turns into an error, and the workgroups leave.
+__device__ __forceinline__ void grid_sync(Ctx& c, UPS_CONST const RexDev& x) {
+    __builtin_amdgcn_s_waitcnt(WAIT_VMEM);  // every wave's: thread 0's fence waits for its own wave's stores
+    __syncthreads();
+    leave_if(*c.lost);
+    if (c.tid == 0) {
+        __threadfence();
+        unsigned long long old = __hip_atomic_fetch_add(x.grid_bar, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        unsigned long long target = (old / (unsigned long long)x.n_wg + 1ull) * (unsigned long long)x.n_wg;
+        unsigned spins = 0;
+        while (__hip_atomic_load(x.grid_bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
+            __builtin_amdgcn_s_sleep(2);
+            if (++spins > c.spin_limit ||
+                __hip_atomic_load(x.grid_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) {
+                __hip_atomic_store(x.grid_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                *c.lost = 1;
+                break;
+            }
+        }
+        __threadfence();
+    }
+    __syncthreads();
+    leave_if(*c.lost);
 }
 
 // Drop the CU's L1, which may hold lines of the arenas from before other

@@ -1352,33 +1352,6 @@ __device__ __forceinline__ float total_potential(Ctx& c, SysC& S) {
     return t;
 }
 
-// Barrier over every workgroup of the launch that takes part in replica
-// exchange (teams on different XCDs: device-scope fences on both sides), on a
-// monotonic arrival counter as team_sync.  Bounded: a timeout sets the flag,
-// which the host turns into an error, and the workgroups leave.
-__device__ __forceinline__ void grid_sync(Ctx& c, UPS_CONST const RexDev& x) {
-    __syncthreads();
-    leave_if(*c.lost);
-    if (c.tid == 0) {
-        __threadfence();
-        unsigned long long old = __hip_atomic_fetch_add(x.grid_bar, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        unsigned long long target = (old / (unsigned long long)x.n_wg + 1ull) * (unsigned long long)x.n_wg;
-        unsigned spins = 0;
-        while (__hip_atomic_load(x.grid_bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
-            __builtin_amdgcn_s_sleep(2);
-            if (++spins > c.spin_limit ||
-                __hip_atomic_load(x.grid_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) {
-                __hip_atomic_store(x.grid_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                *c.lost = 1;
-                break;
-            }
-        }
-        __threadfence();
-    }
-    __syncthreads();
-    leave_if(*c.lost);
-}
-
 // One replica-exchange attempt after `done` completed rounds (see RexDev):
 // all teams of the launch, each having evaluated its potential.  The decisions follow attempt_swaps
 // (src/main.cpp:243-316): criterion 0 keeps a swap unless the change of the
