@@ -224,7 +224,7 @@ __device__ __forceinline__ void pacc(const Ctx& c, int slot, unsigned long long 
 // multiple of G.  Nothing is reset between barriers, and the counter is a
 // multiple of G between launches (the host zeroes it when the team size
 // changes).  Every workgroup keeps the count that opens its next barrier
-// (bar_base at the start, then + G per barrier), so its arrival is a
+// (bar_first at the start, then + G per barrier), so its arrival is a
 // no-return atomic: it does not wait for the counter's old value before it
 // starts polling.  A stale poll can only prolong a wait.
 //   Memory ordering: a team spread over XCDs (separate L2s) needs
@@ -234,7 +234,8 @@ __device__ __forceinline__ void pacc(const Ctx& c, int slot, unsigned long long 
 // before the workgroup barrier, which does not wait for them.  On one XCD
 // nothing is invalidated: a device-scope invalidate of L1 after the wait, with
 // plain loads, is served by the shared L2 one CU after the other (a barrier of
-// 2, 8, 16, 32 workgroups and reads of three others' data: 1.07, 1.38, 1.82, 2.92 us with it; 0.95, 0.92, 0.93, 1.12 without).
+// 2, 8, 16, 32 workgroups and reads of three others' data: 1.07, 1.38, 1.82,
+// 2.92 us with it; 0.95, 0.92, 0.93, 1.12 without).
 //   The wait is bounded (RunArgs::spin_limit): a workgroup that has polled that
 // often, or sees that another of its team gave up, records a timeout and closes
 // the counter for good (BAR_CLOSED), and so any other that it comes to

@@ -11,6 +11,7 @@
 // d loss / d delta_r = (p_r - t_r) / n_rows.
 #include <hip/hip_runtime.h>
 #include <cstdio>
+#include <type_traits>
 #include "warmstart.h"
 
 namespace upside {
@@ -91,14 +92,25 @@ __device__ __forceinline__ void store_t(__bf16* T, int blk, f32x4 v, int wave) {
     for (int i = 0; i < 4; ++i) T[(blk * 16 + 4 * g + i) * TR_LD + wave * 16 + c] = (__bf16)v[i];
 }
 
+// Bits ob * 4 + i of the entries that a ReLU kept.
+__device__ __forceinline__ unsigned relu_mask(f32x4 a, int ob) {
+    unsigned m = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) m |= (a[i] > 0.f ? 1u : 0u) << (ob * 4 + i);
+    return m;
+}
+
 // Partial gradients of the loss over the rows [row0, row0 + n_batch) (taken
 // modulo n_rows) handled by this workgroup: chunks b, b + gridDim.x, ... of
 // TR_CHUNK rows, in that order, two at a time.  partial[blockIdx.x][TR_PARTIAL].
 //   Bound by latency: 64 rows are a few hundred matrix instructions, so a
 // workgroup's time is its chain of dependent products and LDS trips.  Hence two
 // chunks side by side, eight waves on the 82 blocks of the weight gradients,
-// and conflict-free LDS rows.  A training step on 4096 rows (with the Adam
-// kernel and no wait between steps): 78 us before, 42 now.
+// and conflict-free LDS rows; what a workgroup does not have (a second chunk:
+// its rows, their part of the products and sums) is left out.  A training step
+// on 4096 rows (with the Adam kernel and no wait between steps) 35 us, 78 with
+// one chunk at a time; on 50 to 2048 rows 24 to 28 us, 40 while the waves of a
+// missing chunk worked on zeros and 77 registers spilled.
 __global__ void __launch_bounds__(TR_THREADS) mlp_train_partial_kernel(MlpDev w, const float* feat,
                                                                         const float* tgt, int n_rows, int row0,
                                                                         int n_batch, float inv_n, float* partial) {
@@ -122,76 +134,96 @@ __global__ void __launch_bounds__(TR_THREADS) mlp_train_partial_kernel(MlpDev w,
     const int n_chunks = (n_batch + TR_CHUNK - 1) / TR_CHUNK;
     for (int ch = blockIdx.x; ch < n_chunks; ch += 2 * gridDim.x) {
         // one 16-row tile per wave: rows of the batch, wrapped into the data
-        // (a second chunk past the batch has no live rows)
+        // (without a second chunk the waves of its rows help with the products)
+        const bool two = ch + (int)gridDim.x < n_chunks;
+        const bool mine = two || wave < TR_CHUNK_WAVES;
         const int tb = (ch + (wave / TR_CHUNK_WAVES) * gridDim.x) * TR_CHUNK +
                        (wave % TR_CHUNK_WAVES) * 16;   // batch position of the tile's first row
         const int bpos = tb + c;
         const bool live = bpos < n_batch;
         const int row = live ? (row0 + bpos) % n_rows : 0;
-        // forward (as mlp_tile_forward, on this lane's wrapped row), keeping
-        // the inputs transposed in LDS for the layer-1 weight gradient
-        f32x4 h1[MLP_H / 16], h2[MLP_H / 16], y;
-        {
-            bf16x8 x;
+        // forward (as mlp_tile_forward, on this lane's wrapped row).  The bf16
+        // copies for the weight gradients go to LDS (transposed, dead rows as
+        // zeros) as they are made; of the hidden layers only the masks of their
+        // ReLUs are kept (bit ob * 4 + i), so that nothing spills.
+        if (mine) {
+            const unsigned keep = live ? ~0u : 0u;
+            unsigned m1 = 0, m2 = 0;
+            f32x4 y;
+            {
+                bf16x8 x;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) x[j] = (__bf16)(live ? feat[row * MLP_IN + 8 * g + j] : 0.f);
+                for (int j = 0; j < 8; ++j) x[j] = (__bf16)(live ? feat[row * MLP_IN + 8 * g + j] : 0.f);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) XT[(8 * g + j) * TR_LD + wave * 16 + c] = x[j];
+                for (int j = 0; j < 8; ++j) XT[(8 * g + j) * TR_LD + wave * 16 + c] = x[j];
+                bf16x8 b[MLP_H / 32], b2[MLP_H / 32];
 #pragma unroll
-            for (int ob = 0; ob < MLP_H / 16; ++ob) {
-                f32x4 a = mfma_bf16(ld_bf16x8(w.w1 + (ob * 16 + c) * MLP_IN + 8 * g), x, z4);
+                for (int kb = 0; kb < MLP_H / 32; ++kb) {
+                    f32x4 h[2];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) a[i] = fmaxf(a[i] + w.b1[ob * 16 + 4 * g + i], 0.f);
-                h1[ob] = a;
-            }
-            bf16x8 b[MLP_H / 32];
+                    for (int q = 0; q < 2; ++q) {
+                        const int ob = 2 * kb + q;
+                        f32x4 a = mfma_bf16(ld_bf16x8(w.w1 + (ob * 16 + c) * MLP_IN + 8 * g), x, z4);
 #pragma unroll
-            for (int kb = 0; kb < MLP_H / 32; ++kb) b[kb] = pack_blocks(h1[2 * kb], h1[2 * kb + 1]);
+                        for (int i = 0; i < 4; ++i) a[i] = fmaxf(a[i] + w.b1[ob * 16 + 4 * g + i], 0.f);
+                        m1 |= relu_mask(a, ob);
+                        store_t(H1T, ob, live ? a : z4, wave);
+                        h[q] = a;
+                    }
+                    b[kb] = pack_blocks(h[0], h[1]);
+                }
 #pragma unroll
-            for (int ob = 0; ob < MLP_H / 16; ++ob) {
+                for (int kb2 = 0; kb2 < MLP_H / 32; ++kb2) {
+                    f32x4 h[2];
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        const int ob = 2 * kb2 + q;
+                        f32x4 a = z4;
+#pragma unroll
+                        for (int kb = 0; kb < MLP_H / 32; ++kb)
+                            a = mfma_bf16(ld_bf16x8(w.w2p + (ob * 16 + c) * MLP_H + kb * 32 + 8 * g), b[kb], a);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) a[i] = fmaxf(a[i] + w.b2[ob * 16 + 4 * g + i], 0.f);
+                        m2 |= relu_mask(a, ob);
+                        store_t(H2T, ob, live ? a : z4, wave);
+                        h[q] = a;
+                    }
+                    b2[kb2] = pack_blocks(h[0], h[1]);
+                }
                 f32x4 a = z4;
 #pragma unroll
                 for (int kb = 0; kb < MLP_H / 32; ++kb)
-                    a = mfma_bf16(ld_bf16x8(w.w2p + (ob * 16 + c) * MLP_H + kb * 32 + 8 * g), b[kb], a);
+                    a = mfma_bf16(ld_bf16x8(w.w3p + c * MLP_H + kb * 32 + 8 * g), b2[kb], a);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) a[i] = fmaxf(a[i] + w.b2[ob * 16 + 4 * g + i], 0.f);
-                h2[ob] = a;
+                for (int i = 0; i < 4; ++i) a[i] += w.b3[4 * g + i];
+                y = a;
             }
-#pragma unroll
-            for (int kb = 0; kb < MLP_H / 32; ++kb) b[kb] = pack_blocks(h2[2 * kb], h2[2 * kb + 1]);
-            f32x4 a = z4;
-#pragma unroll
-            for (int kb = 0; kb < MLP_H / 32; ++kb) a = mfma_bf16(ld_bf16x8(w.w3p + c * MLP_H + kb * 32 + 8 * g), b[kb], a);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] += w.b3[4 * g + i];
-            y = a;
-        }
-        if (!live) {  // rows past the batch contribute nothing
-#pragma unroll
-            for (int ob = 0; ob < MLP_H / 16; ++ob) { h1[ob] = z4; h2[ob] = z4; }
-        }
-        // loss and output gradient (a dead row reads row 0 and is zeroed)
-        f32x4 dy;
-        {
+            // loss and output gradient (a dead row reads row 0 and is zeroed)
+            f32x4 dy;
             float lz = row_loss_grad(feat, tgt, n_rows, row, y, inv_n, dy);
             if (!live) { dy = z4; lz = 0.f; }
             if (wave < TR_CHUNK_WAVES) loss += lz;
             else lrow[(wave - TR_CHUNK_WAVES) * 64 + l] = lz;  // added below, after the first chunk's
-        }
-        // backward through layer 3: dH2^T = W3^T dY^T, masked by ReLU
-        f32x4 dh2[MLP_H / 16], dh1[MLP_H / 16];
-        {
-            const bf16x8 b = pack_blocks(dy, z4);
-#pragma unroll
-            for (int jb = 0; jb < MLP_H / 16; ++jb) {
-                f32x4 a = mfma_bf16(ld_bf16x8(w.w3tp + (jb * 16 + c) * 32 + 8 * g), b, z4);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) a[i] = h2[jb][i] > 0.f ? a[i] : 0.f;
-                dh2[jb] = a;
-            }
+            store_t(DYT, 0, dy, wave);
+            // backward through layer 3: dH2^T = W3^T dY^T, masked by ReLU, then layer 2
+            m1 &= keep;
+            m2 &= keep;
+            const bf16x8 d = pack_blocks(dy, z4);
             bf16x8 bb[MLP_H / 32];
 #pragma unroll
-            for (int kb = 0; kb < MLP_H / 32; ++kb) bb[kb] = pack_blocks(dh2[2 * kb], dh2[2 * kb + 1]);
+            for (int kb = 0; kb < MLP_H / 32; ++kb) {
+                f32x4 h[2];
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    const int jb = 2 * kb + q;
+                    f32x4 a = mfma_bf16(ld_bf16x8(w.w3tp + (jb * 16 + c) * 32 + 8 * g), d, z4);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) a[i] = (m2 >> (jb * 4 + i)) & 1u ? a[i] : 0.f;
+                    store_t(DH2T, jb, a, wave);
+                    h[q] = a;
+                }
+                bb[kb] = pack_blocks(h[0], h[1]);
+            }
 #pragma unroll
             for (int ib = 0; ib < MLP_H / 16; ++ib) {
                 f32x4 a = z4;
@@ -199,35 +231,32 @@ __global__ void __launch_bounds__(TR_THREADS) mlp_train_partial_kernel(MlpDev w,
                 for (int kb = 0; kb < MLP_H / 32; ++kb)
                     a = mfma_bf16(ld_bf16x8(w.w2tp + (ib * 16 + c) * MLP_H + kb * 32 + 8 * g), bb[kb], a);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) a[i] = h1[ib][i] > 0.f ? a[i] : 0.f;
-                dh1[ib] = a;
+                for (int i = 0; i < 4; ++i) a[i] = (m1 >> (ib * 4 + i)) & 1u ? a[i] : 0.f;
+                store_t(DH1T, ib, a, wave);
             }
         }
-        // transposed bf16 copies for the weight gradients
-#pragma unroll
-        for (int ob = 0; ob < MLP_H / 16; ++ob) {
-            store_t(H1T, ob, h1[ob], wave);
-            store_t(H2T, ob, h2[ob], wave);
-            store_t(DH2T, ob, dh2[ob], wave);
-            store_t(DH1T, ob, dh1[ob], wave);
-        }
-        store_t(DYT, 0, dy, wave);
         __syncthreads();
         // weight gradients: dW[o][i] = sum over the chunk's rows of dH[row][o] * In[row][i]
+        int at = c * TR_LD + 8 * g;
+        asm volatile("" : "+v"(at));  // the addresses are formed here: kept over the loop they would spill
+        auto products = [&](auto n_kb) {
 #pragma unroll
-        for (int k = 0; k < TR_BLK_PER_WAVE; ++k) {
-            const int blk = wave + k * TR_WAVES;
-            if (blk >= TR_NBLK) break;
-            const __bf16 *A, *B;
-            int mb, nb;
-            if (blk < TR_BLK1) { mb = blk / (MLP_IN / 16); nb = blk % (MLP_IN / 16); A = DH1T; B = XT; }
-            else if (blk < TR_BLK1 + TR_BLK2) { const int q = blk - TR_BLK1; mb = q / (MLP_H / 16); nb = q % (MLP_H / 16); A = DH2T; B = H1T; }
-            else { const int q = blk - TR_BLK1 - TR_BLK2; mb = 0; nb = q; A = DYT; B = H2T; }
+            for (int k = 0; k < TR_BLK_PER_WAVE; ++k) {
+                const int blk = wave + k * TR_WAVES;
+                if (blk >= TR_NBLK) break;
+                const __bf16 *A, *B;
+                int mb, nb;
+                if (blk < TR_BLK1) { mb = blk / (MLP_IN / 16); nb = blk % (MLP_IN / 16); A = DH1T; B = XT; }
+                else if (blk < TR_BLK1 + TR_BLK2) { const int q = blk - TR_BLK1; mb = q / (MLP_H / 16); nb = q % (MLP_H / 16); A = DH2T; B = H1T; }
+                else { const int q = blk - TR_BLK1 - TR_BLK2; mb = 0; nb = q; A = DYT; B = H2T; }
 #pragma unroll
-            for (int kb = 0; kb < TR_KB; ++kb)
-                acc[k] = mfma_bf16(ld_bf16x8(A + (mb * 16 + c) * TR_LD + kb * 32 + 8 * g),
-                                   ld_bf16x8(B + (nb * 16 + c) * TR_LD + kb * 32 + 8 * g), acc[k]);
-        }
+                for (int kb = 0; kb < n_kb.value; ++kb)
+                    acc[k] = mfma_bf16(ld_bf16x8(A + mb * 16 * TR_LD + kb * 32 + at),
+                                       ld_bf16x8(B + nb * 16 * TR_LD + kb * 32 + at), acc[k]);
+            }
+        };
+        if (two) products(std::integral_constant<int, TR_KB>());
+        else products(std::integral_constant<int, TR_KB / 2>());
         // bias gradients: b1 (128), b2 (128), b3 (16) from the same bf16
         // values, rows in order; waves 0..3 a b1 or b2 entry per thread, the
         // first lanes of wave 4 a b3 entry
@@ -237,12 +266,12 @@ __global__ void __launch_bounds__(TR_THREADS) mlp_train_partial_kernel(MlpDev w,
                                 : t < 2 * MLP_H ? DH2T + (t - MLP_H) * TR_LD
                                                 : DYT + (t - 2 * MLP_H) * TR_LD;
             if (t < 2 * MLP_H + MLP_OUT)
-                for (int r = 0; r < TR_ROWS; r += 8) {
+                for (int r = 0; r < (two ? TR_ROWS : TR_CHUNK); r += 8) {
                     const bf16x8 v = ld_bf16x8(src + r);
 #pragma unroll
                     for (int q = 0; q < 8; ++q) bacc += (float)v[q];
                 }
-            if (wave < TR_CHUNK_WAVES) loss += lrow[wave * 64 + l];
+            if (two && wave < TR_CHUNK_WAVES) loss += lrow[wave * 64 + l];
         }
         __syncthreads();
     }
@@ -312,14 +341,15 @@ __global__ void mlp_reduce_adam_kernel(const float* partial, int n_part, float* 
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p > MLP_NPARAM) return;
     float gsum = 0.f;
-    double lsum = 0.;  // the loss (as in the partial sums)
+    if (p < MLP_NPARAM) {
 #pragma unroll 16
-    for (int b = 0; b < n_part; ++b) {
-        const float x = partial[(size_t)b * TR_PARTIAL + p];
-        gsum += x;
-        lsum += x;
+        for (int b = 0; b < n_part; ++b) gsum += partial[(size_t)b * TR_PARTIAL + p];
+    } else {  // the loss, in 64 bits (as in the partial sums)
+        double lsum = 0.;
+#pragma unroll 16
+        for (int b = 0; b < n_part; ++b) lsum += partial[(size_t)b * TR_PARTIAL + p];
+        gsum = (float)lsum;
     }
-    if (p == MLP_NPARAM) gsum = (float)lsum;
     if (grad_out) grad_out[p] = gsum;
     if (loss_out && p == MLP_NPARAM) *loss_out = gsum;
     if (!adam || p == MLP_NPARAM) return;
@@ -410,12 +440,16 @@ hipError_t upside_mlp_launch_forward(const MlpDev& w, const float* feat, int n, 
 
 int upside_mlp_partial_size() { return TR_PARTIAL; }
 
-// Workgroups of the gradient kernel for n_batch rows: MLP_PARTS up to 4096
-// rows (two chunks each, one trip through the kernel), then one more per two
-// chunks until the chip is full.  Loss and gradient of 97,801 rows: 0.86 ms on
-// 32 workgroups of one chunk at a time, 0.19 ms on 256.
+// Workgroups of the gradient kernel for n_batch rows: one per chunk up to
+// MLP_PARTS (an empty one would write 91 KB of zeros for the reduction to read),
+// as many up to 4096 rows (two chunks each, one trip through the kernel), then
+// one more per two chunks until the chip is full.  Loss and gradient of 128,
+// 1000 and 2048 rows: 60, 63, 63 us on 32 workgroups with empty chunks, 45, 48,
+// 50 now; of 97,801 rows 826 us on 32 workgroups of one chunk at a time, 141 on
+// 256 of two.
 int upside_mlp_parts(int n_batch) {
     const int chunks = (n_batch + TR_CHUNK - 1) / TR_CHUNK;
+    if (chunks < MLP_PARTS) return chunks;
     const int want = (chunks + 1) / 2;
     return want < MLP_PARTS ? MLP_PARTS : want > MLP_MAX_PARTS ? MLP_MAX_PARTS : want;
 }
