@@ -18,6 +18,8 @@ namespace upside {
 // coefficient tables (the largest, the rotamer pair table, is 20*20*54 floats
 // = 86.4 KB, plus read-past padding), cell grids, and the rotamer solve state.
 constexpr int LDS_FLOATS = 39936;
+// Residue types of an environment coverage (a lane's bins lie in LDS).
+constexpr int MAX_AA_TYPES = 79;
 // Rotamer statistics words: [0] iterations of the last solve, [1] solves at
 // the iteration limit, [2] total iterations, [3] solves, [4] BP edges, [5]
 // residue-pair candidates, [6] solves held in LDS, [7] warm-started solves,

@@ -679,8 +679,11 @@ __device__ __forceinline__ void env_coverage_fwd(Ctx& c, OpC& op, GraphC& G) {
     // the group's lanes in lane order
     lp<float> mine = c.lds + c.tid * naa;
     lp<float> grp_bins = c.lds + (c.tid & ~(GW - 1)) * naa;
-    const int grp = c.gtid / GW, gl = c.gtid % GW, NG = c.gsize / GW;
-    for (int base = 0; base < G.n1; base += NG) {
+    // (with more than 78 types, on the waves whose bins fit)
+    const int waves = min(NWAVE, LDS_FLOATS / (64 * naa));
+    const int n = c.tid < 64 * waves ? G.n1 : 0;
+    const int grp = c.gtid / GW, gl = c.gtid % GW, NG = waves * 64 * c.G / GW;
+    for (int base = 0; base < n; base += NG) {
         const int i = base + grp;
         const bool ok = i < G.n1;
         for (int t = 0; t < naa; ++t) mine[t] = 0.f;
