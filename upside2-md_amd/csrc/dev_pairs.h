@@ -229,15 +229,16 @@ __device__ __forceinline__ int cell_bucket(int mask, int cx, int cy, int cz) {
     return (int)(h & (uint32_t)mask);
 }
 
+// Points that a grid holds: with 4096 buckets up to 7167, with 2048 the rest
+// (the rows are the same).
+constexpr int GRID_POINTS = 7320;
+static_assert((2048 + 4) * 4 + GRID_POINTS * 20 <= LDS_FLOATS * 4, "a grid in LDS");
 __device__ __forceinline__ int lgrid_buckets(int m) {
     int nb = 64;
     while (nb < m && nb < 4096) nb *= 2;
-    return nb;
+    return (nb + 4) * 4 + m * 20 <= LDS_FLOATS * 4 ? nb : nb / 2;
 }
-__device__ __forceinline__ bool lgrid_fits(int m) {
-    int nb = lgrid_buckets(m);
-    return (nb + 4) * 4 + m * 20 <= LDS_FLOATS * 4;
-}
+__device__ __forceinline__ bool lgrid_fits(int m) { return m <= GRID_POINTS; }
 
 // Build the grid of the m points pts (stride 3) in this workgroup's LDS
 // (every workgroup of a team builds its own copy).  All threads of the workgroup.
@@ -245,7 +246,7 @@ __device__ __forceinline__ bool lgrid_fits(int m) {
 // order by counting, for each of its elements, those with a smaller index: a
 // cell holds some 25 beads, and one thread sorting it by insertion was most of
 // the build.
-constexpr int GRID_U = (LDS_FLOATS * 4 / 20 + NT - 1) / NT;
+constexpr int GRID_U = (GRID_POINTS + NT - 1) / NT;
 __device__ __forceinline__ LGrid lgrid_build(Ctx& c, GraphC& G, ap<const float> pts, gp<const int> ids, int m) {
     float x[GRID_U][3];
     int id[GRID_U], at[GRID_U];
