@@ -365,7 +365,7 @@ int upside_mlp_forward(UpsideMlp* net, const float* features, int n_rows, float*
  * bits), on buffers the caller owns in device memory: params[n_param],
  * features[n_rows][32], targets[n_rows][8], out[n_param + 1] (gradient, then
  * the loss).  Every intermediate lives in a static device array of the
- * library (about 20 MB per GPU, held until the process ends); n_rows must be
+ * library (23.4 MB per GPU, held until the process ends); n_rows must be
  * in [1, 2^24].  Calls that overlap on one GPU share that array and race.
  * Runs on the null stream and returns when out is written; 0 on success. */
 int upside_mlp_loss_grad_noalloc(const float* params, const float* features, const float* targets, int n_rows,

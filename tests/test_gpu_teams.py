@@ -171,3 +171,28 @@ def test_every_evaluation_in_threads(ue, chain_file):
 
     with concurrent.futures.ThreadPoolExecutor(4) as pool:
         assert sum(f.result() for f in [pool.submit(work, k) for k in range(4)]) == 80
+
+
+@pytest.mark.parametrize("n_res", [199, 200])
+def test_evaluation_without_a_rotamer_solve(ue, tmp_path, monkeypatch, n_res):
+    """Pair lists but no rotamer node, on both sides of the rule's line for them."""
+    import upconfig
+    rng = np.random.default_rng(n_res)
+    seq = upconfig.random_sequence(n_res, rng)
+    g = upconfig.build_ff21(seq, upconfig.random_initial_config(n_res, rng))
+    keep = ["Distance3D", "Spring_bond", "Angle", "Spring_angle", "Dihedral_omega", "Spring_omega", "rama_map_pot",
+            "rama_map_pot_ref", "backbone_pairs", "infer_H_O", "protein_hbond", "hbond_energy", "Dihedral_phi",
+            "Dihedral_psi", "rama_coord", "affine_alignment"]
+    kept = lambda p: not p.startswith("/input/potential/") or p.split("/")[3] in keep
+    g.order = [p for p in g.order if kept(p)]
+    g.dsets = {p: a for p, a in g.dsets.items() if kept(p)}
+    path = str(tmp_path / "backbone.up")
+    upconfig.write_up(path, g)
+    a = ue.Upside(path, quiet=True)
+    monkeypatch.setenv("UPSIDE_TEAM", "1")
+    b = ue.Upside(path, quiet=True)
+    for _ in range(3):
+        pos = np.ascontiguousarray(upconfig.random_initial_config(n_res, rng), np.float32)
+        np.testing.assert_allclose(a.energy(pos), b.energy(pos), rtol=1e-5)
+        np.testing.assert_array_equal(a.deriv(pos), b.deriv(pos))
+        np.testing.assert_array_equal(a.get_output("protein_hbond"), b.get_output("protein_hbond"))

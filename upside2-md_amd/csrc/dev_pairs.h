@@ -11,12 +11,12 @@
 // edge set does not depend on how the cache was built.
 //
 // Rebuild: the other side is put into a hashed cell grid in LDS (or streamed
-// in tiles when it does not fit) and every row scans it twice, once to count
-// partners and, after a team scan of the counts, once to write them.  Row
-// order is canonical (fixed cell-visit order, index order inside a cell).
-// Transposed rows (the forward slots of each side-2 element) are placed by
-// per-column counters and then ordered by slot, so every order is
-// independent of scheduling.
+// in tiles when it does not fit) and every row scans it once, keeping the
+// partners in a slab; after a team scan of the counts they are copied to their
+// slots (a row that outgrew its slab is scanned again).  Row order is canonical
+// (fixed cell-visit order, index order inside a cell).  Transposed rows (the
+// forward slots of each side-2 element) are placed by their arrival in the
+// column and then ordered by slot, so every order is independent of scheduling.
 #pragma once
 #include "dev_common.h"
 

@@ -1255,12 +1255,11 @@ __device__ __forceinline__ int rot_solve_team(Ctx& c, RotC& R) {
 // team barrier).
 //
 // One workgroup's iteration grows with the edges and has no team barrier;
-// several share the edges and pay two.  ms per step, one workgroup / several
-// (edges in brackets): on 16 workgroups 0.336 / 0.357 (285), 0.471 / 0.460
-// (546), 0.637 / 0.609 (825), 0.814 / 0.747 (1287); on 32 0.344 / 0.383 (285),
-// 0.462 / 0.469 (546), 0.599 / 0.584 (825), 0.704 / 0.633 (1287), 0.900 /
-// 0.755 (500 residues).  Half of a team of 8 or 4 never won (67 to 500
-// residues).
+// several share the edges and pay one.  ms per step, one workgroup / several:
+//   residues            67            130           150           180           200           300           500
+//   16 workgroups  .332 / .349   .406 / .412   .457 / .443   .471 / .473   .563 / .514   .711 / .677   .760 / .723
+//   32             .340 / .378   .406 / .410   .453 / .435   .480 / .448   .546 / .489   .667 / .596   .707 / .669
+// (about 600 edges at 180 residues).  Half of a team of 8 or 4 never won.
 constexpr int BP_TEAM_MIN = 16, BP_WG_EDGES = 600;
 __device__ __forceinline__ bool bp_on_one_wg(const Ctx& c, RotC& R, int nbp, int bp_layout) {
     if (c.G == 1 || bp_layout == 2) return true;

@@ -320,8 +320,9 @@ struct RunArgs {
     // 3 dt (r+1) from each system's initial temperature
     int anneal;
     double anneal_factor, anneal_start, anneal_end, anneal_duration;
-    // rotamer solves: 0 on one workgroup when the BP state fits its LDS, else
-    // on the whole team; 1 always the team; 2 always one workgroup
+    // rotamer solves: 0 on one workgroup or on several by edges and team; 1
+    // always the whole team; 2 always one workgroup; 3 always several (see
+    // bp_on_one_wg)
     int bp_layout;
     // rotamer solve schedule: 0 the reference's (start from the node
     // probabilities, stop when the one-sided change is at most the node's

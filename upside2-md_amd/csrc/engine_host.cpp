@@ -2682,19 +2682,23 @@ struct DerivEngine {
     // and a team's cooperative launch costs 20 us.  us per evaluation with the
     // derivative, on 1 / 4 / 8 / 16 / 32 workgroups:
     //   a whole force field (a rotamer solve)
-    //      10 residues  480 /  416 /  421 /  433 /  462
-    //      40           716 /  514 /  503 /  523 /  577
-    //      67          1154 /  658 /  607 /  589 /  619
-    //     101          1445 /  748 /  657 /  643 /  693
-    //     150          2890 / 1226 /  969 /  857 /  832
-    //     500         11227 / 4302 / 2700 / 1927 / 1593
+    //      10 residues  485 /  418 /  406 /  435 /  440
+    //      25           592 /  435 /  435 /  444 /  482
+    //      55           820 /  517 /  505 /  492 /  576
+    //     101          1385 /  713 /  626 /  589 /  647
+    //     125          1820 /  864 /  747 /  662 /  694
+    //     150          2363 / 1066 /  861 /  749 /  725
+    //     500          8139 / 3070 / 2076 / 1547 / 1257
     //   pair lists, but no rotamer solve (backbone pairs and hydrogen bonds)
-    //     120           210 /  186 /  188 /  197 /  219
-    //     200           266 /  216 /  206 /  213 /  234
-    //     500           600 /  326 /  279 /  262 /  281
+    //      60           180 /  176 /  183 /  185 /  215
+    //     120           205 /  184 /  184 /  192 /  206
+    //     200           256 /  207 /  200 /  207 /  226
+    //     500           476 /  293 /  264 /  255 /  272
     //   bonded terms only
-    //     500           120 /  141 /  144 /  152 /  166
-    // The lines are drawn where the next team overtakes.
+    //     500           122 /  143 /  142 /  153 /  158
+    // With a rotamer solve the lines are drawn where the next team overtakes.
+    // Without, one workgroup is kept beyond that (about 80 residues), up to where
+    // it takes a fifth longer: it needs one CU and waits for nobody.
     static int eval_team(const Topology& T) {
         if (!T.rots.empty()) return T.n_atom <= 75 ? 4 : T.n_atom <= 165 ? 8 : T.n_atom <= 375 ? 16 : 32;
         return T.graphs.empty() || T.n_atom < 600 ? 1 : 8;
