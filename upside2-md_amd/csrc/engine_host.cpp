@@ -1929,7 +1929,7 @@ struct Batch {
         const float time = 3.f * dt * (float)(nr + 1);
         for (auto& s : sys) s.temperature = (float)anneal_temp((double)s.temp0, (double)time);
     }
-    unsigned spin_limit = BAR_SPIN_LIMIT;  // RunArgs::spin_limit
+    unsigned spin_limit = 0;     // RunArgs::spin_limit
     bool profile = false;
     vector<unsigned long long*> prof;
     // wall-clock ticks per op, fixed slots, then team barriers per op (+1: outside the ops)
@@ -2077,7 +2077,9 @@ struct Batch {
         return d;
     }
 
-    void create(const vector<string>& paths, const vector<float>& temps, int n_atom_hint) {
+    void create(const vector<string>& paths, const vector<float>& temps, int n_atom_hint,
+                unsigned spins = BAR_SPIN_LIMIT) {
+        spin_limit = spins;
         std::map<string, std::shared_ptr<Program>> by_path;
         // UPSIDE_CAPACITY_SCALE (e.g. 0.05) starts with small neighbour-list
         // capacities; overflow regrowth then doubles them as needed
@@ -2086,7 +2088,11 @@ struct Batch {
             if (v > 0.0 && v <= 64.0) cap_scale = v;
         }
         // UPSIDE_BARRIER_SPINS: polls after which a barrier gives up (0: at the first one not yet met)
-        if (const char* e = std::getenv("UPSIDE_BARRIER_SPINS")) spin_limit = (unsigned)std::strtoul(e, nullptr, 10);
+        if (const char* e = std::getenv("UPSIDE_BARRIER_SPINS")) {
+            char* end = nullptr;
+            const unsigned long v = std::strtoul(e, &end, 10);
+            if (end != e && v <= 0xfffffffful) spin_limit = (unsigned)v;
+        }
         hip_check(hipStreamCreate(&stream), "stream");
         hip_check(hipEventCreate(&ev0), "event");
         hip_check(hipEventCreate(&ev1), "event");
@@ -3194,12 +3200,11 @@ DerivEngine* construct_deriv_engine(int n_atom, const char* potential_file, bool
     ABI_TRY
     (void)quiet;
     std::unique_ptr<DerivEngine> e(new DerivEngine);
-    e->batch.create({string(potential_file)}, {1.f}, n_atom);
+    // an evaluation can be repeated on one workgroup: it need not wait as long as a run (0.8 s)
+    e->batch.create({string(potential_file)}, {1.f}, n_atom, BAR_SPIN_LIMIT / 4);
     if (e->batch.sys[0].prog->T.n_atom != n_atom) fail("n_atom mismatch");
     if (!std::getenv("UPSIDE_TEAM"))
         e->batch.set_team(std::min(DerivEngine::eval_team(e->batch.sys[0].prog->T), e->batch.max_team()));
-    // an evaluation can be repeated on one workgroup: it need not wait as long as a run (0.8 s)
-    if (!std::getenv("UPSIDE_BARRIER_SPINS")) e->batch.spin_limit = BAR_SPIN_LIMIT / 4;
     return e.release();
     ABI_CATCH(nullptr)
 }
